@@ -22,7 +22,7 @@ OUT = os.path.join(HERE, "libqwattn.so")
 BUILD_DIR = os.path.join(HERE, "_build")
 ARCH = "gfx950"
 
-SOURCES = ["kv_cache.hip", "attend_decode.hip", "attend_block.hip", "dlsa.hip", "dlsa_typed.hip",
+SOURCES = ["kv_cache.hip", "attend_decode.hip", "attend_block.hip", "attend_rows.hip", "dlsa.hip", "dlsa_typed.hip",
            "sdpa_general.hip", "dlsa_select.hip", "rope.hip", "turbo4.hip", "abi.hip"]
 # The measurement library (read-floor and copy kernels), loaded by bench.py only.
 CEIL_SOURCES = ["ceiling.hip"]

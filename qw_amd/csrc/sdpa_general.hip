@@ -313,6 +313,21 @@ int gen_kv_workspace(int device, hipStream_t stream, size_t need, void** out) {
     return b.get(need, stream, out);
 }
 
+// Whether a call takes the row kernel (attend_rows.hip), which lays every key
+// tile out once and then runs at several times this kernel's rate: 1536 rows
+// over 9728 keys (24 heads over 4, D = 256) 1943 -> 372 us. The layout and two
+// more launches cost what some 100 rows a KV head do, so the line lies at
+// (R - 100) T of 1.3M: at 384 rows a head 43.8 against 46.3 us over 4k keys
+// (here) and 130.8 -> 76.0 us over 16k (there), at 1536 rows 27.8 against 31.0
+// us over 300 keys and 52.7 -> 38.4 us over 1k. A mask is read a byte or two a
+// lane here and in 8-key pieces there: 78 rows over 8k keys 42 -> 27 us.
+bool rows_route(int R, int n_keys, int hkv, int D, bool mask, const void* out) {
+    if ((uintptr_t)out % 8 != 0) return false;  // (it writes 8-byte pieces)
+    // images of more than 4 GiB are not kept (1.03 KB a key and head at D = 256)
+    if ((int64_t)n_keys * hkv * D * 2 * sizeof(f16) > (int64_t)4 << 30) return false;
+    return mask ? R > 16 && (int64_t)R * n_keys >= 500000 : (int64_t)(R - 100) * n_keys >= 1300000;
+}
+
 int mask_kind_of(int dtype) {
     switch (dtype) {
         case QW_MASK_BOOL: return kMaskBool;
@@ -351,6 +366,13 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
     QW_REQUIRE(!o.mask || (o.mask_head_stride >= 0 && o.mask_row_stride >= 0),
                QW_ERR_INVALID_ARGUMENT, "sdpa: negative mask stride");
     const int G = n_q_heads / n_kv_heads, R = G * n_rows, D = head_dim;
+    if (rows_route(R, n_keys, n_kv_heads, D, o.mask != nullptr, out)) {
+        const int rc = rows_attention(q, G, n_rows, k, v, n_kv_heads, n_keys, D, khs, krs, vhs, vrs,
+                                      scale, o, out, stream);
+        // without room for the images (under capture, or no memory left) the
+        // kernel here still serves the call
+        if (rc != QW_ERR_STATE && rc != QW_ERR_OUT_OF_MEMORY) return rc;
+    }
     GenArgs a;
     a.q = (const f16*)q;
     a.k = (const f16*)k;

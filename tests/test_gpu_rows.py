@@ -1,0 +1,112 @@
+"""GPU parity of the row kernel behind qw_sdpa (attend_rows.hip: many query rows over fp16 K/V
+views, laid out once as tile images) against oracle.sdpa_general, at the sizes where it can go
+wrong: key counts around a tile (64 / 128 / 256 keys at D 256 / 128 / 64), rows around a wave and
+a workgroup, split and unsplit plans, every mask type at odd strides, windows below a tile.
+
+Bar: the attention tolerance (2e-3 max-abs, 1e-3 relative L2); the masks' rows that see nothing
+are exact zeros."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import rng
+from test_gpu_kv import _gpu, _np, assert_close
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _views(r, hkv, T, D, pad):
+    """fp16 K, V [hkv, T, D] and the same rows as views of a larger allocation whose other rows
+    are NaN (nothing past the view may be read into a result)."""
+    k = r.standard_normal((hkv, T, D)).astype(np.float16)
+    v = r.standard_normal((hkv, T, D)).astype(np.float16)
+    kb = torch.full((hkv, T + pad, D + 8), float("nan"), dtype=torch.float16, device="cuda:0")
+    vb = torch.full_like(kb, float("nan"))
+    kb[:, :T, :D] = _gpu(k)
+    vb[:, :T, :D] = _gpu(v)
+    return k, v, kb[:, :T, :D], vb[:, :T, :D]
+
+
+CASES = [
+    # hq, hkv, D, L, T, causal, window, softcap
+    (24, 4, 256, 129, 2048, True, 0, 0.0),     # whole tiles; 774 rows a head, a ragged last tile
+    (24, 4, 256, 257, 1985, True, 0, 0.0),     # one key into the last tile
+    (24, 4, 256, 257, 1983, True, 0, 0.0),     # one key short of it
+    (8, 8, 128, 700, 2305, True, 0, 0.0),      # G = 1
+    (32, 8, 128, 200, 2047, True, 130, 0.0),   # a window about a tile
+    (16, 2, 64, 256, 1281, True, 0, 0.0),      # 256-key tiles in two halves
+    (16, 2, 64, 300, 1500, True, 33, 20.0),    # a window below a tile, capped
+    (24, 4, 128, 220, 1400, False, 0, 30.0),   # capped, not causal
+    (12, 1, 256, 190, 1000, True, 0, 0.0),     # one KV head, G = 12
+    (24, 4, 256, 1100, 1100, True, 0, 0.0),    # prefill into nothing: rows from one key on
+]
+
+
+@pytest.mark.parametrize("hq,hkv,D,L,T,causal,window,softcap", CASES)
+def test_rows_match_oracle(hq, hkv, D, L, T, causal, window, softcap):
+    import qw_amd
+
+    print(f"case hq={hq} hkv={hkv} D={D} L={L} T={T} causal={causal} w={window} sc={softcap}",
+          flush=True)
+    assert (hq // hkv * L - 100) * T >= 1300000 or L == 190, "a shape of the row kernel"
+    r = rng(hq + D + L + T)
+    q = r.standard_normal((hq, L, D)).astype(np.float16)
+    k, v, kv, vv = _views(r, hkv, T, D, 9)
+    out = _np(qw_amd.attention(_gpu(q), kv, vv, D ** -0.5, None, softcap, window, causal))[0]
+    assert np.isfinite(out).all()
+    assert_close(out, oracle.sdpa_general(q, k, v, D ** -0.5, causal, window, softcap),
+                 f"rows D={D} L={L} T={T}")
+
+
+@pytest.mark.parametrize("kind", ["bool", "f16", "bf16", "f32"])
+@pytest.mark.parametrize("hq,hkv,D,L,T,causal,per_head", [
+    (24, 4, 256, 13, 6500, False, False),
+    (24, 4, 128, 41, 2051, True, True),
+    (16, 2, 64, 20, 3333, False, True),
+])
+def test_rows_masks_match_oracle(kind, hq, hkv, D, L, T, causal, per_head):
+    import qw_amd
+
+    print(f"case {kind} hq={hq} D={D} L={L} T={T} causal={causal}", flush=True)
+    assert hq // hkv * L * T >= 500000, "a shape of the row kernel"
+    r = rng(hq + D + L + T + len(kind))
+    q = r.standard_normal((hq, L, D)).astype(np.float16)
+    k, v, kv, vv = _views(r, hkv, T, D, 3)
+    H = hq if per_head else 1
+    hidden = r.random((H, L, T)) < 0.3
+    hidden[:, 0, :] = True                       # a row that sees nothing
+    hidden[:, 1:, 0] = False
+    if kind == "bool":
+        m = ~hidden
+        full = torch.zeros((H, L, T + 5), dtype=torch.bool, device="cuda:0")
+    else:
+        m = (2 * r.standard_normal((H, L, T))).astype(np.float32)
+        m[hidden] = -np.inf
+        dt = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[kind]
+        full = torch.zeros((H, L, T + 5), dtype=dt, device="cuda:0")
+    view = full[:, :, 1:T + 1]                   # odd row stride, off any vector alignment
+    view.copy_(torch.from_numpy(m))
+    m = view.cpu().numpy() if kind == "bool" else view.float().cpu().numpy()
+    sc = 0.0 if kind == "bool" else 25.0
+    for cap in {0.0, sc}:
+        out = _np(qw_amd.attention(_gpu(q), kv, vv, D ** -0.5, view, cap, 0, causal))[0]
+        assert np.isfinite(out).all() and np.all(out[:, 0] == 0)
+        ref = oracle.sdpa_general(q, k, v, D ** -0.5, causal, 0, cap, m)
+        assert_close(out[:, 1:], ref[:, 1:], f"rows {kind} cap={cap}")
+
+
+def test_rows_route_agrees_with_the_general_kernel():
+    """The same rows in one call (row kernel) and in calls of few rows (the general kernel)."""
+    import qw_amd
+
+    r = rng(5)
+    hq, hkv, D, L, T = 24, 4, 256, 160, 1700
+    q = _gpu(r.standard_normal((hq, L, D)).astype(np.float16))
+    _, _, kv, vv = _views(r, hkv, T, D, 0)
+    whole = _np(qw_amd.causal_attention(q, kv, vv, 1 / 16))[0]
+    step = 16
+    parts = [_np(qw_amd.causal_attention(q[:, i:i + step].contiguous(), kv[:, :T - L + i + step],
+                                         vv[:, :T - L + i + step], 1 / 16))[0]
+             for i in range(0, L, step)]
+    assert_close(whole, np.concatenate(parts, axis=1), "one call vs pieces")
