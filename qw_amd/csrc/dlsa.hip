@@ -41,6 +41,9 @@ struct DlsaArgs {
     float2* part_ml; // [L][Hq][parts]
     int L, W, hq, hkv, G, T, parts;
     float scale2;    // scale * log2(e)
+    // != null: only the rows of the groups flagged there (dlsa_rows.hip left them)
+    const int* flags; // [ceil(L / group_rows)][hkv]
+    int group_rows;   // even
 };
 
 constexpr int kDlsaNT = 2;  // tiles per batch a wave keeps in flight
@@ -587,6 +590,8 @@ __device__ __forceinline__ void dlsa_body(const DlsaArgs& a, const Src& src) {
 // fast_flag), else the separately rounded one.
 template <int D, int GMAX, class Src, int RP = 1>
 __global__ __launch_bounds__(256, 2) void dlsa_kernel(DlsaArgs a, Src src, const int* fast_flag) {
+    // (two-row workgroups never straddle groups: both counts are even)
+    if (a.flags && !a.flags[(int)(blockIdx.y * RP) / a.group_rows * a.hkv + blockIdx.z]) return;
     if constexpr (Src::kAffine) {
         // The exact 2-op dequant runs without waiting for the cache's fast
         // flag; a cache holding a scale outside its exact range takes the
@@ -792,8 +797,10 @@ static int dlsa_sparse_attention_impl(const void* q, const DlsaSource& src,
     QW_HIP_CHECK(hipGetDevice(&dev));
     // bytes of one part's partials: an fp32 output row and an (m, l) pair per (row, q head)
     const size_t part_bytes = (size_t)n_rows * n_q_heads * (head_dim * sizeof(float) + sizeof(float2));
+    bool auto_one_pass = false;
     if (parts <= 0) {
         parts = auto_parts(n_rows * n_kv_heads, width);
+        auto_one_pass = parts == 1 && waves == 0 && !scratch;
         if (scratch) parts = (int)std::min<size_t>((size_t)parts, scratch_bytes / part_bytes);
     }
     parts = std::max(1, std::min(parts, kDlsaMaxParts));
@@ -818,6 +825,21 @@ static int dlsa_sparse_attention_impl(const void* q, const DlsaSource& src,
     a.T = n_keys;
     a.parts = parts;
     a.scale2 = scale * kLog2e;
+    a.flags = nullptr;
+    a.group_rows = 1;
+    if (auto_one_pass && !src.cache && dlsa_rows_pays(n_rows, width, n_kv_heads)) {
+        // prefill row counts: neighbouring rows share their keys' gathers; the
+        // kernel below then serves the groups that this one leaves
+        const int rc = dlsa_rows_attention(q, src.k, src.v, false, src.khs, src.krs, src.vhs, src.vrs,
+                                           lists, lengths, n_rows, width, n_q_heads, n_kv_heads,
+                                           head_dim, n_keys, scale, out, &a.flags, stream);
+        if (rc == QW_OK)
+            a.group_rows = dlsa_rows_per_group(G);
+        else if (rc != QW_ERR_STATE && rc != QW_ERR_OUT_OF_MEMORY)
+            return rc;
+        else
+            a.flags = nullptr;  // (under capture, or no memory left: every row there)
+    }
     if (parts > 1) {
         const size_t no = (size_t)n_rows * n_q_heads * parts;
         void* ws = scratch;

@@ -1,0 +1,657 @@
+// dlsa_rows.hip - the D-LSA gathered read (K2) for prefill row counts, gfx950:
+// neighbouring rows read the keys that any of them lists once.
+//
+// Contract: dlsa.hip's (the reference's dlsa_attention::sparse_attention,
+// crates/mlxcel-core/src/dlsa_attention.rs:31-63): row r attends over the keys
+// of its own list, entries outside [0, T) skipped, fp32 scores, softmax and sums,
+// a row without a valid entry zeros. fp16 or bf16 q, K and V (alike), output in
+// that type.
+//
+// The rows of a prefill chunk list nearly the same keys (the sinks, the chunk's
+// long-range blocks, windows that slide by one), but one row fills 6 of an MFMA
+// tile's 16 columns and gathering its keys alone moves them once a row: 29 GB of
+// L1 / L2 traffic for 1536 rows of 4612 keys. Here
+//   dlsa_plan_kernel, one workgroup a group of NR neighbouring rows (NR G <= 128),
+//     marks every listed key in an LDS bitmap word (bit i: row i of the group) and
+//     compacts the marked keys in ascending order, with their words;
+//   dlsa_rows_kernel, a workgroup a (group, KV head) as the block kernels have it:
+//     128 columns (row, head), 64-key tiles gathered by the key list into the LDS
+//     layout of block_tile.hpp, and for each score the key's bit of its row;
+//   dlsa_rows_merge_kernel sums the fp32 partials of the groups whose keys were
+//     split (the last, partial round of workgroups).
+// P enters P.V as a high part plus a remainder in the element type, as in
+// dlsa.hip (fp16; 16 bits of P in bf16, far below the output's 8).
+// What bounds it: MFMAs and LDS operand reads, as in attend_rows.hip, with three
+// MFMAs a (key, column, dim) where that kernel has two. Measured (24 heads over 4,
+// D = 256, lists of 4 sinks, a 512-key window and 8 shared 512-key blocks): 1536 rows
+// at 32k in fp16 1312 us by row pairs -> 347 us here (502 TFLOP/s; the plan 26 us, the
+// merge 6 us of it), 512 rows at 16k in bf16 7572 -> 157 us.
+//
+// A group is left to the row-by-row kernels, launched behind with the flags of
+// this one, where (a) a row lists a key twice (it counts twice), (b) the union is
+// larger than max_union (the rows share too little), or (c) an output came out
+// infinite or NaN: a key's V reaches every row of its group here with weight 0,
+// and 0 x inf is NaN.
+#include <algorithm>
+#include <map>
+#include <mutex>
+
+#include "block_tile.hpp"
+#include "kv_cache.hpp"
+#include "qw_common.hpp"
+
+namespace qw {
+
+namespace {
+
+typedef __bf16 bhalf8 __attribute__((ext_vector_type(8)));
+typedef uint16_t ushort4v __attribute__((ext_vector_type(4)));
+typedef uint16_t ushort8v __attribute__((ext_vector_type(8)));
+
+constexpr int kPlanSeg = 40448;  // keys a bitmap pass covers (158 KB of LDS)
+constexpr int kPlanThreads = 1024;
+
+// Group blockIdx.x: rows NR * blockIdx.x .. +NR-1. Writes its keys (ascending,
+// padded with (0, no rows) to whole tiles of KT), their row words and the count;
+// flags[group][hkv] = 1 and count 0 if the group is not served.
+__global__ __launch_bounds__(kPlanThreads) void dlsa_plan_kernel(
+    const int32_t* __restrict__ lists, const int32_t* __restrict__ lengths, int L, int W, int T,
+    int NR, int KT, int max_union, int cap, int hkv, int32_t* __restrict__ keys,
+    uint32_t* __restrict__ words, int* __restrict__ counts, int* __restrict__ flags) {
+    constexpr int NWV = kPlanThreads / 64;
+    extern __shared__ __attribute__((aligned(16))) uint32_t bm[];  // min(T, kPlanSeg) words, whole u32x4
+    __shared__ int wave_n[NWV];
+    __shared__ int listed, marked;  // valid entries of the group's lists / bits set for them
+    const int grp = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r0 = grp * NR, nr = min(NR, L - r0), n_chunks = (W + 255) / 256;
+    int32_t* const gk = keys + (int64_t)grp * cap;
+    uint32_t* const gw = words + (int64_t)grp * cap;
+    if (tid == 0) listed = marked = 0;
+    const int my_len = lane < nr ? min(lengths[r0 + lane], W) : 0;  // lane i: row i's length
+    int total = 0, n_listed = 0, n_marked = 0;
+    for (int seg = 0; seg < T; seg += kPlanSeg) {
+        const int n = min(kPlanSeg, T - seg), n4 = (n + 3) / 4;
+        __syncthreads();  // the previous segment's words are read
+        for (int i = tid; i < n4; i += kPlanThreads) ((u32x4*)bm)[i] = u32x4{0, 0, 0, 0};
+        __syncthreads();
+        // 256-entry chunks of the lists (four entries a lane), dealt to the waves in
+        // turn, eight of a wave in flight before the first is marked: a few
+        // workgroups read all the lists from HBM (an entry a lane at a time, its
+        // mark's old value awaited: 94 us for 1536 rows of 4612 entries)
+        int r = 0, c = wave;  // the wave's next chunk: chunk c of row r
+        auto next = [&]() {
+            while (c >= n_chunks && r < nr) {
+                c -= n_chunks;
+                r++;
+            }
+        };
+        next();
+        while (r < nr) {
+            constexpr int AH = 8;
+            u32x4 x[AH];
+            int row[AH];
+#pragma unroll
+            for (int i = 0; i < AH; i++) {
+                row[i] = min(r, nr - 1);
+                const int e = 256 * c + 4 * lane;
+                const int left = r < nr ? __builtin_amdgcn_readlane(my_len, row[i]) - e : 0;
+                const int32_t* p = lists + (int64_t)(r0 + row[i]) * W + e;
+                x[i] = u32x4{~0u, ~0u, ~0u, ~0u};
+                if (left >= 4) {
+                    __builtin_memcpy(&x[i], p, 16);  // (rows are 4-byte aligned)
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 3; j++)
+                        if (j < left) x[i][j] = (uint32_t)p[j];
+                }
+                c += NWV;
+                next();
+            }
+#pragma unroll
+            for (int i = 0; i < AH; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t key = x[i][j] - (uint32_t)seg;  // (below seg: wraps past n)
+                    if ((int)x[i][j] >= 0 && key < (uint32_t)n) {
+                        atomicOr(&bm[key], 1u << row[i]);
+                        n_listed++;
+                    }
+                }
+        }
+        __syncthreads();
+        // a wave's share in steps of 256 keys, four a lane: counted, then placed
+        const int share = (n4 + 64 * NWV - 1) / (64 * NWV) * 64;  // (in quads)
+        const int i0 = min(n4, wave * share), i1 = min(n4, i0 + share);
+        auto quad = [&](int i) {
+            return i + lane < i1 ? ((const u32x4*)bm)[i + lane] : u32x4{0, 0, 0, 0};
+        };
+        int cnt = 0;
+        for (int i = i0; i < i1; i += 64) {
+            const u32x4 w = quad(i);
+            cnt += (w.x != 0) + (w.y != 0) + (w.z != 0) + (w.w != 0);
+            n_marked += __popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w);
+        }
+        for (int x = 1; x < 64; x <<= 1) cnt += __shfl_xor(cnt, x);
+        if (lane == 0) wave_n[wave] = cnt;
+        __syncthreads();
+        int pos = total;
+        for (int w = 0; w < NWV; w++) {
+            if (w < wave) pos += wave_n[w];
+            total += wave_n[w];
+        }
+        for (int i = i0; i < i1; i += 64) {
+            const u32x4 w = quad(i);
+            const int c = (w.x != 0) + (w.y != 0) + (w.z != 0) + (w.w != 0);
+            const uint64_t b0 = __ballot(c & 1), b1 = __ballot(c & 2), b2 = __ballot(c & 4);
+            const uint64_t lt = (1ull << lane) - 1;
+            int p = pos + __popcll(b0 & lt) + 2 * __popcll(b1 & lt) + 4 * __popcll(b2 & lt);
+            pos += __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (w[j] != 0) {
+                    if (p < cap) {
+                        gk[p] = seg + 4 * (i + lane) + j;
+                        gw[p] = w[j];
+                    }
+                    p++;
+                }
+        }
+    }
+    // a key that a row lists twice set one bit for two entries
+    if (n_listed) atomicAdd(&listed, n_listed);
+    if (n_marked) atomicAdd(&marked, n_marked);
+    __syncthreads();
+    const bool bad = listed != marked || total > max_union;
+    if (!bad) {
+        const int padded = (total + KT - 1) / KT * KT;  // <= cap
+        for (int i = total + tid; i < padded; i += kPlanThreads) {
+            gk[i] = 0;
+            gw[i] = 0;
+        }
+    }
+    if (tid == 0) counts[grp] = bad ? 0 : total;
+    for (int h = tid; h < hkv; h += kPlanThreads) flags[grp * hkv + h] = bad ? 1 : 0;
+}
+
+struct DlsaRowsArgs {
+    const void* q;  // [hq][L][D]
+    const void* k;  // element (h, t, d) at h * khs + t * krs + d
+    const void* v;
+    int64_t khs, krs, vhs, vrs;
+    void* out;       // [hq][L][D]
+    float* part_o;   // [hkv][n_split][PR][D] in V slot order, rows from prow0
+    float2* part_ml; // [hkv][n_split][PR] (m in log2 units)
+    const int32_t* keys;    // [groups][cap]
+    const uint32_t* words;
+    const int* counts;      // [groups]
+    int* flags;             // [groups][hkv]
+    int L, G, hkv, NR, cap, groups;
+    int n_main, qt0, n_split, prow0, PR;  // as RowsArgs (attend_rows.hip)
+    float scale2;           // scale * log2(e)
+};
+
+template <bool BF>
+struct Elem;
+template <>
+struct Elem<false> {
+    typedef half8 V8;
+    __device__ static float4v mfma(V8 a, V8 b, float4v c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+    typedef f16 T;
+};
+template <>
+struct Elem<true> {
+    typedef bhalf8 V8;
+    __device__ static float4v mfma(V8 a, V8 b, float4v c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+    typedef __bf16 T;
+};
+
+template <int D, bool BF>
+__global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
+    using S = BlockShape<D>;
+    using E = Elem<BF>;
+    using V8 = typename E::V8;
+    using ET = typename E::T;
+    constexpr int KT = S::KT, NSUB = S::NSUB, NM = S::NM, NT = S::NT, BUF = S::BUF, KBUF = S::KBUF;
+    constexpr int VROW = S::VROW, TPR = S::TPR, TPB = S::TPB;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    uint32_t* const sW = (uint32_t*)(lds + 2 * BUF);  // [2][KT] row words
+    int sp = 0, qt, h, n_split = 1;
+    {
+        const int lin = blockIdx.x;
+        if (lin < a.n_main) {
+            qt = lin / a.hkv;
+            h = lin % a.hkv;
+        } else {
+            const int t = lin - a.n_main;
+            n_split = a.n_split;
+            sp = t % n_split;
+            h = (t / n_split) % a.hkv;
+            qt = a.qt0 + t / (n_split * a.hkv);
+        }
+    }
+    if (a.flags[qt * a.hkv + h]) return;  // (uniform, before any barrier)
+    const int tid = threadIdx.x, lane = tid & 63;
+    {
+        // Where more than a quarter of the groups is left, the fp16 row kernel serves
+        // all of them: both launches are then long, and a mixture costs their sum
+        // (512 rows of which half share too little: 649 us, 364 us by rows alone).
+        int left = 0;
+        for (int i = 0; i < a.groups; i += 512)
+            left += __syncthreads_count(i + tid < a.groups && a.flags[(i + tid) * a.hkv + h] != 0);
+        if (!BF && 4 * left > a.groups) {
+            if (tid == 0) a.flags[qt * a.hkv + h] = 1;
+            return;
+        }
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int n_tiles = (a.counts[qt] + KT - 1) / KT, tps = (n_tiles + n_split - 1) / n_split;
+    const int t0 = sp * tps, t1 = min(n_tiles, t0 + tps);
+    // columns: (row of the group, head), row * G + head
+    const int R = a.L * a.G, row0 = qt * a.NR * a.G, row_end = min(R, row0 + a.NR * a.G);
+    const int wrow0 = row0 + 16 * wave, rho = wrow0 + r16;
+    const bool wave_live = wrow0 < row_end, row_ok = rho < row_end;
+    const int r = row_ok ? rho / a.G : 0, qh = h * a.G + (row_ok ? rho - r * a.G : 0);
+    const int bit = row_ok ? r - qt * a.NR : 0;  // the column's row in the words
+    // the rows of the wave's columns
+    const int b_lo = wave_live ? (wrow0 - row0) / a.G : 0;
+    const int b_hi = wave_live ? (min(row_end, wrow0 + 16) - 1 - row0) / a.G : 0;
+    const uint32_t need = (b_hi - b_lo == 31 ? ~0u : ((1u << (b_hi - b_lo + 1)) - 1)) << b_lo;
+
+    V8 qb[NM];
+    {
+        const ET* qrow = (const ET*)a.q + ((int64_t)qh * a.L + r) * D;
+#pragma unroll
+        for (int m = 0; m < NM; m++) qb[m] = *(const V8*)(qrow + 32 * m + 8 * g);
+    }
+
+    // tile loads: the 32-dim slice q32 of key kk of K, and 4 dims from 4 vj of
+    // the 8 keys of block vb of V (64 lanes read whole rows); the keys of the
+    // tile after the one being loaded are already in registers
+    static_assert(KT * TPR == 512 && (KT / 8) * TPB == 512, "one slice of each kind a thread");
+    const int q32 = (tid >> 4) & (TPR - 1), kk = (tid & 15) | ((tid >> (4 + S::LTPR)) << 4);
+    const int vb = tid / TPB, vj = tid % TPB;
+    const uint16_t* const kh = (const uint16_t*)a.k + h * a.khs + 32 * q32;
+    const uint16_t* const vh = (const uint16_t*)a.v + h * a.vhs + 4 * vj;
+    const int32_t* const gk = a.keys + (int64_t)qt * a.cap;
+    const uint32_t* const gw = a.words + (int64_t)qt * a.cap;
+    int ki, vi[8];
+    auto index = [&](int t) {
+        ki = gk[t * KT + kk];
+        const int32_t* p = gk + t * KT + 8 * vb;
+#pragma unroll
+        for (int i = 0; i < 8; i++) vi[i] = p[i];
+    };
+    u32x4 kc[4];
+    ushort4v vr[8];
+    uint32_t word;
+    auto load = [&](int t) {
+        const u32x4* ks = (const u32x4*)(kh + ki * a.krs);
+#pragma unroll
+        for (int w = 0; w < 4; w++) kc[w] = ks[w];
+#pragma unroll
+        for (int i = 0; i < 8; i++) vr[i] = *(const ushort4v*)(vh + vi[i] * a.vrs);
+        if (tid < KT) word = gw[t * KT + tid];
+    };
+    auto store = [&](int b) {
+        u32x4* const sK = (u32x4*)(lds + BUF * b) + kaddr<KT>(kk, 4 * q32);
+        ushort8v* const sV = (ushort8v*)(lds + BUF * b + KBUF) + vb * VROW;
+#pragma unroll
+        for (int w = 0; w < 4; w++) sK[w * KT] = kc[w];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            ushort8v y;
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = vr[i][e];
+            const int sl = v_phys_dim(4 * vj + e, D, 16);
+            sV[sl + (sl >> 4)] = y;
+        }
+        if (tid < KT) sW[b * KT + tid] = word;
+    };
+
+    float m_run = -INFINITY, l_run = 0.0f;
+    float4v acc_o[NT];
+#pragma unroll
+    for (int mm = 0; mm < NT; mm++) acc_o[mm] = float4v{0.f, 0.f, 0.f, 0.f};
+
+    // NU 32-key sub-blocks from sub-block ub of buffer b
+    constexpr int NU = NSUB < 4 ? NSUB : 4;
+    auto tile = [&](int b, int ub) {
+        const V8* sK8 = (const V8*)(lds + BUF * b) + 32 * ub;
+        const V8* sV8 = (const V8*)(lds + BUF * b + KBUF) + 4 * ub * VROW;
+        // the lane's keys 32u + 8g + e
+        uint32_t w[NU][8], all = ~0u, any = 0;
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+            const u32x4* p = (const u32x4*)(sW + b * KT + 32 * (ub + u) + 8 * g);
+            const u32x4 x = p[0], y = p[1];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                w[u][e] = e < 4 ? x[e & 3] : y[e & 3];
+                all &= w[u][e];
+                any |= w[u][e];
+            }
+        }
+        if (!__any((any & need) != 0)) return;  // none of the wave's rows lists any of them
+        const bool full = __all((all & need) == need);
+        const int key0 = 8 * (r16 >> 2) + (r16 & 3);
+        const int b4 = (key0 >> 4) & 1;
+        const V8* kbase0 = sK8 + g * KT + key0 + 4 * b4;
+        const V8* kbase1 = sK8 + g * KT + key0 + 4 * (b4 ^ 1);
+        float4v acc[NU][2];
+#pragma unroll
+        for (int u = 0; u < NU; u++) acc[u][0] = acc[u][1] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NM; m++)
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const V8 ka = kbase0[4 * m * KT + 32 * u], kb2 = kbase1[4 * m * KT + 32 * u];
+                acc[u][0] = E::mfma(ka, qb[m], acc[u][0]);
+                acc[u][1] = E::mfma(kb2, qb[m], acc[u][1]);
+            }
+        {
+            constexpr int NQ = NM * NU * 2, AH = 4;
+            __builtin_amdgcn_sched_group_barrier(0x100, AH, 0);
+#pragma unroll
+            for (int i = 0; i < NQ - AH; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, AH, 0);
+        }
+        float sf[NU][8];
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) sf[u][e] = acc[u][e >> 2][e & 3] * a.scale2;
+        if (!full) {
+#pragma unroll
+            for (int u = 0; u < NU; u++)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (((w[u][e] >> bit) & 1u) == 0) sf[u][e] = -INFINITY;
+        }
+        float mx = sf[0][0];
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) mx = fmaxf(mx, sf[u][e]);
+        // lazy reference in log2 units (p <= 2^5.5)
+        if (__any(mx > m_run + 5.5f)) {
+            const float m_new = fmaxf(m_run, wave_max_g(mx));
+            if (__any(m_run != -INFINITY)) {
+                const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                l_run *= alpha;
+                float f[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) f[i] = __shfl(alpha, 4 * g + i);
+#pragma unroll
+                for (int mm = 0; mm < NT; mm++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc_o[mm][i] *= f[i];
+            }
+            m_run = m_new;
+        }
+        const float mref = m_run == -INFINITY ? 0.0f : m_run;
+        V8 ph[NU], pl[NU];
+#pragma unroll
+        for (int u = 0; u < NU; u++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float p = __builtin_amdgcn_exp2f(sf[u][e] - mref);
+                l_run += p;
+                ph[u][e] = (ET)p;
+                pl[u][e] = (ET)(p - (float)ph[u][e]);
+            }
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+            const V8* vb8 = sV8 + (4 * u + g) * VROW + r16;
+#pragma unroll
+            for (int mm = 0; mm < NT; mm++) {
+                const V8 vv = vb8[17 * mm];
+                acc_o[mm] = E::mfma(ph[u], vv, acc_o[mm]);
+                acc_o[mm] = E::mfma(pl[u], vv, acc_o[mm]);
+            }
+        }
+        {
+            constexpr int NQ = NU * NT, AH = 4;
+            __builtin_amdgcn_sched_group_barrier(0x100, AH, 1);
+#pragma unroll
+            for (int i = 0; i < NQ - AH; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 2 * AH, 1);
+        }
+    };
+
+    // round t: tile t+1 (in registers) into the free buffer, the loads of tile
+    // t+2 and the key indexes of tile t+3, tile t's math; one barrier
+    if (t0 < t1) {
+        index(t0);
+        load(t0);
+        if (t0 + 1 < t1) index(t0 + 1);
+        store(0);
+        if (t0 + 1 < t1) load(t0 + 1);
+        if (t0 + 2 < t1) index(t0 + 2);
+    }
+    __syncthreads();
+    for (int t = t0; t < t1; t++) {
+        const int b = (t - t0) & 1;
+        if (t + 1 < t1) {
+            store(b ^ 1);
+            if (t + 2 < t1) load(t + 2);
+            if (t + 3 < t1) index(t + 3);
+        }
+        if (wave_live) {
+#pragma unroll
+            for (int ub = 0; ub < NSUB; ub += NU) tile(b, ub);
+        }
+        __syncthreads();
+    }
+
+    const float lsum = wave_sum_g(l_run);
+    if (n_split == 1) {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float l = __shfl(lsum, 4 * g + i);
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const int row = wrow0 + 4 * g + i;
+            if (row >= row_end) continue;
+            ET* orow = (ET*)a.out + ((int64_t)(h * a.G + row % a.G) * a.L + row / a.G) * D;
+            // slot 16mm + r16 is dim NT r16 + mm: a lane's NT dims are consecutive
+#pragma unroll
+            for (int mm = 0; mm < NT; mm++) {
+                const float o = acc_o[mm][i] * inv;
+                bad |= !(fabsf(o) < INFINITY);
+                orow[NT * r16 + mm] = (ET)o;
+            }
+            bad |= !(fabsf(l) < INFINITY);
+        }
+        if (bad) a.flags[qt * a.hkv + h] = 1;
+    } else {
+        const int64_t pbase = ((int64_t)h * n_split + sp) * a.PR - a.prow0;
+        if (g == 0 && row_ok) a.part_ml[pbase + rho] = float2{m_run, lsum};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = wrow0 + 4 * g + i;
+            if (row >= row_end) continue;
+            float* prow = a.part_o + (pbase + row) * D;
+#pragma unroll
+            for (int mm = 0; mm < NT; mm++) prow[16 * mm + r16] = acc_o[mm][i];
+        }
+    }
+}
+
+// out row = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s over the splits, in the
+// element type. grid (rows of the split groups / 4, KV heads), a wave a row, a lane
+// D / 64 consecutive slots, the partials loaded four at a time.
+template <int D, bool BF>
+__global__ __launch_bounds__(256) void dlsa_rows_merge_kernel(DlsaRowsArgs a) {
+    using ET = typename Elem<BF>::T;
+    constexpr int SPL = D / 64;
+    typedef float vec __attribute__((ext_vector_type(SPL)));
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int pr = blockIdx.x * 4 + wave, h = blockIdx.y;
+    if (pr >= a.PR) return;
+    const int row = a.prow0 + pr, grp = row / (a.NR * a.G), fl = grp * a.hkv + h;
+    if (a.flags[fl]) return;  // left to the row kernel
+    const int64_t base = (int64_t)h * a.n_split * a.PR + pr;
+    float M = -INFINITY, l = 0.0f;
+    vec o = {};
+    for (int c0 = 0; c0 < a.n_split; c0 += 4) {
+        float2 ml[4];
+        vec x[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int64_t at = base + (int64_t)min(c0 + i, a.n_split - 1) * a.PR;
+            ml[i] = a.part_ml[at];
+            x[i] = *(const vec*)(a.part_o + at * D + SPL * lane);
+            if (c0 + i >= a.n_split) ml[i] = float2{-INFINITY, 0.0f};
+        }
+        float m = M;
+#pragma unroll
+        for (int i = 0; i < 4; i++) m = fmaxf(m, ml[i].x);
+        if (m == -INFINITY) continue;
+        const float f0 = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - m);
+        o = o * f0;
+        l *= f0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float f = ml[i].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[i].x - m);
+            o += f * x[i];
+            l = __builtin_fmaf(f, ml[i].y, l);
+        }
+        M = m;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int r = row / a.G, qh = h * a.G + row % a.G;
+    ET* const orow = (ET*)a.out + ((int64_t)qh * a.L + r) * D;
+    bool bad = !(fabsf(l) < INFINITY);
+#pragma unroll
+    for (int j = 0; j < SPL; j++) {
+        const float y = o[j] * inv;
+        bad |= !(fabsf(y) < INFINITY);
+        orow[v_logical_dim(SPL * lane + j, D, 16)] = (ET)y;
+    }
+    if (bad) a.flags[fl] = 1;
+}
+
+std::mutex g_plan_mu;
+std::map<std::pair<int, hipStream_t>, GrowBuffer> g_plan_ws;
+
+template <int D, bool BF>
+int launch_rows(const DlsaRowsArgs& a, int grid, hipStream_t stream) {
+    const size_t shmem = 2 * BlockShape<D>::BUF + 2 * BlockShape<D>::KT * sizeof(uint32_t);
+    if (int rc = ensure_dynamic_lds((const void*)dlsa_rows_kernel<D, BF>, shmem)) return rc;
+    hipLaunchKernelGGL((dlsa_rows_kernel<D, BF>), dim3(grid), dim3(512), shmem, stream, a);
+    QW_HIP_CHECK(hipGetLastError());
+    if (a.n_split > 1) {
+        hipLaunchKernelGGL((dlsa_rows_merge_kernel<D, BF>), dim3((a.PR + 3) / 4, a.hkv), dim3(256), 0,
+                           stream, a);
+        QW_HIP_CHECK(hipGetLastError());
+    }
+    return QW_OK;
+}
+
+}  // namespace
+
+// A group's union may hold 0.35 of its rows' entries less 1500 keys (the launches'
+// fixed cost): there the tiles cost what gathering the rows by pairs does (512 rows
+// in groups of 20, D = 256: of 2048 entries 334 against 364 us at 0.3, 407 at 0.4; of
+// 512 entries 98 against 106 us at 0.2, 126 at 0.3). The typed kernel behind the bf16
+// calls takes fifteen times as long a row (512 rows of 4612: 7.6 ms), so there any
+// union is served.
+static int64_t union_limit(int width, int NR, bool bf16) {
+    return (int64_t)((bf16 ? 1.0 : 0.35) * NR * width) - (bf16 ? 0 : 1500);
+}
+
+int dlsa_rows_per_group(int G) { return std::min(32, 128 / G) & ~1; }
+
+int dlsa_rows_attention(const void* q, const void* k, const void* v, bool bf16, int64_t khs,
+                        int64_t krs, int64_t vhs, int64_t vrs, const int32_t* lists,
+                        const int32_t* lengths, int n_rows, int width, int n_q_heads,
+                        int n_kv_heads, int D, int n_keys, float scale, void* out,
+                        const int** flags, hipStream_t stream) {
+    const int G = n_q_heads / n_kv_heads, NR = dlsa_rows_per_group(G);
+    const int KT = 16384 / D, groups = (n_rows + NR - 1) / NR;
+    const int64_t most = std::min<int64_t>(n_keys, (int64_t)NR * width);
+    const int max_union = (int)std::min<int64_t>(most, std::max<int64_t>(KT, union_limit(width, NR, bf16)));
+    const int cap = (max_union + KT - 1) / KT * KT;
+    // whole rounds of unsplit workgroups, the rest split over their keys
+    DlsaRowsArgs a;
+    const int units = groups * n_kv_heads;
+    int q_main = 0;
+    if (units >= 256 && 256 % n_kv_heads == 0) q_main = units / 256 * (256 / n_kv_heads);
+    const int tail = (groups - q_main) * n_kv_heads;
+    const int tiles = (width + KT - 1) / KT;
+    a.n_split = tail > 0 ? std::max(1, std::min({256 / tail, tiles / 2, 32})) : 1;
+    a.n_main = q_main * n_kv_heads;
+    a.qt0 = q_main;
+    a.prow0 = q_main * NR * G;
+    a.PR = n_rows * G - a.prow0;
+    const size_t n_part = a.n_split > 1 ? (size_t)n_kv_heads * a.n_split * a.PR : 0;
+    const size_t part_bytes = n_part * (D * sizeof(float) + sizeof(float2));
+    const size_t list_bytes = (size_t)groups * cap * sizeof(int32_t);
+    const size_t count_bytes = (size_t)(groups + 3) / 4 * 4 * sizeof(int);
+    int dev = 0;
+    QW_HIP_CHECK(hipGetDevice(&dev));
+    void* ws = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_plan_mu);
+        GrowBuffer& b = g_plan_ws[{dev, stream}];
+        b.stream_owned = true;
+        if (int rc = b.get(part_bytes + 2 * list_bytes + count_bytes + (size_t)units * sizeof(int), stream, &ws))
+            return rc;
+    }
+    char* p = (char*)ws;
+    a.part_o = (float*)p;
+    a.part_ml = (float2*)(p + n_part * D * sizeof(float));
+    p += part_bytes;
+    int32_t* keys = (int32_t*)p;
+    uint32_t* words = (uint32_t*)(p + list_bytes);
+    int* counts = (int*)(p + 2 * list_bytes);
+    a.flags = (int*)(p + 2 * list_bytes + count_bytes);
+    a.keys = keys;
+    a.words = words;
+    a.counts = counts;
+    a.q = q;
+    a.k = k;
+    a.v = v;
+    a.khs = khs;
+    a.krs = krs;
+    a.vhs = vhs;
+    a.vrs = vrs;
+    a.out = out;
+    a.L = n_rows;
+    a.G = G;
+    a.hkv = n_kv_heads;
+    a.NR = NR;
+    a.cap = cap;
+    a.groups = groups;
+    a.scale2 = scale * kLog2e;
+    *flags = a.flags;
+    const size_t plan_lds = (size_t)(std::min(n_keys, kPlanSeg) + 3) / 4 * 16;
+    if (int rc = ensure_dynamic_lds((const void*)dlsa_plan_kernel, (size_t)kPlanSeg * sizeof(uint32_t)))
+        return rc;
+    hipLaunchKernelGGL(dlsa_plan_kernel, dim3(groups), dim3(kPlanThreads), plan_lds, stream, lists,
+                       lengths, n_rows, width, n_keys, NR, KT, max_union, cap, n_kv_heads, keys, words,
+                       counts, a.flags);
+    QW_HIP_CHECK(hipGetLastError());
+    const int grid = a.n_main + (groups - q_main) * n_kv_heads * a.n_split;
+    if (bf16)
+        return D == 256   ? launch_rows<256, true>(a, grid, stream)
+               : D == 128 ? launch_rows<128, true>(a, grid, stream)
+                          : launch_rows<64, true>(a, grid, stream);
+    return D == 256   ? launch_rows<256, false>(a, grid, stream)
+           : D == 128 ? launch_rows<128, false>(a, grid, stream)
+                      : launch_rows<64, false>(a, grid, stream);
+}
+
+}  // namespace qw

@@ -81,6 +81,9 @@ struct TypedArgs {
     float2* part_ml;         // [parts][L][hq]
     int L, W, hq, G, T, parts;
     float scale;
+    // != null: only the rows of the groups flagged there (dlsa_rows.hip left them)
+    const int* flags;  // [ceil(L / group_rows)][KV heads]
+    int group_rows;
 };
 
 // Waves a workgroup at most: 16 (the reference's simdgroups range), 8 at
@@ -99,6 +102,7 @@ __global__ __launch_bounds__(64 * typed_max_waves<D>()) void dlsa_typed_kernel(T
     constexpr int EPW = 64 / LPE;         // entries a wave step
     constexpr int DPL = D / LPE;          // dims a lane
     const int part = blockIdx.x, row = blockIdx.y, h = blockIdx.z;
+    if (a.flags && !a.flags[row / a.group_rows * gridDim.z + h]) return;
     const int NW = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int sub = lane / LPE, sl = lane % LPE;
     const int G = a.G;
@@ -286,11 +290,13 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     QW_REQUIRE((uintptr_t)q % dtype_size(q_dtype) == 0 && (uintptr_t)k % es == 0 &&
                    (uintptr_t)v % es == 0 && (uintptr_t)out % dtype_size(q_dtype) == 0,
                QW_ERR_UNSUPPORTED, "dlsa_sparse_attention_typed: misaligned pointer");
+    bool auto_one_pass = false;
     if (parts <= 0) {
         // the reference's policy shape (mlx_cxx_dlsa_attention.cpp:379-400): one pass when
         // the rows and KV heads alone give enough workgroups, else split each list
         const int units = n_rows * n_kv_heads;
         parts = units >= 192 ? 1 : std::min(kTypedMaxParts, std::max(1, std::min(192 / units, width / 16)));
+        auto_one_pass = parts == 1 && waves == 0;
     }
     parts = std::max(1, std::min(parts, kTypedMaxParts));
     const int nw = waves > 0 ? waves : 4;
@@ -316,6 +322,27 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     a.T = n_keys;
     a.parts = parts;
     a.scale = scale;
+    a.flags = nullptr;
+    a.group_rows = 1;
+    // bf16 throughout and laid out for 16-byte row pieces: neighbouring rows share
+    // their keys' gathers (dlsa_rows.hip), and the kernel here serves the groups
+    // which that leaves (or every row, without room for its lists). From 20k entries
+    // over all heads: 512 rows of 4612 entries (24 heads over 4, D = 256) 7572 -> 157
+    // us, 48 rows of 128 79 -> 33 to 54 us.
+    const bool aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 &&
+                         khs % 8 == 0 && krs % 8 == 0 && vhs % 8 == 0 && vrs % 8 == 0;
+    if (auto_one_pass && q_dtype == QW_DTYPE_BF16 && kv_dtype == QW_DTYPE_BF16 && head_dim >= 64 &&
+        aligned && (int64_t)n_rows * width * n_kv_heads >= 20000) {
+        const int rc = dlsa_rows_attention(q, k, v, true, khs, krs, vhs, vrs, lists, lengths, n_rows,
+                                           width, n_q_heads, n_kv_heads, head_dim, n_keys, scale, out,
+                                           &a.flags, stream);
+        if (rc == QW_OK)
+            a.group_rows = dlsa_rows_per_group(G);
+        else if (rc != QW_ERR_STATE && rc != QW_ERR_OUT_OF_MEMORY)
+            return rc;
+        else
+            a.flags = nullptr;
+    }
     if (parts > 1) {
         const size_t no = (size_t)parts * n_rows * n_q_heads;
         void* ws = nullptr;

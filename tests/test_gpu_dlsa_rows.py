@@ -1,0 +1,125 @@
+"""GPU parity of the D-LSA read for prefill row counts (dlsa_rows.hip: groups of neighbouring rows
+read the union of their keys once) against the float64 restatement, where it can go wrong: lists
+that share all, some or none of their keys, entries that are -1 or out of range, a key listed
+twice, ragged and zero lengths, a last group that is not full, unions around a tile, keys past one
+bitmap pass, infinite values that only some rows list.
+
+fp16: the attention tolerance (2e-3 max-abs, 1e-3 relative L2). bf16: the output's rounding, half
+a unit of 2^-8 relative to each value, plus 1e-5 of the row for the 32-bit sums."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import rng
+from test_gpu_kv import _gpu, _np, assert_close
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _lists(r, kind, L, W, T):
+    if kind == "shared":     # one set for all rows, each row in its own order
+        base = r.choice(T, W, replace=False)
+        return np.stack([r.permutation(base) for _ in range(L)]).astype(np.int32)
+    if kind == "sliding":    # a shared half and a window that moves by one
+        base = np.sort(r.choice(T - W - L, W - W // 2, replace=False))
+        return np.stack([np.concatenate([base, T - L - W // 2 + i + np.arange(W // 2)])
+                         for i in range(L)]).astype(np.int32)
+    if kind == "own":        # nothing in common but chance
+        return np.stack([r.choice(T, W, replace=False) for _ in range(L)]).astype(np.int32)
+    if kind == "mixed":      # the groups of the first half share, the others do not
+        a = _lists(r, "sliding", L // 2, W, T)
+        return np.concatenate([a, _lists(r, "own", L - L // 2, W, T)])
+    raise ValueError(kind)
+
+
+def _check(out, q, k, v, lists, lengths, scale, bf16, what):
+    ref = oracle.dlsa_attention_f64(q, k, v, lists, lengths, scale)
+    assert np.isfinite(out).all(), what
+    if not bf16:
+        assert_close(out, ref.astype(np.float32), what)
+        return
+    bound = np.abs(ref) * 2.0 ** -8 + 1e-5 * np.linalg.norm(ref, axis=-1, keepdims=True)
+    assert np.all(np.abs(out.astype(np.float64) - ref) <= bound), what
+
+
+def _run(q, k, v, lists, lengths, scale, bf16):
+    import qw_amd
+
+    if not bf16:
+        return _np(qw_amd.sparse_attention(_gpu(q), _gpu(k), _gpu(v), _gpu(lists), _gpu(lengths),
+                                           scale))[0]
+    t = [_gpu(x).to(torch.bfloat16) for x in (q, k, v)]
+    return qw_amd.sparse_attention_typed(*t, _gpu(lists), _gpu(lengths), scale)[0].float().cpu().numpy()
+
+
+CASES = [
+    # hq, hkv, D, L, T, W, kind (fp16 calls take the kernel from 96 rows and 850k entries over all heads)
+    (24, 4, 256, 101, 8000, 2200, "sliding"),   # the last group one row
+    (24, 4, 256, 700, 2000, 320, "shared"),     # the union exactly five tiles
+    (24, 4, 256, 700, 2000, 321, "shared"),     # one key past them
+    (24, 4, 256, 112, 40000, 2000, "own"),      # every group left to the row kernel (fp16)
+    (24, 4, 256, 160, 40000, 1400, "mixed"),
+    (8, 8, 128, 130, 4000, 900, "sliding"),     # G = 1: 32 rows a group
+    (24, 3, 128, 96, 6000, 3000, "sliding"),    # KV heads that do not divide 256
+    (16, 2, 64, 300, 9000, 1500, "sliding"),    # 256-key tiles in two halves
+    (16, 1, 128, 600, 4000, 1500, "shared"),    # G = 16: 8 rows a group
+    (24, 4, 256, 96, 90000, 2300, "sliding"),   # three bitmap passes
+    (24, 4, 256, 1300, 2600, 400, "sliding"),   # whole rounds and a split rest
+]
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("hq,hkv,D,L,T,W,kind", CASES)
+def test_rows_match_oracle(hq, hkv, D, L, T, W, kind, bf16):
+    print(f"case hq={hq} hkv={hkv} D={D} L={L} T={T} W={W} {kind} bf16={bf16}", flush=True)
+    assert L >= 96 and L * W * hkv >= 850000, "a shape of the kernel"
+    if bf16 and hq // hkv > 8:
+        pytest.skip("the typed read takes at most 8 heads a KV head")
+    r = rng(hq + D + L + T + W)
+    f = (lambda x: torch.from_numpy(x).to(torch.bfloat16).float().numpy()) if bf16 else (
+        lambda x: x.astype(np.float16))
+    q, k, v = (f(r.standard_normal(s).astype(np.float32))
+               for s in ((hq, L, D), (hkv, T, D), (hkv, T, D)))
+    lists = _lists(r, kind, L, W, T)
+    lists[::5, 3::11] = -1
+    lists[::7, 5::13] = T + 4
+    lengths = np.where(np.arange(L) % 9 == 4, r.integers(0, W, L), W).astype(np.int32)
+    lengths[2] = 0
+    out = _run(q, k, v, lists, lengths, D ** -0.5, bf16)
+    assert np.all(out[:, 2] == 0)
+    _check(out, q, k, v, lists, lengths, D ** -0.5, bf16, f"{kind} D={D} L={L}")
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_a_key_listed_twice_counts_twice(bf16):
+    r = rng(3)
+    hq, hkv, D, L, T, W = 24, 4, 128, 100, 5000, 2200
+    f = (lambda x: torch.from_numpy(x).to(torch.bfloat16).float().numpy()) if bf16 else (
+        lambda x: x.astype(np.float16))
+    q, k, v = (f(r.standard_normal(s).astype(np.float32))
+               for s in ((hq, L, D), (hkv, T, D), (hkv, T, D)))
+    lists = _lists(r, "shared", L, W, T)
+    lists[50, 7] = lists[50, 2080]
+    lengths = np.full(L, W, np.int32)
+    out = _run(q, k, v, lists, lengths, 0.1, bf16)
+    _check(out, q, k, v, lists, lengths, 0.1, bf16, "a key twice")
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_infinite_values_stay_with_the_rows_that_list_them(bf16):
+    r = rng(4)
+    hq, hkv, D, L, T, W = 24, 4, 128, 100, 5000, 2200
+    f = (lambda x: torch.from_numpy(x).to(torch.bfloat16).float().numpy()) if bf16 else (
+        lambda x: x.astype(np.float16))
+    q, k, v = (f(r.standard_normal(s).astype(np.float32))
+               for s in ((hq, L, D), (hkv, T, D), (hkv, T, D)))
+    lists = np.stack([r.permutation(T - 1)[:W] for _ in range(2)])[np.zeros(L, int)].astype(np.int32)
+    lists[41, 3] = T - 1
+    v[:, T - 1, 5] = np.inf
+    lengths = np.full(L, W, np.int32)
+    out = _run(q, k, v, lists, lengths, 0.1, bf16)
+    rows = np.setdiff1d(np.arange(L), [40, 41])  # (row 40 is row 41's pair in the row kernel)
+    _check(out[:, rows], q[:, rows], k, np.where(np.isinf(v), 0, v), lists[rows], lengths[rows], 0.1,
+           bf16, "rows without the infinite key")
+    assert not np.isfinite(out[:, 41, 5]).any()
