@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <climits>
 #include <map>
 #include <mutex>
 #include <string>
@@ -317,9 +318,68 @@ __global__ __launch_bounds__(256) void append_affine_kernel(
                     fast_flag, t_old / 8 + blockIdx.x, blockIdx.y, threadIdx.x, blockDim.x, sc);
 }
 
-// fp16 mode append: K rows copied, V scattered into 8-key blocks.
+// fp16 mode append: K rows copied, V transposed into 8-key blocks. A thread takes
+// 8 dims of one block's 8 tokens: 16-byte loads of both (all issued first), K rows
+// stored as they are, a dim's 8 keys of V as one 16-byte piece where the append
+// fills the block (single elements where it does not). HBM-bound; 131072 rows of 4
+// heads, D = 256: 730 us an element a thread -> 198 us.
 template <int D>
 __global__ __launch_bounds__(256) void append_fp16_kernel(RowSrc rs, int n_tokens, int t_old,
+                                                          int cap, f16* __restrict__ k_data,
+                                                          f16* __restrict__ v_data) {
+    constexpr int OCT = D / 8;
+    const int h = blockIdx.y, unit = blockIdx.x * 256 + threadIdx.x;
+    const int blk = t_old / 8 + unit / OCT, d0 = unit % OCT * 8;
+    const int r0 = 8 * blk - t_old;  // the source row of the block's first key
+    if (r0 >= n_tokens) return;
+    // (rows and pieces off 16 bytes: the caller's pointers and strides decide)
+    const bool wide = (((uintptr_t)rs.k | (uintptr_t)rs.v) % 16 == 0) && rs.row_stride % 8 == 0 &&
+                      rs.head_stride % 8 == 0;
+    half8 kr[8], vr[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int r = min(max(r0 + i, 0), n_tokens - 1);
+        const int64_t src = (int64_t)r * rs.row_stride + (int64_t)h * rs.head_stride + d0;
+        if (wide) {
+            kr[i] = *(const half8*)(rs.k + src);
+            vr[i] = *(const half8*)(rs.v + src);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                kr[i][e] = rs.k[src + e];
+                vr[i][e] = rs.v[src + e];
+            }
+        }
+    }
+    const int64_t gblk = (int64_t)h * (cap / 8) + blk;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int r = r0 + i;
+        if (r < 0 || r >= n_tokens) continue;
+        *(half8*)(k_data + (gblk * 8 + i) * D + d0) = kr[i];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        f16* p = v_data + (gblk * D + v_phys_dim(d0 + e, D, 16)) * 8;
+        if (r0 >= 0 && r0 + 8 <= n_tokens) {
+            half8 y;
+#pragma unroll
+            for (int i = 0; i < 8; i++) y[i] = vr[i][e];
+            *(half8*)p = y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (r0 + i >= 0 && r0 + i < n_tokens) p[i] = vr[i][e];
+        }
+    }
+}
+
+// The same with an element a thread: K rotated on the load (the library's sine and
+// cosine are most of the work), and appends below a block, which would leave most of
+// the pieces above empty (one token into 131071: 58.0 against 59.2 us for the whole
+// sparse decode step).
+template <int D>
+__global__ __launch_bounds__(256) void append_fp16_elem_kernel(RowSrc rs, int n_tokens, int t_old,
                                                           int cap, f16* __restrict__ k_data,
                                                           f16* __restrict__ v_data) {
     const int h = blockIdx.y;
@@ -329,9 +389,8 @@ __global__ __launch_bounds__(256) void append_fp16_kernel(RowSrc rs, int n_token
         const int r = (int)(i / D), d = (int)(i % D);
         const int t = r + t_old;
         const int64_t src = (int64_t)r * rs.row_stride + (int64_t)h * rs.head_stride;
-        const f16 kv = rs.rope_dims > 0 ? (f16)rope_elem(rs.k + src, d, rs.rope_dims, rs.traditional,
-                                                       rs.log2_base, rs.scale, rs.position0 + r)
-                                        : rs.k[src + d];
+        const f16 kv = (f16)rope_elem(rs.k + src, d, rs.rope_dims, rs.traditional, rs.log2_base,
+                                      rs.scale, rs.position0 + r);
         const f16 vv = rs.v[src + d];
         k_data[((int64_t)h * cap + t) * D + d] = kv;
         v_data[(((int64_t)h * (cap / 8) + t / 8) * D + v_phys_dim(d, D, 16)) * 8 + (t & 7)] = vv;
@@ -377,16 +436,18 @@ int KVCache::update_rows(const RowSrc& rs, int n_tokens, hipStream_t stream) {
                                int8() ? 1 : 0, cap, (uint32_t*)k_data, k_params,
                                (uint32_t*)v_data, (f16*)v_params, fast_flag);
     } else {
-        const int64_t n = (int64_t)n_tokens * D;
-        dim3 grid((unsigned)std::min<int64_t>((n + 255) / 256, 1024), hkv);
+        const int nblk = (offset + n_tokens - 1) / 8 - offset / 8 + 1;
+        const bool elem = rs.rope_dims > 0 || n_tokens < 8;
+        const int64_t threads = elem ? (int64_t)n_tokens * D : (int64_t)nblk * (D / 8);
+        const dim3 grid((unsigned)std::min<int64_t>((threads + 255) / 256, elem ? 1024 : INT_MAX), hkv);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, rs, n_tokens, offset, cap,
+                               (f16*)k_data, (f16*)v_data);
+        };
         if (D == 256)
-            hipLaunchKernelGGL(append_fp16_kernel<256>, grid, dim3(256), 0, stream,
-                               rs, n_tokens, offset, cap,
-                               (f16*)k_data, (f16*)v_data);
+            elem ? launch(append_fp16_elem_kernel<256>) : launch(append_fp16_kernel<256>);
         else
-            hipLaunchKernelGGL(append_fp16_kernel<128>, grid, dim3(256), 0, stream,
-                               rs, n_tokens, offset, cap,
-                               (f16*)k_data, (f16*)v_data);
+            elem ? launch(append_fp16_elem_kernel<128>) : launch(append_fp16_kernel<128>);
     }
     QW_HIP_CHECK(hipGetLastError());
     offset += n_tokens;
@@ -407,48 +468,68 @@ __device__ inline f16 mlx_dequant(uint32_t c, int off, f16 s, f16 b) {
     return (f16)((float)prod + (float)b);
 }
 
-// One thread per (head, row, 8 dims); writes 16 bytes of K and of V.
-__global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict__ k_codes,
-                                                      const uint32_t* __restrict__ k_params,
-                                                      const uint32_t* __restrict__ v_codes,
-                                                      const f16* __restrict__ v_params,
-                                                      int bits, int code_off, int D, int cap,
-                                                      int hkv, int start, int n,
-                                                      f16* __restrict__ k_out,
-                                                      f16* __restrict__ v_out) {
-    const int64_t oct = D / 8;
-    const int64_t total = (int64_t)hkv * n * oct;
-    const int NG = D / kGroup;
-    const int nw = D * bits / 32;
-    const uint32_t m = (1u << bits) - 1u;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int h = (int)(i / (n * oct));
-        const int r = (int)((i / oct) % n);
-        const int d0 = (int)(i % oct) * 8;
-        const int t = start + r;
-        const int g = d0 / kGroup;
-        const half2v ksb = __builtin_bit_cast(
-            half2v, k_params[((int64_t)h * cap + t) * NG + k_param_slot(g, NG)]);
-        const f16* vp = v_params + (((int64_t)h * (cap / 8) + t / 8) * NG + g) * 16;
-        const f16 vs = vp[t & 7], vbias = vp[8 + (t & 7)];
-        const uint32_t* krow = k_codes + ((int64_t)h * cap + t) * nw;
-        const uint32_t* vblk = v_codes + ((int64_t)h * (cap / 8) + t / 8) * (D * bits / 4);
+// A thread takes 8 dims of the 8 keys of one V block: V's codes (fp16: values) as
+// 16-byte pieces that hold all 8 keys of a dim or two, K's as one word or two (16
+// bytes) a key, every load issued before the first is used; then a 16-byte store a
+// key and plane, 64 lanes covering whole rows. HBM-bound: 8192 rows of 4 heads, D =
+// 256, 4-bit (9.4 MB in, 33.6 out) in 8.8 us; one key a thread, each element's code
+// gathered for itself, took 26.4 us.
+template <int BITS, int D>
+__global__ __launch_bounds__(256) void fetch_kernel(const void* __restrict__ k_data,
+                                                    const uint32_t* __restrict__ k_params,
+                                                    const void* __restrict__ v_data,
+                                                    const f16* __restrict__ v_params, int code_off,
+                                                    int cap, int start, int n,
+                                                    f16* __restrict__ k_out,
+                                                    f16* __restrict__ v_out) {
+    constexpr int OCT = D / 8, NG = D / kGroup;
+    constexpr int NV = BITS / 2;       // 16-byte pieces of V
+    constexpr int E = 16 / BITS;       // dims a piece
+    constexpr int KW = BITS / 4;       // words of 8 dims of a K row
+    const int h = blockIdx.y, unit = blockIdx.x * 256 + threadIdx.x;
+    const int blk = start / 8 + unit / OCT, d0 = unit % OCT * 8, g = d0 / kGroup;
+    if (8 * blk >= start + n) return;
+    const int64_t gblk = (int64_t)h * (cap / 8) + blk;
+    u32x4 vc[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++)
+        vc[j] = ((const u32x4*)v_data)[(gblk * D + v_phys_dim(d0 + E * j, D, BITS)) / E];
+    u32x4 vs = {}, vb = {};
+    if constexpr (BITS != 16) {
+        const u32x4* vp = (const u32x4*)(v_params + (gblk * NG + g) * 16);
+        vs = vp[0];
+        vb = vp[1];
+    }
+    uint32_t kc[8][KW], ksb[8] = {};
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int64_t row = gblk * 8 + k;  // (rows of a block exist up to cap)
+        const uint32_t* p = (const uint32_t*)k_data + (row * D + d0) * BITS / 32;
+#pragma unroll
+        for (int w = 0; w < KW; w++) kc[k][w] = p[w];
+        if constexpr (BITS != 16) ksb[k] = k_params[row * NG + k_param_slot(g, NG)];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int r = 8 * blk + k - start;
+        if (r < 0 || r >= n) continue;
         half8 ko, vo;
+        const half2v sb = h2(ksb[k]);
+        const f16 s = h2(vs[k / 2])[k & 1], b = h2(vb[k / 2])[k & 1];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const int d = d0 + e;
-            const int epw = 32 / bits;
-            const uint32_t kcode = (krow[d / epw] >> ((d % epw) * bits)) & m;
-            ko[e] = mlx_dequant(kcode, code_off, ksb.x, ksb.y);
-            const int p = v_phys_dim(d, D, bits);
-            const int k = t & 7;
-            uint32_t vcode;
-            if (bits == 4)
-                vcode = (vblk[p] >> (4 * v4_nibble_pos(k))) & 0xFu;
-            else
-                vcode = (vblk[2 * p + (k >> 2)] >> (8 * (k & 3))) & 0xFFu;
-            vo[e] = mlx_dequant(vcode, code_off, vs, vbias);
+            // piece e / E holds dims in turn, each 32 / 64 / 128 bits of 8 keys
+            const u32x4 w = vc[e / E];
+            if constexpr (BITS == 16) {
+                ko[e] = h2(kc[k][e / 2])[e & 1];
+                vo[e] = h2(w[k / 2])[k & 1];
+            } else if constexpr (BITS == 8) {
+                ko[e] = mlx_dequant((kc[k][e / 4] >> (8 * (e & 3))) & 0xFFu, code_off, sb.x, sb.y);
+                vo[e] = mlx_dequant((w[2 * (e & 1) + k / 4] >> (8 * (k & 3))) & 0xFFu, code_off, s, b);
+            } else {
+                ko[e] = mlx_dequant((kc[k][0] >> (4 * e)) & 0xFu, code_off, sb.x, sb.y);
+                vo[e] = mlx_dequant((w[e & 3] >> (4 * v4_nibble_pos(k))) & 0xFu, code_off, s, b);
+            }
         }
         const int64_t o = ((int64_t)h * n + r) * D + d0;
         *(half8*)(k_out + o) = ko;
@@ -456,7 +537,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
     }
 }
 
-// fp16 mode: K rows copied; V gathered out of the 8-key blocks.
+// fp16 mode into outputs off 16-byte alignment: element by element.
 __global__ __launch_bounds__(256) void fetch_fp16_kernel(const f16* __restrict__ k_data,
                                                          const f16* __restrict__ v_data, int D,
                                                          int cap, int hkv, int start, int n,
@@ -482,17 +563,27 @@ int KVCache::dequantize(int start, int n, void* k_out, void* v_out, hipStream_t 
     QW_REQUIRE(k_out && v_out, QW_ERR_INVALID_ARGUMENT, "dequantize: null output");
     DeviceGuard dg(device);
     if (turbo4()) return turbo4_dequantize(start, n, k_out, v_out, stream);
-    const int64_t work = affine() ? (int64_t)hkv * n * (D / 8) : (int64_t)hkv * n * D;
-    const unsigned blocks = (unsigned)std::min<int64_t>((work + 255) / 256, 4096);
-    if (affine())
-        hipLaunchKernelGGL(dequant_kernel, dim3(blocks), dim3(256), 0, stream,
-                           (const uint32_t*)k_data, k_params, (const uint32_t*)v_data,
-                           (const f16*)v_params, bits, int8() ? 128 : 0, D, cap, hkv, start, n,
-                           (f16*)k_out, (f16*)v_out);
-    else
+    if (!affine() && (((uintptr_t)k_out | (uintptr_t)v_out) % 16) != 0) {
+        const unsigned blocks = (unsigned)std::min<int64_t>(((int64_t)hkv * n * D + 255) / 256, 4096);
         hipLaunchKernelGGL(fetch_fp16_kernel, dim3(blocks), dim3(256), 0, stream,
                            (const f16*)k_data, (const f16*)v_data, D, cap, hkv, start, n,
                            (f16*)k_out, (f16*)v_out);
+        QW_HIP_CHECK(hipGetLastError());
+        return QW_OK;
+    }
+    const int nblk = (start + n - 1) / 8 - start / 8 + 1;
+    const dim3 grid((unsigned)(((int64_t)nblk * (D / 8) + 255) / 256), hkv);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, k_data, k_params, v_data,
+                           (const f16*)v_params, int8() ? 128 : 0, cap, start, n, (f16*)k_out,
+                           (f16*)v_out);
+    };
+    if (D == 256)
+        bits == 4 ? launch(fetch_kernel<4, 256>)
+                  : bits == 8 ? launch(fetch_kernel<8, 256>) : launch(fetch_kernel<16, 256>);
+    else
+        bits == 4 ? launch(fetch_kernel<4, 128>)
+                  : bits == 8 ? launch(fetch_kernel<8, 128>) : launch(fetch_kernel<16, 128>);
     QW_HIP_CHECK(hipGetLastError());
     return QW_OK;
 }
