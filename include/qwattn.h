@@ -174,7 +174,9 @@ int qw_kv_attention(qw_kv_cache* cache, const void* q, int n_q_heads, int n_rows
  *     scores (in fp16 without softcap); a bool mask with softcap is refused
  *     (QW_ERR_UNSUPPORTED: the reference would cast it to 0/1 offsets);
  *   out [n_q_heads][n_rows][head_dim] fp16; a row with no visible key is 0.
- * A generic kernel (sdpa_general.hip), not the tuned fused paths. */
+ * Calls of many rows lay the key tiles out once and run the row kernel
+ * (attend_rows.hip; a per-stream workspace of about 1 KB a key and KV head at
+ * head_dim 256), the others a generic kernel (sdpa_general.hip). */
 int qw_sdpa(const void* q, int n_q_heads, int n_rows, const void* k, const void* v,
             int n_kv_heads, int n_keys, int head_dim, int64_t k_head_stride, int64_t k_row_stride,
             int64_t v_head_stride, int64_t v_row_stride, float scale, int causal, int window,
@@ -182,12 +184,14 @@ int qw_sdpa(const void* q, int n_q_heads, int n_rows, const void* k, const void*
             int64_t mask_row_stride, void* out, void* stream);
 
 /* The same over a cache (n_keys = its offset): without mask, softcap or
- * window it is qw_kv_attention; otherwise the cache's rows are dequantized
- * into a per-stream workspace and attended as qw_sdpa does, the route of the
- * runtime's masked branch (update_and_fetch + layers::attention,
- * qwen3_next.rs:316-324). On a Turbo4 cache: the rotated expansion, q rotated
- * in and the output rotated back (update_and_turbo4_attention with a mask,
- * cache.rs:3495 -> turbo/sparse_v.rs:1051-1072). The update form appends
+ * window it is qw_kv_attention; with one of them what the runtime's masked
+ * branch computes (update_and_fetch + layers::attention, qwen3_next.rs:
+ * 316-324): a mask alone, or a window or softcap without a mask, on the codes
+ * in place; the other combinations, and masked calls of more than 4096 query
+ * rows a KV head, over the rows dequantized into a per-stream workspace. On a
+ * Turbo4 cache: in the rotated basis, q rotated in and the output rotated back
+ * (update_and_turbo4_attention with a mask, cache.rs:3495 ->
+ * turbo/sparse_v.rs:1051-1072). The update form appends
  * k_new / v_new ([n_kv_heads][n_rows][head_dim]) first; invalid options are
  * refused before the append. */
 int qw_kv_attention_general(qw_kv_cache* cache, const void* q, int n_q_heads, int n_rows,

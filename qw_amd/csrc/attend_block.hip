@@ -96,6 +96,10 @@ struct BlockArgs {
     int window = 0;
     // CAP launches (a logit softcap): s = tanh(f16(q . k) scale / softcap) softcap
     float softcap = 0.0f, scale = 0.0f;
+    // MASK launches: an explicit mask [hq or broadcast][Tq][T], key stride 1
+    const void* mask = nullptr;
+    int mask_dtype = 0;
+    int64_t mask_hs = 0, mask_rs = 0;
     float t4_post;        // Turbo4 fused pass: scale * log2(e) in fp32
     float scale_h;      // f16(scale) as float
     uint32_t code_off2; // magic offset pair of the separately rounded dequant
@@ -185,8 +189,10 @@ constexpr bool kSetprio(int pm) {
 // PM (tile images): 0 none; 1 the expansion launch (workgroup (t, h) writes
 // the image of key tile t of head h and returns); 2 attention from the images
 // (each tile's LDS buffer copied in by LDS-DMA, no dequant in the loop).
+// MASK: an explicit mask (bool, or an fp16 term added to the fp16 score); the split
+// partials stay fp32.
 template <int BITS, int D, int RT, bool FAST, int T4M = 0, bool APP = false, int PM = 0,
-          bool ROPE = false, bool WIN = false, bool CAP = false>
+          bool ROPE = false, bool WIN = false, bool CAP = false, bool MASK = false>
 __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
     using S = BlockShape<D>;
     constexpr int KT = S::KT, NSUB = S::NSUB, NM = S::NM, NT = S::NT, NG = S::NG;
@@ -342,6 +348,7 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
     // mask) and of its first row (tiles wholly below it are skipped)
     const int wave_lo_max = WIN ? a.T - a.Tq + wave_last / a.G - a.window + 1 : 0;
     const int wave_lo_min = WIN ? a.T - a.Tq + wrow0 / a.G - a.window + 1 : 0;
+    int64_t moff[RT];  // (MASK) the row's mask entries
     half8 qb[RT][NM];
     // Turbo4: the workgroup's rows are rotated into the K basis (the rotation
     // kernels' arithmetic; wave w takes rows w, w + NW, ..., four at a time
@@ -470,6 +477,8 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
         lim[rt] = row_ok[rt] ? cut(a.causal ? a.T - a.Tq + rho / a.G : a.T - 1) : -1;
         wlo[rt] = WIN && row_ok[rt] ? a.T - a.Tq + rho / a.G - a.window + 1 : 0;
         const int rr = row_ok[rt] ? rho : 0;
+        if constexpr (MASK)
+            moff[rt] = (int64_t)(h * a.G + rr % a.G) * a.mask_hs + (int64_t)(rr / a.G) * a.mask_rs;
         // (Turbo4 padding rows read the workgroup's first staged row; their scale is 0)
         const f16* qrow = T4     ? sq + (row_ok[rt] ? wrow0 - row0 + 16 * rt + r16 : 0) * D
                           : ROPE ? sqr + (row_ok[rt] ? wrow0 - row0 + 16 * rt + r16 : 0) * D
@@ -679,6 +688,16 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
         const int b4 = (key0 >> 4) & 1;
         const half8* kbase0 = sK8 + g * KT + key0 + 4 * b4;
         const half8* kbase1 = sK8 + g * KT + key0 + 4 * (b4 ^ 1);
+        // the lane's 8 mask entries of each sub-block, requested before the MFMAs
+        u32x4 mraw[MASK ? NU : 1][2];
+        if constexpr (MASK) {
+            static_assert(!MASK || RT == 1, "one row tile a wave");
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const int t = kt0 + 32 * (ub + u) + 8 * g;
+                mask_load8(a.mask, a.mask_dtype, moff[0] + t, row_ok[0] ? a.T - t : 0, mraw[u]);
+            }
+        }
         float4v acc[NU][2][RT];
 #pragma unroll
         for (int u = 0; u < NU; u++)
@@ -846,6 +865,22 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
                         const float4v& av = acc[u][j >> 1][rt];
                         sh[u][j] = half2v{(f16)av[2 * (j & 1)], (f16)av[2 * (j & 1) + 1]};
                     }
+                if constexpr (MASK) {
+                    if (a.mask_dtype == QW_MASK_BOOL) {
+#pragma unroll
+                        for (int u = 0; u < NU; u++)
+#pragma unroll
+                            for (int e = 0; e < 8; e++)
+                                if (mask_hides(mraw[u], e)) sh[u][e >> 1][e & 1] = (f16)(-INFINITY);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < NU; u++)
+#pragma unroll
+                            for (int e = 0; e < 8; e++)
+                                sh[u][e >> 1][e & 1] = (f16)((float)sh[u][e >> 1][e & 1] +
+                                                             (float)mask_term(mraw[u], a.mask_dtype, e));
+                    }
+                }
                 if (mask) {
 #pragma unroll
                     for (int u = 0; u < NU; u++)
@@ -1128,7 +1163,7 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
                     a.out[obase + d] = (f16)(acc_o[rt][mm][i] * inv[i]);
                 }
             }
-        } else if constexpr (kPart16 && !FUSED) {
+        } else if constexpr (kPart16 && !FUSED && !MASK) {
             // fp16 partials: row O / l rounded once, lane r16's NT slots
             // 16 mm + r16 at places NT r16 + mm (whole 16-byte stores), and
             // (m, l) in fp32
@@ -1176,11 +1211,12 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
 }
 
 template <int BITS, int D, int RT, int T4M = 0, bool APP = false, int PM = 0, bool ROPE = false,
-          bool WIN = false, bool CAP = false>
+          bool WIN = false, bool CAP = false, bool MASK = false>
 __global__ __launch_bounds__(64 * block_waves<PM>(), 1) void attend_block_kernel(BlockArgs a) {
     static_assert(!ROPE || (APP && PM == 0), "RoPE launches are verify blocks that append");
     static_assert(!WIN || (PM == 0 && !APP && T4M == 0), "window launches attend a cache as it is");
     static_assert(!CAP || WIN, "softcap launches are window launches (an unbounded window)");
+    static_assert(!MASK || (PM == 0 && !APP && !WIN && T4M != 2), "masked launches attend a cache as it is");
     // two buffers, each a K and a V tile of KT keys in fp16 (~130 KB)
     extern __shared__ __attribute__((aligned(16))) char lds_buf[];
     // The exact 2-op dequant runs without waiting for the cache's fast flag;
@@ -1223,27 +1259,27 @@ __global__ __launch_bounds__(64 * block_waves<PM>(), 1) void attend_block_kernel
         // the images hold the dequantized tiles: no dequant, no fast flag
         block_body<BITS, D, RT, false, T4M, APP, 2>(a, lds_buf);
     } else if (T4M == 0 && (BITS == 16 || a.fast_flag != nullptr)) {
-        block_body<BITS, D, RT, true, 0, APP, PM, ROPE, WIN, CAP>(a, lds_buf);
+        block_body<BITS, D, RT, true, 0, APP, PM, ROPE, WIN, CAP, MASK>(a, lds_buf);
         if (BITS != 16 && *a.fast_flag == 0) {
             __syncthreads();
-            block_body<BITS, D, RT, false, 0, APP, PM, ROPE, WIN, CAP>(a, lds_buf);
+            block_body<BITS, D, RT, false, 0, APP, PM, ROPE, WIN, CAP, MASK>(a, lds_buf);
         }
     } else {
-        block_body<BITS, D, RT, false, T4M, APP, PM, ROPE, WIN, CAP>(a, lds_buf);
+        block_body<BITS, D, RT, false, T4M, APP, PM, ROPE, WIN, CAP, MASK>(a, lds_buf);
     }
 }
 
 template <int BITS, int D, int RT, int T4M, bool APP = false, int PM = 0, bool ROPE = false,
-          bool WIN = false, bool CAP = false>
+          bool WIN = false, bool CAP = false, bool MASK = false>
 static int launch_block_rt(KVCache& cc, BlockArgs& a, int n_qt, hipStream_t stream) {
     // two tile buffers (+ the Turbo4 centroid-pair table)
     const size_t shmem = (size_t)2 * BlockShape<D>::BUF + (T4M ? 256 * sizeof(float2) : 0);
-    int rc = ensure_dynamic_lds((const void*)attend_block_kernel<BITS, D, RT, T4M, APP, PM, ROPE, WIN, CAP>, shmem);
+    int rc = ensure_dynamic_lds((const void*)attend_block_kernel<BITS, D, RT, T4M, APP, PM, ROPE, WIN, CAP, MASK>, shmem);
     if (rc) return rc;
     const dim3 grid = a.n_app > 0    ? dim3(a.n_app + cc.hkv * (a.n_split - 1))
                       : a.n_main > 0 ? dim3(a.n_main + n_qt * cc.hkv * a.n_split)
                                      : dim3(a.n_split, n_qt, cc.hkv);
-    hipLaunchKernelGGL((attend_block_kernel<BITS, D, RT, T4M, APP, PM, ROPE, WIN, CAP>), grid, dim3(64 * block_waves<PM>()), shmem,
+    hipLaunchKernelGGL((attend_block_kernel<BITS, D, RT, T4M, APP, PM, ROPE, WIN, CAP, MASK>), grid, dim3(64 * block_waves<PM>()), shmem,
                        stream, a);
     QW_HIP_CHECK(hipGetLastError());
     return QW_OK;
@@ -1348,7 +1384,7 @@ static void split_keys(int n_tiles, int want, int* n_split, int* tps, int min_ti
 template <int BITS, int D, int T4M = 0>
 static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float scale, bool causal,
                              f16* out, hipStream_t stream, const float* t4_tab = nullptr,
-                             int window = 0, float softcap = 0.0f) {
+                             int window = 0, float softcap = 0.0f, const SdpaOptions* masked = nullptr) {
     using S = BlockShape<D>;
     const int T = cc.offset;
     const int R = G * Tq;
@@ -1356,7 +1392,7 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     // long prefill calls dequantize (fp16: lay out) each key tile once into an
     // image of its LDS buffer and attend from the images, in query tiles of
     // 16 kImageWaves rows
-    const bool images = QW_BLOCK_IMAGES && T4M != 2 && window <= 0 && softcap <= 0.0f &&
+    const bool images = QW_BLOCK_IMAGES && T4M != 2 && window <= 0 && softcap <= 0.0f && !masked &&
                         R >= (T4M ? kT4ImageMinRows : kImageMinRows) && n_tiles > 0;
     const int rt = images ? 1 : pick_rt(R, cc.hkv);
     const int wg_rows = 16 * (images ? kImageWaves : kBlockWaves) * rt;
@@ -1401,6 +1437,12 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     a.window = window > 0 ? window : softcap > 0.0f ? (1 << 30) : 0;
     a.softcap = softcap;
     a.scale = scale;
+    if (masked) {
+        a.mask = masked->mask;
+        a.mask_dtype = masked->mask_dtype;
+        a.mask_hs = masked->mask_head_stride;
+        a.mask_rs = masked->mask_row_stride;
+    }
     int rc;
     if constexpr (T4M != 2) {
         if (images) {
@@ -1434,6 +1476,8 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     const int q_tail = n_qt - q_main;
     auto launch = [&](BlockArgs& x, int n_qt_) {
         if constexpr (T4M != 2) {
+            if (masked)
+                return launch_block_rt<BITS, D, 1, T4M, false, 0, false, false, false, true>(cc, x, n_qt_, stream);
             if (images) return launch_one<BITS, D, T4M, 2>(cc, x, rt, n_qt_, stream);
         }
         if constexpr (T4M == 0) {
@@ -1482,7 +1526,7 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     if (n_split > 1 && T4M == 2)
         return launch_t4_merge_rotate(t.part_o, t.part_ml, n_split, t.PR, R, cc.hkv, D, G, Tq, 16,
                                       true, t4_tab, out, stream);
-    if (n_split > 1 && kPart16)
+    if (n_split > 1 && kPart16 && !masked)
         return launch_partial_merge_h((const f16*)t.part_o, t.part_ml, n_split, t.PR, t.prow0, t.PR,
                                       cc.hkv, D, G, Tq, out, stream, T4M ? 16 : BITS);
     if (n_split > 1)
@@ -1508,6 +1552,24 @@ int launch_block_attention_ext(KVCache& cc, const f16* q, int G, int n_rows, flo
     if (cc.bits == 4) return launch_block_bits<4, 128>(cc, q, G, n_rows, scale, causal, out, stream, nullptr, w, softcap);
     if (cc.bits == 8) return launch_block_bits<8, 128>(cc, q, G, n_rows, scale, causal, out, stream, nullptr, w, softcap);
     return launch_block_bits<16, 128>(cc, q, G, n_rows, scale, causal, out, stream, nullptr, w, softcap);
+}
+
+int launch_block_attention_masked(KVCache& cc, const f16* q, int G, int n_rows, float scale,
+                                  const SdpaOptions& o, const float* t4_tab, f16* out,
+                                  hipStream_t stream) {
+    QW_REQUIRE(o.mask && o.window <= 0 && o.softcap == 0.0f && (cc.D == 128 || cc.D == 256),
+               QW_ERR_INVALID_ARGUMENT, "block attention: masked launch outside its shapes");
+    auto run = [&](auto d) {
+        constexpr int D = decltype(d)::value;
+        if (cc.turbo4())
+            return launch_block_bits<4, D, 1>(cc, q, G, n_rows, scale, o.causal, out, stream, t4_tab, 0, 0.0f, &o);
+        if (cc.bits == 4)
+            return launch_block_bits<4, D>(cc, q, G, n_rows, scale, o.causal, out, stream, nullptr, 0, 0.0f, &o);
+        if (cc.bits == 8)
+            return launch_block_bits<8, D>(cc, q, G, n_rows, scale, o.causal, out, stream, nullptr, 0, 0.0f, &o);
+        return launch_block_bits<16, D>(cc, q, G, n_rows, scale, o.causal, out, stream, nullptr, 0, 0.0f, &o);
+    };
+    return cc.D == 256 ? run(std::integral_constant<int, 256>{}) : run(std::integral_constant<int, 128>{});
 }
 
 int launch_block_attention_t4(KVCache& cc, const f16* q, int G, int n_rows, float scale,

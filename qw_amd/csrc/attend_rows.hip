@@ -180,41 +180,7 @@ __global__ __launch_bounds__(64 * NW, 1) void rows_attend_kernel(RowsArgs a) {
             for (int u = 0; u < NU; u++) {
                 const int t = kt0 + 32 * u + 8 * g;
                 const int n = row_ok ? min(8, a.T - t) : 0;
-                raw[u][0] = raw[u][1] = u32x4{0, 0, 0, 0};
-                if (a.mask_dtype == QW_MASK_BOOL) {
-                    const uint8_t* p = (const uint8_t*)a.mask + moff + t;
-                    if (n == 8) {
-                        u32x2 w;
-                        __builtin_memcpy(&w, p, 8);
-                        raw[u][0].x = w.x;
-                        raw[u][0].y = w.y;
-                    } else {
-                        for (int e = 0; e < n; e++) {
-                            const uint32_t x = (uint32_t)p[e] << (8 * (e & 3));
-                            if (e < 4) raw[u][0].x |= x;
-                            else raw[u][0].y |= x;
-                        }
-                    }
-                } else if (a.mask_dtype == QW_DTYPE_F32) {
-                    const uint32_t* p = (const uint32_t*)a.mask + moff + t;
-                    if (n == 8) {
-                        __builtin_memcpy(&raw[u][0], p, 16);
-                        __builtin_memcpy(&raw[u][1], p + 4, 16);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 8; e++)
-                            if (e < n) raw[u][e >> 2][e & 3] = p[e];
-                    }
-                } else {
-                    const uint16_t* p = (const uint16_t*)a.mask + moff + t;
-                    if (n == 8) {
-                        __builtin_memcpy(&raw[u][0], p, 16);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 8; e++)
-                            if (e < n) raw[u][0][e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
-                    }
-                }
+                mask_load8(a.mask, a.mask_dtype, moff + t, n, raw[u]);
             }
         }
         // S^T: A row r16 of 16-key MFMA tile (u, tt) is key 32u + 8(r16>>2) + 4tt +
@@ -270,21 +236,13 @@ __global__ __launch_bounds__(64 * NW, 1) void rows_attend_kernel(RowsArgs a) {
                 for (int u = 0; u < NU; u++)
 #pragma unroll
                     for (int e = 0; e < 8; e++)
-                        if (((raw[u][0][e >> 2] >> (8 * (e & 3))) & 0xFFu) == 0) hide(u, e);
+                        if (mask_hides(raw[u], e)) hide(u, e);
             } else {
 #pragma unroll
                 for (int u = 0; u < NU; u++)
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
-                        // the additive term cast to fp16, as the reference casts float masks
-                        f16 ad;
-                        const uint32_t w = raw[u][0][e >> 1] >> (16 * (e & 1));
-                        if (a.mask_dtype == QW_DTYPE_F32)
-                            ad = (f16)__uint_as_float(raw[u][e >> 2][e & 3]);
-                        else if (a.mask_dtype == QW_DTYPE_BF16)
-                            ad = (f16)__uint_as_float(w << 16);
-                        else
-                            ad = __builtin_bit_cast(f16, (uint16_t)w);
+                        const f16 ad = mask_term(raw[u], a.mask_dtype, e);
                         if constexpr (CAP)
                             sf[u][e] += (float)ad;
                         else

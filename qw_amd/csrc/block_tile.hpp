@@ -64,4 +64,55 @@ __device__ __forceinline__ float wave_sum_g(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// An explicit mask in a key tile: a lane's 8 consecutive keys of one row, from
+// element offset off of a mask with key stride 1 (any alignment), n of them inside
+// the mask (n <= 0: none); raw, so that the loads can be issued ahead of the MFMAs.
+__device__ __forceinline__ void mask_load8(const void* mask, int dtype, int64_t off, int n,
+                                           u32x4 (&raw)[2]) {
+    raw[0] = raw[1] = u32x4{0, 0, 0, 0};
+    if (dtype == QW_MASK_BOOL) {
+        const uint8_t* p = (const uint8_t*)mask + off;
+        if (n >= 8) {
+            u32x2 w;
+            __builtin_memcpy(&w, p, 8);
+            raw[0].x = w.x;
+            raw[0].y = w.y;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (e < n) raw[0][e >> 2] |= (uint32_t)p[e] << (8 * (e & 3));
+        }
+    } else if (dtype == QW_DTYPE_F32) {
+        const uint32_t* p = (const uint32_t*)mask + off;
+        if (n >= 8) {
+            __builtin_memcpy(&raw[0], p, 16);
+            __builtin_memcpy(&raw[1], p + 4, 16);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (e < n) raw[e >> 2][e & 3] = p[e];
+        }
+    } else {
+        const uint16_t* p = (const uint16_t*)mask + off;
+        if (n >= 8) {
+            __builtin_memcpy(&raw[0], p, 16);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (e < n) raw[0][e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
+        }
+    }
+}
+// Key e of them: whether a bool mask hides it; an additive mask's term, cast to
+// fp16 as the reference casts float masks.
+__device__ __forceinline__ bool mask_hides(const u32x4 (&raw)[2], int e) {
+    return ((raw[0][e >> 2] >> (8 * (e & 3))) & 0xFFu) == 0;
+}
+__device__ __forceinline__ f16 mask_term(const u32x4 (&raw)[2], int dtype, int e) {
+    const uint32_t w = raw[0][e >> 1] >> (16 * (e & 1));
+    if (dtype == QW_DTYPE_F32) return (f16)__uint_as_float(raw[e >> 2][e & 3]);
+    if (dtype == QW_DTYPE_BF16) return (f16)__uint_as_float(w << 16);
+    return __builtin_bit_cast(f16, (uint16_t)w);
+}
+
 }  // namespace qw

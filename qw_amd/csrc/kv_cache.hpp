@@ -333,6 +333,13 @@ SdpaOptions shift_keys(const SdpaOptions& o, int lo);
 // q rotated in and the output rotated back) and sdpa_general.
 int cache_attention_general(KVCache& c, const void* q, int n_q_heads, int n_rows, float scale,
                             const SdpaOptions& o, void* out, hipStream_t stream);
+// Whether a masked call over a cache runs the block kernel on the codes, and that
+// launch (attend_block.hip; a Turbo4 cache: q unrotated, t4_tab its tables, out the
+// rows in the rotated basis).
+bool masked_block_route(const KVCache& c, const void* q, int G, int n_rows, const SdpaOptions& o);
+int launch_block_attention_masked(KVCache& c, const f16* q, int G, int n_rows, float scale,
+                                  const SdpaOptions& o, const float* t4_tab, f16* out,
+                                  hipStream_t stream);
 int turbo4_attention_general(KVCache& c, const void* q, int n_q_heads, int n_rows, float scale,
                              const SdpaOptions& opts, void* out, hipStream_t stream);
 

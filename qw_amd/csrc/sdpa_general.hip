@@ -25,6 +25,9 @@
 // A row with no visible key is zeros here (MLX: the mean of V for a bool mask,
 // NaN for an additive -inf mask).
 //
+// Calls of many rows go to attend_rows.hip and masked calls over a cache to the
+// block kernel (attend_block.hip); what is left runs here.
+//
 // Layout of the work: grid (key splits, row tiles, KV heads), 16 rows a wave,
 // 4 waves a workgroup (1 for calls of up to 16 rows a KV head). Rows of a KV head are (query row, head in group)
 // pairs, row index r * G + head, as in the other attention kernels. Each
@@ -320,7 +323,8 @@ int gen_kv_workspace(int device, hipStream_t stream, size_t need, void** out) {
 // (R - 100) T of 1.3M: at 384 rows a head 43.8 against 46.3 us over 4k keys
 // (here) and 130.8 -> 76.0 us over 16k (there), at 1536 rows 27.8 against 31.0
 // us over 300 keys and 52.7 -> 38.4 us over 1k. A mask is read a byte or two a
-// lane here and in 8-key pieces there: 78 rows over 8k keys 42 -> 27 us.
+// lane here and in 8-key pieces there, so a masked call's line lies lower: 78 rows
+// over 8k keys 49 -> 33 us with the layout and the merge.
 bool rows_route(int R, int n_keys, int hkv, int D, bool mask, const void* out) {
     if ((uintptr_t)out % 8 != 0) return false;  // (it writes 8-byte pieces)
     // images of more than 4 GiB are not kept (1.03 KB a key and head at D = 256)
@@ -440,6 +444,13 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
 #define QW_FUSED_WINDOW 1
 #endif
 
+// Query rows a KV head up to which a masked call over a cache runs the block kernel
+// on the codes (dequantizing them again for each 128-row tile): at 2160 rows, 24 heads
+// over 4, D = 256, 8-bit, 138 against 159 us over 8k keys and 475 against 561 us over 33k
+// for dequantizing once and the row kernel; 78 rows 75 -> 23 us over 8k, where the
+// general kernel took them.
+constexpr int kMaskedBlockRows = 4096;
+
 int window_first_key(const SdpaOptions& o, int T, int n_rows, int align) {
     if (o.window <= 0 || !o.causal) return 0;
     const int lo = std::max(0, T - n_rows - o.window + 1);
@@ -453,6 +464,12 @@ SdpaOptions shift_keys(const SdpaOptions& o, int lo) {
         s.mask = (const char*)o.mask + (int64_t)lo * es;  // key stride 1
     }
     return s;
+}
+
+bool masked_block_route(const KVCache& c, const void* q, int G, int n_rows, const SdpaOptions& o) {
+    return o.mask && o.window <= 0 && o.softcap == 0.0f && (uintptr_t)q % 16 == 0 &&
+           mask_kind_of(o.mask_dtype) >= 0 && o.mask_head_stride >= 0 && o.mask_row_stride >= 0 &&
+           G * n_rows <= kMaskedBlockRows;
 }
 
 int cache_attention_general(KVCache& c, const void* q, int n_q_heads, int n_rows, float scale,
@@ -476,6 +493,9 @@ int cache_attention_general(KVCache& c, const void* q, int n_q_heads, int n_rows
         (o.window <= 0 || o.causal) && std::isfinite(o.softcap) && (c.D == 128 || c.D == 256))
         return launch_block_attention_ext(c, (const f16*)q, n_q_heads / c.hkv, n_rows, scale,
                                           o.causal, o.window, o.softcap, (f16*)out, stream);
+    if (masked_block_route(c, q, n_q_heads / c.hkv, n_rows, o))
+        return launch_block_attention_masked(c, (const f16*)q, n_q_heads / c.hkv, n_rows, scale, o,
+                                             nullptr, (f16*)out, stream);
     const int T = c.offset, D = c.D;
     // A sliding window sees no key below lo (the first row's window start):
     // only keys lo .. T - 1 are dequantized, and the call runs on them with

@@ -819,7 +819,8 @@ static bool t4_fused_route(bool causal, int n_rows, int T, int G) {
 }
 
 static int turbo4_block(KVCache& c, const void* q, int n_q_heads, int n_rows, float scale,
-                        bool causal, bool fused, void* out, hipStream_t stream) {
+                        bool causal, bool fused, void* out, hipStream_t stream,
+                        const SdpaOptions* masked = nullptr) {
     const int D = c.D, G = n_q_heads / c.hkv;
     const float* tab = c.t4_tables;
     if (fused)
@@ -829,8 +830,10 @@ static int turbo4_block(KVCache& c, const void* q, int n_q_heads, int n_rows, fl
     void* wbuf = nullptr;
     if (int rc0 = t4_workspace(c.device, stream, (size_t)qrows * D * sizeof(f16), &wbuf)) return rc0;
     f16* o_r = (f16*)wbuf;
-    int rc = launch_block_attention_t4(c, (const f16*)q, G, n_rows, scale, causal, false, tab, o_r,
-                                       stream);
+    int rc = masked ? launch_block_attention_masked(c, (const f16*)q, G, n_rows, scale, *masked, tab,
+                                                    o_r, stream)
+                    : launch_block_attention_t4(c, (const f16*)q, G, n_rows, scale, causal, false, tab,
+                                                o_r, stream);
     if (rc) return rc;
     const dim3 rg((qrows + 3) / 4);
     if (D == 256) {
@@ -914,6 +917,8 @@ int turbo4_attention_general(KVCache& c, const void* q, int n_q_heads, int n_row
                              const SdpaOptions& opts, void* out, hipStream_t stream) {
     DeviceGuard dg(c.device);
     QW_REQUIRE(dg.ok, QW_ERR_HIP, "attention: hipSetDevice failed");
+    if (QW_T4_BLOCK && masked_block_route(c, q, n_q_heads / c.hkv, n_rows, opts))
+        return turbo4_block(c, q, n_q_heads, n_rows, scale, opts.causal, false, out, stream, &opts);
     return turbo4_expansion_route(c, q, n_q_heads, n_rows, scale, opts.causal, &opts, out, stream);
 }
 
