@@ -94,8 +94,7 @@ struct BlockArgs {
     // WIN launches (a causal sliding window): the row at position p sees keys
     // p - window + 1 .. p
     int window = 0;
-    // CAP launches (a logit softcap): s = tanh(f16(q . k) scale / softcap) softcap
-    float softcap = 0.0f, scale = 0.0f;
+    Softcap softcap = {};  // CAP launches: s = tanh(f16(q . k) scale / cap) cap
     // MASK launches: an explicit mask [hq or broadcast][Tq][T], key stride 1
     const void* mask = nullptr;
     int mask_dtype = 0;
@@ -800,13 +799,12 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
                 float sf[NU][8];
+                a.softcap.apply([&](auto f) {
 #pragma unroll
-                for (int u = 0; u < NU; u++)
+                    for (int u = 0; u < NU; u++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const float x = (float)(f16)acc[u][e >> 2][rt][e & 3];
-                        sf[u][e] = tanhf(x * a.scale / a.softcap) * a.softcap;
-                    }
+                        for (int e = 0; e < 8; e++) sf[u][e] = f((float)(f16)acc[u][e >> 2][rt][e & 3]);
+                });
                 if (mask) {
 #pragma unroll
                     for (int u = 0; u < NU; u++)
@@ -1435,8 +1433,7 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     a.pair_h = 0;
     // (a softcap launch without a window: one wider than any position)
     a.window = window > 0 ? window : softcap > 0.0f ? (1 << 30) : 0;
-    a.softcap = softcap;
-    a.scale = scale;
+    a.softcap = Softcap::of(scale, softcap);
     if (masked) {
         a.mask = masked->mask;
         a.mask_dtype = masked->mask_dtype;

@@ -53,7 +53,8 @@ struct RowsArgs {
     const void* mask;  // [hq or broadcast][Tq][T], key stride 1
     int mask_dtype;    // QW_MASK_BOOL / QW_DTYPE_*
     int64_t mhs, mrs;
-    float scale, scale_h, softcap;
+    float scale_h;
+    Softcap softcap;
 };
 
 // fp16 K/V rows with strides -> images of the tiles from tile0 on. grid (tiles,
@@ -216,16 +217,19 @@ __global__ __launch_bounds__(64 * NW, 1) void rows_attend_kernel(RowsArgs a) {
         // fp16 scores (softcap: fp32), masked
         half2v sh[CAP ? 1 : NU][4];
         float sf[CAP ? NU : 1][8];
+        if constexpr (CAP) {
+            a.softcap.apply([&](auto f) {
 #pragma unroll
-        for (int u = 0; u < NU; u++)
+                for (int u = 0; u < NU; u++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const f16 x = (f16)acc[u][e >> 2][e & 3];
-                if constexpr (CAP)
-                    sf[u][e] = tanhf((float)x * a.scale / a.softcap) * a.softcap;
-                else
-                    sh[u][e >> 1][e & 1] = x;
-            }
+                    for (int e = 0; e < 8; e++) sf[u][e] = f((float)(f16)acc[u][e >> 2][e & 3]);
+            });
+        } else {
+#pragma unroll
+            for (int u = 0; u < NU; u++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) sh[u][e >> 1][e & 1] = (f16)acc[u][e >> 2][e & 3];
+        }
         auto hide = [&](int u, int e) {
             if constexpr (CAP) sf[u][e] = -INFINITY;
             else sh[u][e >> 1][e & 1] = (f16)(-INFINITY);
@@ -483,9 +487,8 @@ int rows_attention_d(const void* q, int G, int n_rows, const void* k, const void
     a.mask_dtype = o.mask_dtype;
     a.mhs = o.mask_head_stride;
     a.mrs = o.mask_row_stride;
-    a.scale = scale;
     a.scale_h = (float)(f16)scale;
-    a.softcap = o.softcap;
+    a.softcap = Softcap::of(scale, o.softcap);
     if (int rc = ensure_dynamic_lds((const void*)rows_image_kernel<D>, S::BUF)) return rc;
     hipLaunchKernelGGL((rows_image_kernel<D>), dim3(n_tiles - tile0, hkv), dim3(512), S::BUF,
                        stream, (const f16*)k, (const f16*)v, khs, krs, vhs, vrs, n_keys, tile0, (char*)ws);

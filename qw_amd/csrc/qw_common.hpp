@@ -150,6 +150,31 @@ __device__ __forceinline__ float lane_xor(float x, int lane) {
     }
 }
 
+// The softcap of a score S (an fp16 value): tanh(S scale / cap) cap in fp32, as
+// cap - 2 cap / (e^(2 S scale / cap) + 1) by the hardware exponential and reciprocal
+// (five instructions for the library's forty and a division). Its error is absolute,
+// about 1.5e-7 cap, the rounding of a score near the cap; over kSoftcapDirect that
+// would show in scores far below the cap, and tanhf is taken.
+constexpr float kSoftcapDirect = 128.0f;
+struct Softcap {
+    float cap, k;  // k = scale / cap (tanhf), 2 log2(e) scale / cap (direct)
+    static Softcap of(float scale, float cap) {
+        const double r = cap > 0.0f ? (double)scale / cap : 0.0;
+        return {cap, (float)(cap <= kSoftcapDirect ? 2.0 * 1.4426950408889634 * r : r)};
+    }
+    // body(f) once, f the map of one score: one branch for all scores of a tile
+    template <class Body>
+    __device__ __forceinline__ void apply(Body body) const {
+        if (cap <= kSoftcapDirect)
+            body([&](float s) {
+                return __builtin_fmaf(-2.0f * cap,
+                                      __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * k) + 1.0f), cap);
+            });
+        else
+            body([&](float s) { return tanhf(s * k) * cap; });
+    }
+};
+
 template <class Op>
 __device__ __forceinline__ float wave_reduce(float x, Op op) {
     x = op(x, dpp_mov<0xB1>(x));   // quad_perm [1,0,3,2]

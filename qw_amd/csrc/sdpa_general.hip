@@ -62,7 +62,8 @@ struct GenArgs {
     float* part_o;               // [hkv][n_split][R][D]
     float2* part_ml;             // [hkv][n_split][R]
     int G, L, T, R, causal, window, n_split, keys_per_split;
-    float scale, scale_h, softcap;
+    float scale_h;
+    Softcap softcap;
 };
 
 constexpr int kMaskBool = 0, kMaskF16 = 1, kMaskBf16 = 2, kMaskF32 = 3;
@@ -192,13 +193,21 @@ __global__ __launch_bounds__(64 * NWV) void sdpa_general_kernel(GenArgs a) {
         }
         float sv[NU][4];
         float tmax = -INFINITY;
+        float capped[SOFTCAP ? NU : 1][4];
+        if constexpr (SOFTCAP)
+            a.softcap.apply([&](auto f) {
+#pragma unroll
+                for (int u = 0; u < NU; u++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) capped[u][i] = f((float)(f16)s4[u][i]);
+            });
 #pragma unroll
         for (int u = 0; u < NU; u++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int t = t0 + 16 * u + 4 * g + i;
                 float s = (float)(f16)s4[u][i];
-                if constexpr (SOFTCAP) s = tanhf(s * a.scale / a.softcap) * a.softcap;
+                if constexpr (SOFTCAP) s = capped[u][i];
                 bool vis = row_ok && t >= lo && t < hi && t < k_end;
                 if (vis && a.mask) {
                     float add = 0.0f;
@@ -279,7 +288,7 @@ __global__ __launch_bounds__(64 * NWV) void sdpa_general_kernel(GenArgs a) {
 
 template <int D, int NWV>
 void launch_general(const GenArgs& a, dim3 grid, hipStream_t stream) {
-    if (a.softcap > 0.0f)
+    if (a.softcap.cap > 0.0f)
         hipLaunchKernelGGL((sdpa_general_kernel<D, true, NWV>), grid, dim3(64 * NWV), 0, stream, a);
     else
         hipLaunchKernelGGL((sdpa_general_kernel<D, false, NWV>), grid, dim3(64 * NWV), 0, stream,
@@ -398,9 +407,8 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
     a.R = R;
     a.causal = o.causal ? 1 : 0;
     a.window = o.window > 0 ? o.window : 0;
-    a.scale = scale;
     a.scale_h = (float)(f16)scale;
-    a.softcap = o.softcap;
+    a.softcap = Softcap::of(scale, o.softcap);
     // Up to 16 rows a KV head: one-wave workgroups (about 1024 of them);
     // else four-wave ones (about 256). Key splits of whole tiles, at least
     // four tiles each, at most 256 (the merge's limit).

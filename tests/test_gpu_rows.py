@@ -38,6 +38,8 @@ CASES = [
     (16, 2, 64, 256, 1281, True, 0, 0.0),      # 256-key tiles in two halves
     (16, 2, 64, 300, 1500, True, 33, 20.0),    # a window below a tile, capped
     (24, 4, 128, 220, 1400, False, 0, 30.0),   # capped, not causal
+    (24, 4, 128, 220, 1400, True, 0, 128.0),   # the largest cap of the direct form
+    (24, 4, 128, 220, 1400, True, 0, 300.0),   # one past it
     (12, 1, 256, 190, 1000, True, 0, 0.0),     # one KV head, G = 12
     (24, 4, 256, 1100, 1100, True, 0, 0.0),    # prefill into nothing: rows from one key on
 ]
