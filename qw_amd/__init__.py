@@ -123,31 +123,66 @@ def _check(rc: int) -> None:
         raise QwError(rc, lib().qw_last_error().decode())
 
 
-def _torch():
-    import torch  # imported lazily: the ABI itself needs no torch
+_torch_module = None
 
-    return torch
+
+def _torch():
+    global _torch_module
+    if _torch_module is None:
+        import torch  # imported lazily: the ABI itself needs no torch
+
+        _torch_module = torch
+    return _torch_module
+
+
+_raw_stream = None  # torch's current stream of a device index, as its handle
 
 
 def _stream(device) -> int:
-    torch = _torch()
-    return torch.cuda.current_stream(device).cuda_stream
+    # The stream object costs 2 us a call to build; a decode step is 12.
+    global _raw_stream
+    if _raw_stream is None:
+        torch = _torch()
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda index: torch.cuda.current_stream(index).cuda_stream)
+    index = device.index
+    return _raw_stream(_torch().cuda.current_device() if index is None else index)
 
 
-def _as3(t, name: str):
-    """Reference tensors are [1, H, L, D]; accept [H, L, D] as well."""
-    if t.dim() == 4:
-        if t.shape[0] != 1:
+def _hld(t, name: str):
+    """A reference tensor [1, H, L, D] or [H, L, D]: (the tensor, contiguous, with the dims it
+    has; H, L, D). No view is made: the rows lie the same with and without the batch of 1."""
+    shape = t.shape
+    if len(shape) == 4:
+        if shape[0] != 1:
             raise QwError(1, f"{name}: batch must be 1")
-        t = t[0]
-    if t.dim() != 3:
+        _, H, L, D = shape
+    elif len(shape) == 3:
+        H, L, D = shape
+    else:
         raise QwError(1, f"{name}: expected [1, H, L, D] or [H, L, D]")
-    torch = _torch()
-    if t.dtype != torch.float16:
+    if t.dtype is not _torch().float16:
         raise QwError(2, f"{name}: fp16 expected, got {t.dtype}")
     if not t.is_cuda:
         raise QwError(1, f"{name}: must be a device tensor")
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous(), H, L, D
+
+
+def _rows2(qkv, what: str):
+    """A projection [1, L, W] or [L, W], or the first batch of [B, L, W]: (contiguous, L, W)."""
+    shape = qkv.shape
+    if len(shape) == 3:
+        x = qkv if shape[0] == 1 else qkv[0]
+    else:
+        x = qkv
+    if len(shape) not in (2, 3) or x.dtype is not _torch().float16 or not x.is_cuda:
+        raise QwError(1, f"{what}: qkv must be a [1, L, W] or [L, W] fp16 device tensor")
+    return x if x.is_contiguous() else x.contiguous(), shape[-2], shape[-1]
+
+
+def _out_like(t, H: int, L: int, D: int):
+    """An output [1, H, L, D] of t's type on t's device."""
+    return t.new_empty((1, H, L, D))
 
 
 class KVCacheMode:
@@ -229,11 +264,11 @@ class KVCache:
 
     # -- append / fetch
     def update(self, keys, values) -> None:
-        k, v = _as3(keys, "keys"), _as3(values, "values")
-        if k.shape != v.shape or k.shape[0] != self.n_kv_heads or k.shape[2] != self.head_dim:
+        k, H, L, D = _hld(keys, "keys")
+        v, *vs = _hld(values, "values")
+        if vs != [H, L, D] or H != self.n_kv_heads or D != self.head_dim:
             raise QwError(1, "update: keys/values must be [n_kv_heads, L, head_dim]")
-        _check(lib().qw_kv_update(self._h, k.data_ptr(), v.data_ptr(), k.shape[1],
-                                  _stream(self.device)))
+        _check(lib().qw_kv_update(self._h, k.data_ptr(), v.data_ptr(), L, _stream(self.device)))
 
     def rope_update(self, qkv, n_q_heads: int, rope_dims: int, rope_base: float,
                     rope_scale: float = 1.0, traditional: bool = False,
@@ -243,20 +278,15 @@ class KVCache:
         then ``KVCache::update``): ``qkv`` is [1, L, (Hq + 2 Hkv) D] or
         [L, (Hq + 2 Hkv) D] fp16; token t rotates at position0 + t (default:
         the cache offset). Returns the rotated q as [1, Hq, L, D]."""
-        torch = _torch()
-        x = qkv[0] if qkv.dim() == 3 else qkv
-        if x.dim() != 2 or x.dtype != torch.float16 or not x.is_cuda:
-            raise QwError(1, "rope_update: qkv must be a [1, L, W] or [L, W] fp16 device tensor")
-        x = x.contiguous()
-        L, W = x.shape
+        x, L, W = _rows2(qkv, "rope_update")
         if W != (n_q_heads + 2 * self.n_kv_heads) * self.head_dim:
             raise QwError(1, "rope_update: qkv width does not match the head geometry")
         pos = self.offset if position0 is None else position0
-        q = torch.empty((n_q_heads, L, self.head_dim), dtype=torch.float16, device=self.device)
+        q = _out_like(x, n_q_heads, L, self.head_dim)
         _check(lib().qw_kv_rope_update(self._h, x.data_ptr(), n_q_heads, L, rope_dims,
                                        int(traditional), float(rope_base), float(rope_scale),
                                        pos, q.data_ptr(), _stream(self.device)))
-        return q.unsqueeze(0)
+        return q
 
     def rope_update_and_attention(self, qkv, n_q_heads: int, rope_dims: int, rope_base: float,
                                   scale: float, rope_scale: float = 1.0, traditional: bool = False,
@@ -265,33 +295,26 @@ class KVCache:
         attention of the rotated q over the cache; one decode launch for
         decode-route shapes). Returns (out [1, Hq, L, D], rotated q [1, Hq,
         L, D])."""
-        torch = _torch()
-        x = qkv[0] if qkv.dim() == 3 else qkv
-        if x.dim() != 2 or x.dtype != torch.float16 or not x.is_cuda:
-            raise QwError(1, "rope_update_and_attention: qkv must be a [1, L, W] or [L, W] fp16 "
-                             "device tensor")
-        x = x.contiguous()
-        L, W = x.shape
+        x, L, W = _rows2(qkv, "rope_update_and_attention")
         if W != (n_q_heads + 2 * self.n_kv_heads) * self.head_dim:
             raise QwError(1, "rope_update_and_attention: qkv width does not match the head geometry")
         pos = self.offset if position0 is None else position0
-        q = torch.empty((n_q_heads, L, self.head_dim), dtype=torch.float16, device=self.device)
-        out = torch.empty_like(q)
+        q, out = (_out_like(x, n_q_heads, L, self.head_dim) for _ in range(2))
         _check(lib().qw_kv_rope_update_and_attention(
             self._h, x.data_ptr(), n_q_heads, L, rope_dims, int(traditional), float(rope_base),
             float(rope_scale), pos, float(scale), int(causal), q.data_ptr(), out.data_ptr(),
             _stream(self.device)))
-        return out.unsqueeze(0), q.unsqueeze(0)
+        return out, q
 
     def dequantize(self, start: int = 0, n: int | None = None):
         torch = _torch()
         n = self.offset - start if n is None else n
-        k = torch.empty((self.n_kv_heads, n, self.head_dim), dtype=torch.float16,
+        k = torch.empty((1, self.n_kv_heads, n, self.head_dim), dtype=torch.float16,
                         device=self.device)
         v = torch.empty_like(k)
         _check(lib().qw_kv_dequantize(self._h, start, n, k.data_ptr(), v.data_ptr(),
                                       _stream(self.device)))
-        return k.unsqueeze(0), v.unsqueeze(0)
+        return k, v
 
     def update_and_fetch(self, keys, values):
         self.update(keys, values)
@@ -299,22 +322,21 @@ class KVCache:
 
     # -- attention
     def _attn(self, q, keys, values, scale: float, causal: bool):
-        torch = _torch()
-        qq = _as3(q, "q")
-        hq, L, D = qq.shape
-        out = torch.empty_like(qq)
+        qq, hq, L, D = _hld(q, "q")
+        out = _out_like(qq, hq, L, D)
         st = _stream(self.device)
         if keys is None:
             _check(lib().qw_kv_attention(self._h, qq.data_ptr(), hq, L, float(scale),
                                          int(causal), out.data_ptr(), st))
         else:
-            k, v = _as3(keys, "keys"), _as3(values, "values")
-            if k.shape != v.shape or k.shape[1] != L:
+            k, *ks = _hld(keys, "keys")
+            v, *vs = _hld(values, "values")
+            if ks != vs or ks[1] != L:
                 raise QwError(1, "attention: new keys/values must have q's row count")
             _check(lib().qw_kv_update_and_attention(self._h, qq.data_ptr(), hq, L, k.data_ptr(),
                                                     v.data_ptr(), float(scale), int(causal),
                                                     out.data_ptr(), st))
-        return out.unsqueeze(0)
+        return out
 
     def update_and_attention(self, q, keys, values, scale: float, mask=None):
         """Append, then attend (reference ``update_and_turbo4_attention(q, k, v,
@@ -344,10 +366,8 @@ class KVCache:
         return self._general(q, keys, values, scale, causal, window, softcap, mask)
 
     def _general(self, q, keys, values, scale, causal, window, softcap, mask):
-        torch = _torch()
-        qq = _as3(q, "q")
-        hq, L, D = qq.shape
-        out = torch.empty_like(qq)
+        qq, hq, L, D = _hld(q, "q")
+        out = _out_like(qq, hq, L, D)
         T = self.offset + (0 if keys is None else L)
         m, md, mhs, mrs, _keep = _mask_args(mask, hq, L, T)
         st = _stream(self.device)
@@ -356,37 +376,38 @@ class KVCache:
                                                  int(causal), int(window), float(softcap), m, md,
                                                  mhs, mrs, out.data_ptr(), st))
         else:
-            k, v = _as3(keys, "keys"), _as3(values, "values")
-            if k.shape != v.shape or k.shape[1] != L:
+            k, *ks = _hld(keys, "keys")
+            v, *vs = _hld(values, "values")
+            if ks != vs or ks[1] != L:
                 raise QwError(1, "attention: new keys/values must have q's row count")
             _check(lib().qw_kv_update_and_attention_general(
                 self._h, qq.data_ptr(), hq, L, k.data_ptr(), v.data_ptr(), float(scale),
                 int(causal), int(window), float(softcap), m, md, mhs, mrs, out.data_ptr(), st))
-        return out.unsqueeze(0)
+        return out
 
     # -- D-LSA read over the cache (qwen3_next/dlsa.rs:161-177)
     def _dlsa(self, q, keys, values, lists, lengths, scale: float):
         torch = _torch()
-        qq = _as3(q, "q")
-        hq, L, D = qq.shape
+        qq, hq, L, D = _hld(q, "q")
         if lists.dim() != 2 or lists.dtype != torch.int32 or lengths.dim() != 1 or \
                 lengths.dtype != torch.int32 or lists.shape[0] != L or lengths.shape[0] != L:
             raise QwError(1, "dlsa_attention: lists [L,W] i32 and lengths [L] i32 expected")
         lists, lengths = lists.contiguous(), lengths.contiguous()
-        out = torch.empty_like(qq)
+        out = _out_like(qq, hq, L, D)
         st = _stream(self.device)
         if keys is None:
             _check(lib().qw_kv_dlsa_attention(self._h, qq.data_ptr(), hq, L, lists.data_ptr(),
                                               lengths.data_ptr(), lists.shape[1], float(scale),
                                               out.data_ptr(), st))
         else:
-            k, v = _as3(keys, "keys"), _as3(values, "values")
-            if k.shape != v.shape or k.shape[1] != L:
+            k, *ks = _hld(keys, "keys")
+            v, *vs = _hld(values, "values")
+            if ks != vs or ks[1] != L:
                 raise QwError(1, "dlsa_attention: new keys/values must have q's row count")
             _check(lib().qw_kv_update_and_dlsa_attention(
                 self._h, qq.data_ptr(), hq, L, k.data_ptr(), v.data_ptr(), lists.data_ptr(),
                 lengths.data_ptr(), lists.shape[1], float(scale), out.data_ptr(), st))
-        return out.unsqueeze(0)
+        return out
 
     def dlsa_attention(self, q, lists, lengths, scale: float):
         """D-LSA K2 over the cached rows in place: the reference's
@@ -509,24 +530,22 @@ def sparse_attention_with(q, k, v, lists, lengths, scale: float, parts: int = 0,
                           waves: int = 0):
     """D-LSA gathered read with launch knobs (dlsa_attention.rs:44)."""
     torch = _torch()
-    qq = _as3(q, "q")
+    qq, hq, L, D = _hld(q, "q")
     kk, vv = _kv_view(k, "k"), _kv_view(v, "v")
-    if kk.shape != vv.shape or kk.shape[2] != qq.shape[2]:
+    if kk.shape != vv.shape or kk.shape[2] != D:
         raise QwError(1, "sparse_attention: k/v shapes disagree with q")
     if lists.dim() != 2 or lists.dtype != torch.int32 or lengths.dim() != 1 or \
-            lengths.dtype != torch.int32 or lists.shape[0] != qq.shape[1] or \
-            lengths.shape[0] != qq.shape[1]:
+            lengths.dtype != torch.int32 or lists.shape[0] != L or lengths.shape[0] != L:
         raise QwError(1, "sparse_attention: lists [L,W] i32 and lengths [L] i32 expected")
     lists = lists.contiguous()
     lengths = lengths.contiguous()
-    out = torch.empty_like(qq)
-    hq, L, D = qq.shape
+    out = _out_like(qq, hq, L, D)
     hkv, T, _ = kk.shape
     _check(lib().qw_dlsa_sparse_attention_with(
         qq.data_ptr(), kk.data_ptr(), vv.data_ptr(), kk.stride(0), kk.stride(1), vv.stride(0),
         vv.stride(1), lists.data_ptr(), lengths.data_ptr(), L, lists.shape[1], hq, hkv, D, T,
         float(scale), parts, waves, out.data_ptr(), _stream(qq.device)))
-    return out.unsqueeze(0)
+    return out
 
 
 QW_MASK_BOOL = 3
@@ -538,26 +557,31 @@ def _mask_args(mask, hq: int, L: int, T: int):
     additive f16 / bf16 / f32 mask."""
     if mask is None:
         return None, 0, 0, 0, None
-    torch = _torch()
-    m = mask
-    while m.dim() > 3:
-        if m.shape[0] != 1:
-            raise QwError(1, "mask: batch must be 1")
-        m = m[0]
-    if m.dim() == 2:
-        m = m.unsqueeze(0)
-    if m.dim() != 3 or m.shape[0] not in (1, hq) or m.shape[1] != L or m.shape[2] != T:
+    shape = mask.shape
+    n = len(shape)
+    if n > 3 and any(x != 1 for x in shape[:-3]):
+        raise QwError(1, "mask: batch must be 1")
+    if n < 2 or (n > 2 and shape[-3] not in (1, hq)) or shape[-2] != L or shape[-1] != T:
         raise QwError(1, f"mask: shape {tuple(mask.shape)} does not broadcast to [1, {hq}, {L}, {T}]")
-    if not m.is_cuda:
+    if not mask.is_cuda:
         raise QwError(1, "mask: device tensor expected")
-    codes = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2, torch.bool: QW_MASK_BOOL,
-             torch.uint8: QW_MASK_BOOL}
-    if m.dtype not in codes:
-        raise QwError(1, f"mask: bool or f16/bf16/f32 expected, got {m.dtype}")
-    if m.stride(2) != 1:
-        m = m.contiguous()
-    hs = 0 if m.shape[0] == 1 else m.stride(0)
-    return m.data_ptr(), codes[m.dtype], hs, m.stride(1), m
+    code = _mask_codes().get(mask.dtype)
+    if code is None:
+        raise QwError(1, f"mask: bool or f16/bf16/f32 expected, got {mask.dtype}")
+    m = mask if mask.stride(-1) == 1 else mask.contiguous()
+    hs = 0 if n == 2 or shape[-3] == 1 else m.stride(-3)
+    return m.data_ptr(), code, hs, m.stride(-2), m
+
+
+_MASK_CODES = {}
+
+
+def _mask_codes() -> dict:
+    if not _MASK_CODES:
+        torch = _torch()
+        _MASK_CODES.update({torch.float16: 0, torch.bfloat16: 1, torch.float32: 2,
+                            torch.bool: QW_MASK_BOOL, torch.uint8: QW_MASK_BOOL})
+    return _MASK_CODES
 
 
 def attention(q, k, v, scale: float, mask=None, softcap: float = 0.0, window: int = 0,
@@ -565,20 +589,18 @@ def attention(q, k, v, scale: float, mask=None, softcap: float = 0.0, window: in
     """``layers::attention(q, k, v, scale, mask, softcap, window)`` (layers.rs:4010)
     over fp16 K/V [1, Hkv, T, D] (any head/row strides); ``causal`` and
     ``window`` give ``causal_attention``'s masks (lib.rs:3185)."""
-    torch = _torch()
-    qq = _as3(q, "q")
+    qq, hq, L, D = _hld(q, "q")
     kk, vv = _kv_view(k, "k"), _kv_view(v, "v")
-    if kk.shape != vv.shape or kk.shape[2] != qq.shape[2]:
+    if kk.shape != vv.shape or kk.shape[2] != D:
         raise QwError(1, "attention: k/v shapes disagree with q")
-    hq, L, D = qq.shape
     hkv, T, _ = kk.shape
     m, md, mhs, mrs, _keep = _mask_args(mask, hq, L, T)
-    out = torch.empty_like(qq)
+    out = _out_like(qq, hq, L, D)
     _check(lib().qw_sdpa(qq.data_ptr(), hq, L, kk.data_ptr(), vv.data_ptr(), hkv, T, D,
                          kk.stride(0), kk.stride(1), vv.stride(0), vv.stride(1), float(scale),
                          int(causal), int(window), float(softcap), m, md, mhs, mrs,
                          out.data_ptr(), _stream(qq.device)))
-    return out.unsqueeze(0)
+    return out
 
 
 def causal_attention(q, k, v, scale: float, softcap: float = 0.0, window: int = 0):
@@ -678,10 +700,9 @@ def dlsa_select_with(scores, members, positions, total_rows: int, params: DlsaSe
     sc, mb, pos = scores.contiguous(), members.contiguous(), positions.contiguous()
     R = sc.shape[0]
     dev = sc.device
-    lists = torch.empty((R, params.list_width()), dtype=torch.int32, device=dev)
-    lengths = torch.empty((R,), dtype=torch.int32, device=dev)
-    picked = torch.empty((R, params.top_p), dtype=torch.int32, device=dev)
-    status = torch.empty((R,), dtype=torch.int32, device=dev)
+    lists = mb.new_empty((R, params.list_width()))
+    lengths, status = mb.new_empty((R,)), mb.new_empty((R,))
+    picked = mb.new_empty((R, params.top_p))
     _check(lib().qw_dlsa_select(sc.data_ptr(), sc.shape[1], mb.data_ptr(), mb.shape[0],
                                 params.bucket_cap, pos.data_ptr(), R, total_rows, params.window,
                                 params.sink, params.top_k, params.top_p,
