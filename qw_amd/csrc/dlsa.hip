@@ -588,10 +588,14 @@ __device__ __forceinline__ void dlsa_body(const DlsaArgs& a, const Src& src) {
 // One kernel per (head dim, heads per group, row source). Affine sources use
 // the exact 2-op dequant when every cached scale allows it (the cache's
 // fast_flag), else the separately rounded one.
-template <int D, int GMAX, class Src, int RP = 1>
+// FLAGGED: only the groups that dlsa_rows.hip left (an instance of its own: the test
+// cost the cache reads, which never take it, 0.4 of 22 us).
+template <int D, int GMAX, class Src, int RP = 1, bool FLAGGED = false>
 __global__ __launch_bounds__(256, 2) void dlsa_kernel(DlsaArgs a, Src src, const int* fast_flag) {
-    // (two-row workgroups never straddle groups: both counts are even)
-    if (a.flags && !a.flags[(int)(blockIdx.y * RP) / a.group_rows * a.hkv + blockIdx.z]) return;
+    if constexpr (FLAGGED) {
+        // (two-row workgroups never straddle groups: both counts are even)
+        if (!a.flags[(int)(blockIdx.y * RP) / a.group_rows * a.hkv + blockIdx.z]) return;
+    }
     if constexpr (Src::kAffine) {
         // The exact 2-op dequant runs without waiting for the cache's fast
         // flag; a cache holding a scale outside its exact range takes the
@@ -723,14 +727,20 @@ static void launch_dlsa_kernel(const Src& src, const DlsaArgs& a, dim3 grid, con
                                hipStream_t stream) {
     // one-pass calls with rows to spare: two rows a workgroup (the grid keeps
     // at least kPairMinWorkgroups workgroups)
+    auto launch = [&](auto kernel, dim3 g) {
+        hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, a, src, fast);
+    };
+    constexpr bool kStrided = std::is_same_v<Src, SrcStrided<D>>;
     if constexpr (Src::kPairs) {
         if (a.parts == 1 && 2 * a.G <= 16 && (int64_t)a.L * a.hkv >= 2 * kPairMinWorkgroups) {
-            hipLaunchKernelGGL((dlsa_kernel<D, GM, Src, 2>), dim3(grid.x, (a.L + 1) / 2, grid.z),
-                               dim3(256), 0, stream, a, src, fast);
+            const dim3 g(grid.x, (a.L + 1) / 2, grid.z);
+            if (kStrided && a.flags) launch(dlsa_kernel<D, GM, Src, 2, kStrided>, g);
+            else launch(dlsa_kernel<D, GM, Src, 2>, g);
             return;
         }
     }
-    hipLaunchKernelGGL((dlsa_kernel<D, GM, Src>), grid, dim3(256), 0, stream, a, src, fast);
+    if (kStrided && a.flags) launch(dlsa_kernel<D, GM, Src, 1, kStrided>, grid);
+    else launch(dlsa_kernel<D, GM, Src>, grid);
 }
 
 template <int D, int GM>
