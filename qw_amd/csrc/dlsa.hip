@@ -840,8 +840,8 @@ static int dlsa_sparse_attention_impl(const void* q, const DlsaSource& src,
     if (auto_one_pass && !src.cache && dlsa_rows_pays(n_rows, width, n_kv_heads)) {
         // prefill row counts: neighbouring rows share their keys' gathers; the
         // kernel below then serves the groups that this one leaves
-        const int rc = dlsa_rows_attention(q, src.k, src.v, false, src.khs, src.krs, src.vhs, src.vrs,
-                                           lists, lengths, n_rows, width, n_q_heads, n_kv_heads,
+        const int rc = dlsa_rows_attention(q, QW_DTYPE_F16, src.k, src.v, QW_DTYPE_F16, src.khs,
+                                           src.krs, src.vhs, src.vrs, lists, lengths, n_rows, width, n_q_heads, n_kv_heads,
                                            head_dim, n_keys, scale, out, &a.flags, stream);
         if (rc == QW_OK)
             a.group_rows = dlsa_rows_per_group(G);

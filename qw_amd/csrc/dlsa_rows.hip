@@ -4,8 +4,8 @@
 // Contract: dlsa.hip's (the reference's dlsa_attention::sparse_attention,
 // crates/mlxcel-core/src/dlsa_attention.rs:31-63): row r attends over the keys
 // of its own list, entries outside [0, T) skipped, fp32 scores, softmax and sums,
-// a row without a valid entry zeros. fp16 or bf16 q, K and V (alike), output in
-// that type.
+// a row without a valid entry zeros. fp16 or bf16 q, K and V (alike) in those
+// types; other pairs of types, and D = 32, in fp32 (dlsa_rows32_kernel).
 //
 // The rows of a prefill chunk list nearly the same keys (the sinks, the chunk's
 // long-range blocks, windows that slide by one), but one row fills 6 of an MFMA
@@ -25,7 +25,7 @@
 // MFMAs a (key, column, dim) where that kernel has two. Measured (24 heads over 4,
 // D = 256, lists of 4 sinks, a 512-key window and 8 shared 512-key blocks): 1536 rows
 // at 32k in fp16 1312 us by row pairs -> 347 us here (502 TFLOP/s; the plan 26 us, the
-// merge 6 us of it), 512 rows at 16k in bf16 7572 -> 157 us.
+// merge 6 us of it), 512 rows at 16k in bf16 7572 -> 157 us; in f32 7530 -> 744 us.
 //
 // A group is left to the row-by-row kernels, launched behind with the flags of
 // this one, where (a) a row lists a key twice (it counts twice), (b) the union is
@@ -189,6 +189,7 @@ struct DlsaRowsArgs {
     int L, G, hkv, NR, cap, groups;
     int n_main, qt0, n_split, prow0, PR;  // as RowsArgs (attend_rows.hip)
     float scale2;           // scale * log2(e)
+    int q_dtype;            // q's and out's type (the fp32 kernel)
 };
 
 template <bool BF>
@@ -209,6 +210,12 @@ struct Elem<true> {
     }
     typedef __bf16 T;
 };
+
+__device__ __forceinline__ void store_as(void* out, int dtype, int64_t at, float y) {
+    if (dtype == QW_DTYPE_F32) ((float*)out)[at] = y;
+    else if (dtype == QW_DTYPE_F16) ((f16*)out)[at] = (f16)y;
+    else ((__bf16*)out)[at] = (__bf16)y;
+}
 
 template <int D, bool BF>
 __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
@@ -543,6 +550,264 @@ __global__ __launch_bounds__(256) void dlsa_rows_merge_kernel(DlsaRowsArgs a) {
     if (bad) a.flags[fl] = 1;
 }
 
+// The same in fp32 throughout, for every other pair of types (and D = 32): K and V
+// rows widened to fp32 as they are staged, both products on
+// v_mfma_f32_16x16x4_f32. Bound by those MFMAs (a sixteenth of the 16-bit rate).
+// Layouts: tiles of 8192 / D keys; the four MFMAs of a 16-dim chunk take element
+// 0 .. 3 of each lane's 16-byte piece (lane (g, r16): dims 16m + 4g .. +3), so K is
+// read 16 bytes a lane, chunk c of key k at c ^ (k mod 16) against bank conflicts; P
+// leaves the score tile as the A operand (keys 4g + i, MFMA i), and V is read VD dims
+// a lane of one key, one operand for each of VD output tiles.
+template <int D, int DKV>
+__global__ __launch_bounds__(512, 1) void dlsa_rows32_kernel(DlsaRowsArgs a) {
+    constexpr int KT = 8192 / D, CPR = D / 4;  // keys a tile, 16-byte chunks a row
+    constexpr int NM = D / 16, SW = CPR < 16 ? CPR - 1 : 15;
+    constexpr int VD = D < 64 ? 2 : 4, NP = D / (16 * VD);
+    constexpr int KBUF = KT * D * 4;  // bytes of a K (V) tile: 32 KB
+    constexpr int WPT = DKV == QW_DTYPE_F32 ? 4 : 2;  // 16-byte pieces of 16 values
+    typedef float vecv __attribute__((ext_vector_type(VD)));
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    uint32_t* const sW = (uint32_t*)(lds + 4 * KBUF);  // [2][KT] row words
+    int sp = 0, qt, h, n_split = 1;
+    {
+        const int lin = blockIdx.x;
+        if (lin < a.n_main) {
+            qt = lin / a.hkv;
+            h = lin % a.hkv;
+        } else {
+            const int t = lin - a.n_main;
+            n_split = a.n_split;
+            sp = t % n_split;
+            h = (t / n_split) % a.hkv;
+            qt = a.qt0 + t / (n_split * a.hkv);
+        }
+    }
+    if (a.flags[qt * a.hkv + h]) return;  // (uniform, before any barrier)
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int n_tiles = (a.counts[qt] + KT - 1) / KT, tps = (n_tiles + n_split - 1) / n_split;
+    const int t0 = sp * tps, t1 = min(n_tiles, t0 + tps);
+    const int R = a.L * a.G, row0 = qt * a.NR * a.G, row_end = min(R, row0 + a.NR * a.G);
+    const int wrow0 = row0 + 16 * wave, rho = wrow0 + r16;
+    const bool wave_live = wrow0 < row_end, row_ok = rho < row_end;
+    const int r = row_ok ? rho / a.G : 0, qh = h * a.G + (row_ok ? rho - r * a.G : 0);
+    const int bit = row_ok ? r - qt * a.NR : 0;
+    float4v qb[NM];
+    {
+        const int64_t q0 = ((int64_t)qh * a.L + r) * D;
+#pragma unroll
+        for (int m = 0; m < NM; m++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int64_t at = q0 + 16 * m + 4 * g + e;
+                qb[m][e] = a.q_dtype == QW_DTYPE_F32   ? ((const float*)a.q)[at]
+                           : a.q_dtype == QW_DTYPE_F16 ? (float)((const f16*)a.q)[at]
+                                                       : (float)((const __bf16*)a.q)[at];
+            }
+    }
+    // a thread stages 16 dims of one key, of K and of V
+    const int kk = tid / (D / 16), sl = tid % (D / 16);
+    constexpr int ES = DKV == QW_DTYPE_F32 ? 4 : 2;
+    const char* const kh = (const char*)a.k + ES * (h * a.khs + 16 * sl);
+    const char* const vh = (const char*)a.v + ES * (h * a.vhs + 16 * sl);
+    const int32_t* const gk = a.keys + (int64_t)qt * a.cap;
+    const uint32_t* const gw = a.words + (int64_t)qt * a.cap;
+    int ki;
+    u32x4 kc[WPT], vc[WPT];
+    uint32_t word;
+    auto load = [&](int t) {
+        const u32x4* ks = (const u32x4*)(kh + ES * ki * a.krs);
+        const u32x4* vs = (const u32x4*)(vh + ES * ki * a.vrs);
+#pragma unroll
+        for (int w = 0; w < WPT; w++) {
+            kc[w] = ks[w];
+            vc[w] = vs[w];
+        }
+        if (tid < KT) word = gw[t * KT + tid];
+    };
+    auto wide = [&](const u32x4* c, int w) {  // values 4w .. 4w + 3
+        if constexpr (DKV == QW_DTYPE_F32) {
+            return __builtin_bit_cast(float4v, c[w]);
+        } else {
+            const uint32_t x = c[w / 2][2 * (w & 1)], y = c[w / 2][2 * (w & 1) + 1];
+            if constexpr (DKV == QW_DTYPE_F16)
+                return float4v{(float)h2(x).x, (float)h2(x).y, (float)h2(y).x, (float)h2(y).y};
+            else
+                return float4v{__uint_as_float(x << 16), __uint_as_float(x & 0xFFFF0000u),
+                               __uint_as_float(y << 16), __uint_as_float(y & 0xFFFF0000u)};
+        }
+    };
+    auto store = [&](int b) {
+        float4v* const sK = (float4v*)(lds + 2 * KBUF * b) + kk * CPR;
+        float4v* const sV = (float4v*)(lds + 2 * KBUF * b + KBUF) + kk * CPR;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            sK[(4 * sl + w) ^ (kk & SW)] = wide(kc, w);
+            sV[4 * sl + w] = wide(vc, w);
+        }
+        if (tid < KT) sW[b * KT + tid] = word;
+    };
+
+    float m_run = -INFINITY, l_run = 0.0f;
+    float4v acc_o[NP][VD];
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int c = 0; c < VD; c++) acc_o[p][c] = float4v{0.f, 0.f, 0.f, 0.f};
+
+    // 16 keys from key k0 of buffer b: lane (g, r16) has keys 4g + i of column r16
+    auto tile = [&](int b, int k0) {
+        const float4v* const sK = (const float4v*)(lds + 2 * KBUF * b) + (k0 + r16) * CPR;
+        const float* const sV = (const float*)(lds + 2 * KBUF * b + KBUF) + (k0 + 4 * g) * D + VD * r16;
+        const u32x4 w4 = *(const u32x4*)(sW + b * KT + k0 + 4 * g);
+        if (!__any(row_ok && (((w4.x | w4.y | w4.z | w4.w) >> bit) & 1u))) return;
+        float4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            const float4v ka = sK[(4 * m + g) ^ (r16 & SW)];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[e], qb[m][e], acc, 0, 0, 0);
+        }
+        float sf[4];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            sf[i] = (w4[i] >> bit) & 1u ? acc[i] * a.scale2 : -INFINITY;
+            mx = fmaxf(mx, sf[i]);
+        }
+        if (__any(mx > m_run + 5.5f)) {
+            const float m_new = fmaxf(m_run, wave_max_g(mx));
+            if (__any(m_run != -INFINITY)) {
+                const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                l_run *= alpha;
+                float f[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) f[i] = __shfl(alpha, 4 * g + i);
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+#pragma unroll
+                    for (int c = 0; c < VD; c++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc_o[p][c][i] *= f[i];
+            }
+            m_run = m_new;
+        }
+        const float mref = m_run == -INFINITY ? 0.0f : m_run;
+        float pr[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            pr[i] = __builtin_amdgcn_exp2f(sf[i] - mref);
+            l_run += pr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                const vecv vv = *(const vecv*)(sV + i * D + 16 * VD * p);
+#pragma unroll
+                for (int c = 0; c < VD; c++)
+                    acc_o[p][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[i], vv[c], acc_o[p][c], 0, 0, 0);
+            }
+    };
+
+    if (t0 < t1) {
+        ki = gk[t0 * KT + kk];
+        load(t0);
+        if (t0 + 1 < t1) ki = gk[(t0 + 1) * KT + kk];
+        store(0);
+        if (t0 + 1 < t1) load(t0 + 1);
+        if (t0 + 2 < t1) ki = gk[(t0 + 2) * KT + kk];
+    }
+    __syncthreads();
+    for (int t = t0; t < t1; t++) {
+        const int b = (t - t0) & 1;
+        if (t + 1 < t1) {
+            store(b ^ 1);
+            if (t + 2 < t1) load(t + 2);
+            if (t + 3 < t1) ki = gk[(t + 3) * KT + kk];
+        }
+        if (wave_live) {
+#pragma unroll 2
+            for (int k0 = 0; k0 < KT; k0 += 16) tile(b, k0);
+        }
+        __syncthreads();
+    }
+
+    // column 4g + i of the wave, dims 16 VD p + VD r16 + c
+    const float lsum = wave_sum_g(l_run);
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float l = __shfl(lsum, 4 * g + i);
+        const int row = wrow0 + 4 * g + i;
+        if (row >= row_end) continue;
+        if (n_split > 1) {
+            float* prow = a.part_o + (((int64_t)h * n_split + sp) * a.PR - a.prow0 + row) * D;
+#pragma unroll
+            for (int p = 0; p < NP; p++)
+#pragma unroll
+                for (int c = 0; c < VD; c++) prow[16 * VD * p + VD * r16 + c] = acc_o[p][c][i];
+            continue;
+        }
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        bad |= !(fabsf(l) < INFINITY);
+        const int64_t o0 = ((int64_t)(h * a.G + row % a.G) * a.L + row / a.G) * D;
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int c = 0; c < VD; c++) {
+                const float y = acc_o[p][c][i] * inv;
+                bad |= !(fabsf(y) < INFINITY);
+                store_as(a.out, a.q_dtype, o0 + 16 * VD * p + VD * r16 + c, y);
+            }
+    }
+    if (n_split > 1) {
+        if (g == 0 && row_ok)
+            a.part_ml[((int64_t)h * n_split + sp) * a.PR - a.prow0 + rho] = float2{m_run, lsum};
+    } else if (bad) {
+        a.flags[qt * a.hkv + h] = 1;
+    }
+}
+
+// Its merge: grid (rows of the split groups, KV heads), D threads (dims).
+__global__ void dlsa_rows32_merge_kernel(DlsaRowsArgs a) {
+    const int D = blockDim.x, d = threadIdx.x, pr = blockIdx.x, h = blockIdx.y;
+    const int row = a.prow0 + pr, fl = row / (a.NR * a.G) * a.hkv + h;
+    if (a.flags[fl]) return;
+    const int64_t base = (int64_t)h * a.n_split * a.PR + pr;
+    float M = -INFINITY, o = 0.0f, l = 0.0f;
+    for (int c0 = 0; c0 < a.n_split; c0 += 4) {
+        float2 ml[4];
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int64_t at = base + (int64_t)min(c0 + i, a.n_split - 1) * a.PR;
+            ml[i] = a.part_ml[at];
+            x[i] = a.part_o[at * D + d];
+            if (c0 + i >= a.n_split) ml[i] = float2{-INFINITY, 0.0f};
+        }
+        float m = M;
+#pragma unroll
+        for (int i = 0; i < 4; i++) m = fmaxf(m, ml[i].x);
+        if (m == -INFINITY) continue;
+        const float f0 = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - m);
+        o *= f0;
+        l *= f0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float f = ml[i].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[i].x - m);
+            o = __builtin_fmaf(f, x[i], o);
+            l = __builtin_fmaf(f, ml[i].y, l);
+        }
+        M = m;
+    }
+    const float y = l > 0.0f ? o / l : 0.0f;
+    if (!(fabsf(y) < INFINITY) || !(fabsf(l) < INFINITY)) a.flags[fl] = 1;
+    store_as(a.out, a.q_dtype, ((int64_t)(h * a.G + row % a.G) * a.L + row / a.G) * D + d, y);
+}
+
 std::mutex g_plan_mu;
 std::map<std::pair<int, hipStream_t>, GrowBuffer> g_plan_ws;
 
@@ -560,29 +825,55 @@ int launch_rows(const DlsaRowsArgs& a, int grid, hipStream_t stream) {
     return QW_OK;
 }
 
+template <int D, int DKV>
+int launch_rows32(const DlsaRowsArgs& a, int grid, hipStream_t stream) {
+    const size_t shmem = (size_t)4 * 32768 + 2 * (8192 / D) * sizeof(uint32_t);
+    if (int rc = ensure_dynamic_lds((const void*)dlsa_rows32_kernel<D, DKV>, shmem)) return rc;
+    hipLaunchKernelGGL((dlsa_rows32_kernel<D, DKV>), dim3(grid), dim3(512), shmem, stream, a);
+    QW_HIP_CHECK(hipGetLastError());
+    if (a.n_split > 1) {
+        hipLaunchKernelGGL(dlsa_rows32_merge_kernel, dim3(a.PR, a.hkv), dim3(D), 0, stream, a);
+        QW_HIP_CHECK(hipGetLastError());
+    }
+    return QW_OK;
+}
+
+template <int DKV>
+int launch_rows32(const DlsaRowsArgs& a, int D, int grid, hipStream_t stream) {
+    switch (D) {
+        case 32: return launch_rows32<32, DKV>(a, grid, stream);
+        case 64: return launch_rows32<64, DKV>(a, grid, stream);
+        case 128: return launch_rows32<128, DKV>(a, grid, stream);
+        default: return launch_rows32<256, DKV>(a, grid, stream);
+    }
+}
+
 }  // namespace
 
 // A group's union may hold 0.35 of its rows' entries less 1500 keys (the launches'
 // fixed cost): there the tiles cost what gathering the rows by pairs does (512 rows
 // in groups of 20, D = 256: of 2048 entries 334 against 364 us at 0.3, 407 at 0.4; of
-// 512 entries 98 against 106 us at 0.2, 126 at 0.3). The typed kernel behind the bf16
-// calls takes fifteen times as long a row (512 rows of 4612: 7.6 ms), so there any
-// union is served.
-static int64_t union_limit(int width, int NR, bool bf16) {
-    return (int64_t)((bf16 ? 1.0 : 0.35) * NR * width) - (bf16 ? 0 : 1500);
+// 512 entries 98 against 106 us at 0.2, 126 at 0.3). The typed kernel behind the
+// other types' calls takes fifteen times as long a row (512 rows of 4612: 7.6 ms), so there nearly any union is
+// served (in fp32 3.8 ms at 0.45 of the entries).
+static int64_t union_limit(int width, int NR, bool typed) {
+    return (int64_t)((typed ? 0.9 : 0.35) * NR * width) - (typed ? 0 : 1500);
 }
 
 int dlsa_rows_per_group(int G) { return std::min(32, 128 / G) & ~1; }
 
-int dlsa_rows_attention(const void* q, const void* k, const void* v, bool bf16, int64_t khs,
-                        int64_t krs, int64_t vhs, int64_t vrs, const int32_t* lists,
+int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v, int kv_dtype,
+                        int64_t khs, int64_t krs, int64_t vhs, int64_t vrs, const int32_t* lists,
                         const int32_t* lengths, int n_rows, int width, int n_q_heads,
                         int n_kv_heads, int D, int n_keys, float scale, void* out,
                         const int** flags, hipStream_t stream) {
     const int G = n_q_heads / n_kv_heads, NR = dlsa_rows_per_group(G);
-    const int KT = 16384 / D, groups = (n_rows + NR - 1) / NR;
+    const bool fp16 = q_dtype == QW_DTYPE_F16 && kv_dtype == QW_DTYPE_F16;
+    const bool bf16 = q_dtype == QW_DTYPE_BF16 && kv_dtype == QW_DTYPE_BF16;
+    const bool rows32 = !(fp16 || bf16) || D == 32;
+    const int KT = (rows32 ? 8192 : 16384) / D, groups = (n_rows + NR - 1) / NR;
     const int64_t most = std::min<int64_t>(n_keys, (int64_t)NR * width);
-    const int max_union = (int)std::min<int64_t>(most, std::max<int64_t>(KT, union_limit(width, NR, bf16)));
+    const int max_union = (int)std::min<int64_t>(most, std::max<int64_t>(KT, union_limit(width, NR, !fp16 || rows32)));
     const int cap = (max_union + KT - 1) / KT * KT;
     // whole rounds of unsplit workgroups, the rest split over their keys
     DlsaRowsArgs a;
@@ -590,8 +881,9 @@ int dlsa_rows_attention(const void* q, const void* k, const void* v, bool bf16, 
     int q_main = 0;
     if (units >= 256 && 256 % n_kv_heads == 0) q_main = units / 256 * (256 / n_kv_heads);
     const int tail = (groups - q_main) * n_kv_heads;
-    const int tiles = (width + KT - 1) / KT;
-    a.n_split = tail > 0 ? std::max(1, std::min({256 / tail, tiles / 2, 32})) : 1;
+    // (splits of at least four tiles of the largest union served; those past a
+    // smaller one's end cost a launch slot and an empty partial)
+    a.n_split = tail > 0 ? std::max(1, std::min({256 / tail, cap / KT / 4, 32})) : 1;
     a.n_main = q_main * n_kv_heads;
     a.qt0 = q_main;
     a.prow0 = q_main * NR * G;
@@ -645,6 +937,11 @@ int dlsa_rows_attention(const void* q, const void* k, const void* v, bool bf16, 
                        counts, a.flags);
     QW_HIP_CHECK(hipGetLastError());
     const int grid = a.n_main + (groups - q_main) * n_kv_heads * a.n_split;
+    a.q_dtype = q_dtype;
+    if (rows32)
+        return kv_dtype == QW_DTYPE_F32   ? launch_rows32<QW_DTYPE_F32>(a, D, grid, stream)
+               : kv_dtype == QW_DTYPE_F16 ? launch_rows32<QW_DTYPE_F16>(a, D, grid, stream)
+                                          : launch_rows32<QW_DTYPE_BF16>(a, D, grid, stream);
     if (bf16)
         return D == 256   ? launch_rows<256, true>(a, grid, stream)
                : D == 128 ? launch_rows<128, true>(a, grid, stream)

@@ -324,18 +324,19 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     a.scale = scale;
     a.flags = nullptr;
     a.group_rows = 1;
-    // bf16 throughout and laid out for 16-byte row pieces: neighbouring rows share
-    // their keys' gathers (dlsa_rows.hip), and the kernel here serves the groups
-    // which that leaves (or every row, without room for its lists). From 20k entries
-    // over all heads: 512 rows of 4612 entries (24 heads over 4, D = 256) 7572 -> 157
-    // us, 48 rows of 128 79 -> 33 to 54 us.
+    // Rows laid out for 16-byte pieces: neighbouring rows share their keys' gathers
+    // (dlsa_rows.hip), and the kernel here serves the groups which that leaves (or
+    // every row, without room for its lists). From 20k entries over all heads at
+    // D = 256 (as many bytes at others): 512 rows of 4612 entries (24 heads over 4, D =
+    // 256) in bf16 7572 -> 157 us, in f32 7530 -> 744 us; 48 rows of 128 in bf16 79 ->
+    // 38 us, in f32 78 -> 61 us.
+    const int64_t per16 = 16 / (int64_t)es;
     const bool aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 &&
-                         khs % 8 == 0 && krs % 8 == 0 && vhs % 8 == 0 && vrs % 8 == 0;
-    if (auto_one_pass && q_dtype == QW_DTYPE_BF16 && kv_dtype == QW_DTYPE_BF16 && head_dim >= 64 &&
-        aligned && (int64_t)n_rows * width * n_kv_heads >= 20000) {
-        const int rc = dlsa_rows_attention(q, k, v, true, khs, krs, vhs, vrs, lists, lengths, n_rows,
-                                           width, n_q_heads, n_kv_heads, head_dim, n_keys, scale, out,
-                                           &a.flags, stream);
+                         khs % per16 == 0 && krs % per16 == 0 && vhs % per16 == 0 && vrs % per16 == 0;
+    if (auto_one_pass && aligned && (int64_t)n_rows * width * n_kv_heads * head_dim >= 20000 * 256) {
+        const int rc = dlsa_rows_attention(q, q_dtype, k, v, kv_dtype, khs, krs, vhs, vrs, lists,
+                                           lengths, n_rows, width, n_q_heads, n_kv_heads, head_dim,
+                                           n_keys, scale, out, &a.flags, stream);
         if (rc == QW_OK)
             a.group_rows = dlsa_rows_per_group(G);
         else if (rc != QW_ERR_STATE && rc != QW_ERR_OUT_OF_MEMORY)

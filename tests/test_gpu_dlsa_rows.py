@@ -54,7 +54,7 @@ def _run(q, k, v, lists, lengths, scale, bf16):
 
 
 CASES = [
-    # hq, hkv, D, L, T, W, kind (fp16 calls take the kernel from 96 rows and 850k entries over all heads)
+    # hq, hkv, D, L, T, W, kind (fp16 calls take the kernel from 850k entries over all heads)
     (24, 4, 256, 101, 8000, 2200, "sliding"),   # the last group one row
     (24, 4, 256, 700, 2000, 320, "shared"),     # the union exactly five tiles
     (24, 4, 256, 700, 2000, 321, "shared"),     # one key past them
@@ -73,7 +73,7 @@ CASES = [
 @pytest.mark.parametrize("hq,hkv,D,L,T,W,kind", CASES)
 def test_rows_match_oracle(hq, hkv, D, L, T, W, kind, bf16):
     print(f"case hq={hq} hkv={hkv} D={D} L={L} T={T} W={W} {kind} bf16={bf16}", flush=True)
-    assert L >= 96 and L * W * hkv >= 850000, "a shape of the kernel"
+    assert L >= 32 and L * hkv > 256 and L * W * hkv >= 850000, "a shape of the kernel"
     if bf16 and hq // hkv > 8:
         pytest.skip("the typed read takes at most 8 heads a KV head")
     r = rng(hq + D + L + T + W)
@@ -123,3 +123,41 @@ def test_infinite_values_stay_with_the_rows_that_list_them(bf16):
     _check(out[:, rows], q[:, rows], k, np.where(np.isinf(v), 0, v), lists[rows], lengths[rows], 0.1,
            bf16, "rows without the infinite key")
     assert not np.isfinite(out[:, 41, 5]).any()
+
+
+TYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+# half a unit in the last place of the output's type, relative to the value
+ROUND = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 0.0}
+
+
+@pytest.mark.parametrize("qt,kt", [("f32", "f32"), ("bf16", "f16"), ("f16", "f32"), ("f32", "bf16"),
+                                   ("f16", "bf16"), ("f16", "f16")])
+@pytest.mark.parametrize("hq,hkv,D,L,T,W,kind", [
+    (24, 4, 256, 101, 3000, 300, "sliding"),   # 32-key tiles; the last group one row
+    (16, 2, 128, 70, 900, 128, "shared"),      # the union exactly two tiles
+    (16, 2, 128, 70, 900, 129, "own"),
+    (8, 8, 64, 99, 2000, 333, "mixed"),        # G = 1
+    (6, 1, 32, 200, 2000, 500, "sliding"),     # 256-key tiles
+])
+def test_typed_rows_match_float64(qt, kt, hq, hkv, D, L, T, W, kind):
+    """fp32 arithmetic: 1e-5 of the row, as the reference holds its f32 read (dlsa_attention.rs:
+    213-255), and the output's rounding."""
+    import qw_amd
+
+    print(f"case q={qt} kv={kt} hq={hq} hkv={hkv} D={D} L={L} W={W} {kind}", flush=True)
+    r = rng(hq + D + L + T + W)
+    dev = [torch.from_numpy(r.standard_normal(s).astype(np.float32)).to(TYPES[t]).cuda()
+           for s, t in (((hq, L, D), qt), ((hkv, T, D), kt), ((hkv, T, D), kt))]
+    q, k, v = (x.float().cpu().numpy() for x in dev)
+    lists = _lists(r, kind, L, W, T)
+    lists[::5, 3::11] = -1
+    lists[::7, 5::13] = T + 4
+    lengths = np.where(np.arange(L) % 9 == 4, r.integers(0, W, L), W).astype(np.int32)
+    lengths[2] = 0
+    out = qw_amd.sparse_attention_typed(*dev, _gpu(lists), _gpu(lengths), D ** -0.5)[0]
+    assert out.dtype == TYPES[qt]
+    out = out.float().cpu().numpy()
+    assert np.all(out[:, 2] == 0)
+    ref = oracle.dlsa_attention_f64(q, k, v, lists, lengths, D ** -0.5)
+    bound = np.abs(ref) * ROUND[qt] + 1e-5 * np.linalg.norm(ref, axis=-1, keepdims=True) + 1e-7
+    assert np.isfinite(out).all() and np.all(np.abs(out.astype(np.float64) - ref) <= bound)
