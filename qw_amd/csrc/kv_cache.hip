@@ -318,6 +318,136 @@ __global__ __launch_bounds__(256) void append_affine_kernel(
                     fast_flag, t_old / 8 + blockIdx.x, blockIdx.y, threadIdx.x, blockDim.x, sc);
 }
 
+// The same for many tokens of the affine modes: a thread takes 8 dims of the 8 tokens
+// of one V block, of K or of V (16-byte loads, all issued first), and forms their
+// codes in registers: a group is 8 lanes, its extremes three lane moves a token; lane
+// i of them forms token i's scale and bias for all (the divisions once a group, where
+// every lane of the row-wise form divides) and hands them round; the words of a K row
+// and of the V block's dims are assembled in place and stored whole (V in 16-byte
+// pieces). A workgroup that meets a value that is not finite leaves its blocks to the
+// row-wise form (append_block; the other plane's workgroup stores the same bytes), so
+// such rows are stored as before. VALU-bound, two waves a SIMD (about 200
+// registers): 65536 tokens of 4 heads, D = 256, 4-bit 203 us row-wise -> 125 us, 2048
+// tokens 11.4 -> 8.9 us; 8 heads, D = 128, 8-bit 313 -> 131 us. (Int8's codes have no
+// division to share: 363 -> 376 us at 131072 tokens, so it stays row-wise.)
+template <int D, int BITS>
+__global__ __launch_bounds__(256) void append_affine_blocks_kernel(
+    RowSrc rs, int n_tokens, int t_old, int cap, uint32_t* __restrict__ k_codes,
+    uint32_t* __restrict__ k_params, uint32_t* __restrict__ v_codes, f16* __restrict__ v_params,
+    int* __restrict__ fast_flag) {
+    constexpr int OCT = D / 8, NG = D / kGroup, BPW = 256 / OCT;  // blocks a workgroup
+    constexpr int E = 16 / BITS, NV = BITS / 2;                   // dims a piece of V, pieces
+    __shared__ AppendScratch<D> sc;
+    const int tid = threadIdx.x, h = blockIdx.y, lane = tid & 63, l8 = lane & 7;
+    const bool is_v = blockIdx.z != 0;
+    const int b_first = t_old / 8, b_last = (t_old + n_tokens - 1) / 8;
+    const int blk = b_first + blockIdx.x * BPW + tid / OCT, d0 = tid % OCT * 8, grp = d0 / kGroup;
+    const int r0 = 8 * blk - t_old;  // the source row of the block's first key
+    const bool live = blk <= b_last;
+    half8 x[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int r = min(max(r0 + i, 0), n_tokens - 1);
+        const int64_t src = (int64_t)r * rs.row_stride + (int64_t)h * rs.head_stride + d0;
+        x[i] = *(const half8*)((is_v ? rs.v : rs.k) + src);
+    }
+    const int64_t gblk = (int64_t)h * (cap / 8) + (live ? blk : b_last);
+    u32x4* const vw = (u32x4*)(v_codes + gblk * (D * BITS / 4));
+    u32x4 w[NV];  // the 8 dims' words of the V block, in pieces; earlier tokens' codes stay
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        w[j] = u32x4{0, 0, 0, 0};
+        if (is_v && live && r0 < 0) w[j] = vw[v_phys_dim(d0 + E * j, D, BITS) / E];
+    }
+    bool odd = false;
+    float my_mn = 0.0f, my_mx = 0.0f;  // token l8's extremes in this lane's group
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        float mx = (float)x[i][0], mn = mx;
+        odd |= !(fabsf(mx) < INFINITY);
+#pragma unroll
+        for (int e = 1; e < 8; e++) {
+            const float f = (float)x[i][e];
+            odd |= !(fabsf(f) < INFINITY);
+            mx = fmaxf(mx, f);
+            mn = fminf(mn, f);
+        }
+        mx = fmaxf(mx, lane_xor<1>(mx, lane));
+        mn = fminf(mn, lane_xor<1>(mn, lane));
+        mx = fmaxf(mx, lane_xor<2>(mx, lane));
+        mn = fminf(mn, lane_xor<2>(mn, lane));
+        mx = fmaxf(mx, lane_xor<4>(mx, lane));
+        mn = fminf(mn, lane_xor<4>(mn, lane));
+        if (i == l8) {
+            my_mx = mx;
+            my_mn = mn;
+        }
+    }
+    if (__syncthreads_or(odd)) {
+        for (int b = 0; b < BPW; b++) {
+            const int bb = b_first + blockIdx.x * BPW + b;
+            if (bb > b_last) break;
+            append_block<D>(rs, n_tokens, t_old, BITS, false, cap, k_codes, k_params, v_codes, v_params,
+                            fast_flag, bb, h, tid, 256, sc);
+            __syncthreads();
+        }
+        return;
+    }
+    // the halves are converted again below: their floats are not held over the scan
+#pragma unroll
+    for (int i = 0; i < 8; i++) asm volatile("" : "+v"(x[i]));
+    const AffineGroup q = affine_group(my_mn, my_mx, BITS);
+    const float inv = 1.0f / q.scale;
+    if (live && r0 + l8 >= 0 && r0 + l8 < n_tokens) {
+        half2v sb;
+        sb.x = (f16)q.scale;
+        sb.y = (f16)q.bias;
+        check_fast_scale(sb.x, BITS, fast_flag);
+        if (is_v) {
+            f16* vp = v_params + (gblk * NG + grp) * 16;
+            vp[l8] = sb.x;
+            vp[8 + l8] = sb.y;
+        } else {
+            k_params[(gblk * 8 + l8) * NG + k_param_slot(grp, NG)] = __builtin_bit_cast(uint32_t, sb);
+        }
+    }
+    const int base = lane & ~7;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const AffineGroup qi{__shfl(q.scale, base + i), __shfl(q.bias, base + i)};
+        const float ii = __shfl(inv, base + i);
+        const bool ok = live && r0 + i >= 0 && r0 + i < n_tokens;
+        uint32_t c[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) c[e] = (uint32_t)affine_code_inv((float)x[i][e], qi, ii, BITS);
+        if (!ok) continue;
+        if (!is_v) {
+            uint32_t* row = k_codes + ((gblk * 8 + i) * D + d0) * BITS / 32;
+            if constexpr (BITS == 4) {
+                uint32_t word = 0;
+#pragma unroll
+                for (int e = 0; e < 8; e++) word |= c[e] << (4 * e);
+                *row = word;
+            } else {
+                *(u32x2*)row = u32x2{c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24),
+                                     c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24)};
+            }
+        } else {
+            const int sh = BITS == 4 ? 4 * v4_nibble_pos(i) : 8 * (i & 3);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int at = BITS == 4 ? e & 3 : 2 * (e & 1) + i / 4;
+                const uint32_t m = ((1u << BITS) - 1u) << sh;
+                w[e / E][at] = (w[e / E][at] & ~m) | (c[e] << sh);
+            }
+        }
+    }
+    if (is_v && live) {
+#pragma unroll
+        for (int j = 0; j < NV; j++) vw[v_phys_dim(d0 + E * j, D, BITS) / E] = w[j];
+    }
+}
+
 // fp16 mode append: K rows copied, V transposed into 8-key blocks. A thread takes
 // 8 dims of one block's 8 tokens: 16-byte loads of both (all issued first), K rows
 // stored as they are, a dim's 8 keys of V as one 16-byte piece where the append
@@ -409,6 +539,12 @@ int KVCache::update(const void* k_new, const void* v_new, int n_tokens, hipStrea
     return update_rows(rs, n_tokens, stream);
 }
 
+// Halves of K from which an affine append takes the block-wise form (below it its few long
+// chains cost more than the row-wise form's divisions): 4-bit, D = 256, 4 heads, row-wise
+// against it, 700 tokens 8.0 / 8.4 us, 1024 8.2 / 8.5, 1500 9.5 / 8.7, 4096 18.0 / 15.0;
+// 2 heads, 2048 tokens 8.5 / 8.6, 4096 12.2 / 10.0; 16 heads, 512 tokens 12.0 / 9.8.
+constexpr int64_t kBlockAppend = 5 << 18;
+
 int KVCache::update_rows(const RowSrc& rs, int n_tokens, hipStream_t stream) {
     if (n_tokens == 0) return QW_OK;
     DeviceGuard dg(device);
@@ -425,7 +561,24 @@ int KVCache::update_rows(const RowSrc& rs, int n_tokens, hipStream_t stream) {
     } else if (affine()) {
         const int nblk = (offset + n_tokens - 1) / 8 - offset / 8 + 1;
         dim3 grid(nblk, hkv);
-        if (D == 256)
+        // many rows as they are, their pieces on 16 bytes: the block-wise form
+        if ((int64_t)n_tokens * hkv * D >= kBlockAppend && !int8() && rs.rope_dims == 0 &&
+            (((uintptr_t)rs.k | (uintptr_t)rs.v) % 16 == 0) && rs.row_stride % 8 == 0 &&
+            rs.head_stride % 8 == 0) {
+            const int bpw = 256 / (D / 8);
+            grid = dim3((nblk + bpw - 1) / bpw, hkv, 2);
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, rs, n_tokens, offset, cap,
+                                   (uint32_t*)k_data, k_params, (uint32_t*)v_data, (f16*)v_params,
+                                   fast_flag);
+            };
+            if (D == 256)
+                bits == 8 ? launch(append_affine_blocks_kernel<256, 8>)
+                          : launch(append_affine_blocks_kernel<256, 4>);
+            else
+                bits == 8 ? launch(append_affine_blocks_kernel<128, 8>)
+                          : launch(append_affine_blocks_kernel<128, 4>);
+        } else if (D == 256)
             hipLaunchKernelGGL(append_affine_kernel<256>, grid, dim3(256), 0, stream,
                                rs, n_tokens, offset, bits,
                                int8() ? 1 : 0, cap, (uint32_t*)k_data, k_params,

@@ -7,7 +7,8 @@
 // the minimum); q0 = rint(edge / scale); when q0 != 0 the scale is refit to
 // edge / q0 and the bias is the edge. code = clamp(rint((w - bias) / scale)),
 // computed with the fp32 scale and bias; fp16(scale), fp16(bias) are stored.
-// IEEE division and round-half-even rint throughout (no reciprocal tricks).
+// IEEE division and round-half-even rint throughout (affine_code_inv: wherever they
+// decide).
 #pragma once
 
 #include "qw_common.hpp"
@@ -39,6 +40,18 @@ __device__ inline float affine_code(float x, AffineGroup q, int bits) {
     const float n_bins = (float)((1 << bits) - 1);
     float c = __builtin_rintf((x - q.bias) / q.scale);
     return c < 0.0f ? 0.0f : (c > n_bins ? n_bins : c);
+}
+
+// The same code by a multiplication: inv = 1 / scale (IEEE). The product is within
+// three units in the last place of the quotient, below 2^-14 for the 0 .. 255 a code
+// can take, so where it is further than 2^-11 from a tie both round to the same
+// integer; nearer, the division decides. x finite.
+__device__ inline float affine_code_inv(float x, AffineGroup q, float inv, int bits) {
+    const float n_bins = (float)((1 << bits) - 1);
+    const float t = x - q.bias, p = t * inv;
+    float c = __builtin_rintf(p);
+    if (fabsf(p - c) > 0.5f - 0x1p-11f) c = __builtin_rintf(t / q.scale);
+    return fminf(fmaxf(c, 0.0f), n_bins);
 }
 
 // MLX composite dequantize f16(f16(code * scale) + bias), as a float: the

@@ -76,3 +76,38 @@ def test_fp16_pointers_off_16_bytes():
     got = out[1:].cpu().numpy().reshape(2, H, n, D)
     np.testing.assert_array_equal(got[0], k)
     np.testing.assert_array_equal(got[1], v)
+
+
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("mode", ["affine4", "affine8"])
+@pytest.mark.parametrize("odd", [False, True])
+def test_long_affine_append_stores_the_bytes_of_short_ones(mode, D, odd):
+    """One append past the block-wise form's line (4 * n * D >= 5 << 18) from the middle of a block
+    to the middle of one, against the same rows in short appends: ties, constant, zero, tiny and
+    the largest groups; with rows that are not finite as well."""
+    import qw_amd
+
+    r, H, n = rng(D + odd), 4, (5 << 18) // (4 * D) + 11
+    k, v = (r.standard_normal((H, n, D)).astype(np.float16) for _ in range(2))
+    bins = (1 << int(mode[-1])) - 1
+    for x in (k, v):
+        x[0, 20:60] = (r.integers(0, 2 * bins + 1, (40, D)) / 2 - bins / 2).astype(np.float16)
+        x[1, 30:40] = np.float16(0.37)
+        x[1, 50:60] = 0
+        x[2, 70:90] = (x[2, 70:90].astype(np.float32) * 1e-6).astype(np.float16)
+        x[2, 100:120] = np.where(r.random((20, D)) < 0.5, np.float16(65504), np.float16(-65504))
+        x[3, n - 20:] *= np.float16(300)
+    if odd:
+        k[0, 33, 7], k[3, n - 1, D - 1], k[1, 3, 64] = np.inf, np.nan, -np.inf
+        v[0, 35, 9], v[2, n - 2, 0], v[1, 0, 1] = np.nan, -np.inf, np.inf
+    one, many = (qw_amd.KVCache(mode, H, D, capacity=n + 64) for _ in range(2))
+    for c in (one, many):
+        c.update(_gpu(k[:, :5]), _gpu(v[:, :5]))
+    one.update(_gpu(k[:, 5:]), _gpu(v[:, 5:]))
+    for at in range(5, n, 200):
+        many.update(_gpu(k[:, at:at + 200]), _gpu(v[:, at:at + 200]))
+    a, b = one.snapshot_tensors(), many.snapshot_tensors()
+    assert a.keys() == b.keys()
+    for name in a:
+        x, y = (np.asarray(t.cpu() if hasattr(t, "cpu") else t) for t in (a[name], b[name]))
+        np.testing.assert_array_equal(x.view(np.uint8), y.view(np.uint8), err_msg=name)
