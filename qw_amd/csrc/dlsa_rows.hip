@@ -862,6 +862,23 @@ static int64_t union_limit(int width, int NR, bool typed) {
 
 int dlsa_rows_per_group(int G) { return std::min(32, 128 / G) & ~1; }
 
+// The plan and its launches take some 40 us, so the calls that one round of row
+// workgroups serves (256) stay there. By rows against this, rows of a group sharing all
+// keys / a quarter: 66 rows of 4612 entries (24 heads over 4, D = 256) 221 -> 66 / 224 ->
+// 110 us, 48 rows (32 over 8, D = 128) 115 -> 61 / 171 -> 84 us, 512 rows of 512 63 -> 56
+// / 106 -> 98 us; but 192 rows of 512 34 -> 46 / 57 -> 58 us.
+// Where the keys are more than a served union may hold, rows that share next to nothing
+// pay the plan for nothing, or for a part of the groups (24 over 4, 4612 entries of 33k
+// keys in blocks drawn for each row: D = 128, 66 rows 107 -> 178, 400 490 -> 536, 1500
+// 1200 -> 1239 us; D = 256, 140 rows 416 -> 452, 400 853 -> 889, 1500 2646 -> 2506 us), and
+// nothing on the host tells them from rows that share (450 -> 196 us at 400): such a call
+// is taken from 12M entries of 256 dims over the heads, where that loss is at most 3 %.
+bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys) {
+    const int64_t entries = (int64_t)n_rows * width * n_kv_heads;
+    if (n_rows < 32 || n_rows * (int64_t)n_kv_heads <= 256 || entries < 850000) return false;
+    return n_keys <= union_limit(width, dlsa_rows_per_group(G), false) || entries * D >= (int64_t)256 * 12000000;
+}
+
 int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v, int kv_dtype,
                         int64_t khs, int64_t krs, int64_t vhs, int64_t vrs, const int32_t* lists,
                         const int32_t* lengths, int n_rows, int width, int n_q_heads,

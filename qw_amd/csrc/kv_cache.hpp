@@ -248,16 +248,8 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
 // 0; the caller launches a row-by-row kernel behind it for the others.
 // QW_ERR_STATE / QW_ERR_OUT_OF_MEMORY, with nothing enqueued, without a workspace.
 int dlsa_rows_per_group(int G);
-// Whether a one-pass fp16 call is large enough for it: the lists' union takes two
-// more launches and some 30 us, lost where the rows turn out to share too little, so
-// the calls that one round of row workgroups serves (256) stay there.
-// By rows against this, rows of a group sharing all keys / a quarter / next to none:
-// 66 rows of 4612 entries (24 heads over 4, D = 256) 221 -> 66 / 224 -> 110 / 222 ->
-// 255 us, 48 rows (32 over 8, D = 128) 115 -> 61 / 171 -> 84 / 176 -> 118 us, 512 rows of
-// 512 63 -> 56 / 106 -> 98 us; but 192 rows of 512 34 -> 46 / 57 -> 58 us.
-inline bool dlsa_rows_pays(int n_rows, int width, int hkv) {
-    return n_rows >= 32 && n_rows * (int64_t)hkv > 256 && (int64_t)n_rows * width * hkv >= 850000;
-}
+// Whether a one-pass fp16 call takes it (the rule and both sides in dlsa_rows.hip).
+bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys);
 int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v, int kv_dtype,
                         int64_t k_head_stride, int64_t k_row_stride, int64_t v_head_stride, int64_t v_row_stride,
                         const int32_t* lists, const int32_t* lengths, int n_rows, int width,

@@ -66,6 +66,12 @@ CASES = [
     (16, 1, 128, 600, 4000, 1500, "shared"),    # G = 16: 8 rows a group
     (24, 4, 256, 96, 90000, 2300, "sliding"),   # three bitmap passes
     (24, 4, 256, 1300, 2600, 400, "sliding"),   # whole rounds and a split rest
+    (24, 4, 256, 440, 2000, 512, "shared"),     # eight tiles of lists long enough for fp16
+    (24, 4, 256, 440, 2000, 513, "shared"),
+    (24, 4, 256, 700, 700, 321, "shared"),      # (fp16 takes few rows only where any union pays:
+    (16, 2, 64, 300, 6000, 1500, "sliding"),    # these are fp16's of the kinds above)
+    (16, 1, 128, 600, 2500, 1500, "shared"),
+    (24, 4, 256, 1300, 2600, 800, "sliding"),
 ]
 
 
