@@ -103,3 +103,24 @@ def test_masked_cache_with_extreme_scales(mode):
     ref = _reference(cache, mode, q, D, 1 / 16, False, m)
     keep = [0, 2, 3, 4]
     assert_close(out[:, keep], ref[:, keep], f"{mode} extreme scales")
+
+
+@pytest.mark.parametrize("D,L", [(256, 13), (128, 40)])
+def test_masked_largest_weight_is_not_rounded(D, L):
+    """As test_gpu_rows.py's: a key that outweighs an earlier one has a weight of exactly 1 in fp16,
+    and rows of ones come back as ones."""
+    import qw_amd
+
+    hq, hkv, T = 24, 4, 1500
+    s = np.linspace(1, 5.4, L).astype(np.float16)
+    q = np.zeros((hq, L, D), np.float16)
+    q[:, :, 0] = s * np.float16(16)
+    k = np.zeros((hkv, T, D), np.float16)
+    k[:, :, 0] = -60
+    k[:, 1, 0] = 0                      # in one 64 / 128-key tile's first half, the winner in
+    k[:, 200, 0] = 1                    # a later tile of the same split
+    mask = torch.ones((1, 1, L, T), dtype=torch.bool, device="cuda:0")
+    cache = qw_amd.KVCache("fp16", hkv, D)
+    cache.update(_gpu(k), _gpu(np.ones_like(k)))
+    out = _np(cache.attention_general(_gpu(q), 1 / 16, mask=mask))[0]
+    assert np.all(out == 1), np.unique(out)

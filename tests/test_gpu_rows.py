@@ -112,3 +112,23 @@ def test_rows_route_agrees_with_the_general_kernel():
                                          vv[:, :T - L + i + step], 1 / 16))[0]
              for i in range(0, L, step)]
     assert_close(whole, np.concatenate(parts, axis=1), "one call vs pieces")
+
+
+@pytest.mark.parametrize("hkv,D", [(4, 256), (4, 128), (2, 64)])
+def test_rows_largest_weight_is_not_rounded(hkv, D):
+    """One key outweighs an earlier one by a score of 1 to 5, V is 1: P is taken against the running
+    maximum, so that key's weight is exactly 1 in fp16. What is left is the other key's rounding
+    (below e^-1 2^-12) and fp32 sums: the result is within 2^-12 of 1, which rounds to 1."""
+    import qw_amd
+
+    G, L, T = 6, 200, 1300
+    s = np.linspace(1, 5.4, L).astype(np.float16)
+    q = np.zeros((G * hkv, L, D), np.float16)
+    q[:, :, 0] = s * np.float16(16)
+    k = np.zeros((hkv, T, D), np.float16)
+    k[:, :, 0] = -60
+    k[:, 3, 0] = 0
+    k[:, 66 if D == 256 else 130, 0] = 1  # the next 64- or 128-key step of the same key split
+    assert (G * L - 100) * T >= 1300000, "a shape of the row kernel"
+    out = _np(qw_amd.attention(_gpu(q), _gpu(k), _gpu(np.ones_like(k)), 1 / 16))[0]
+    assert np.all(out == 1), np.unique(out)
