@@ -583,9 +583,25 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
     };
     // Dequantize a stage into LDS buffer b: K row kk, chunks 4 q32 .. +3 (dims
     // in the order of the Q operand); V block vb, slots 4 vj .. +3 (8 keys each).
-    auto store = [&](const Stage& st, int b) {
+    // Masked launches: tile t's keys past the last one that a row of the workgroup may
+    // see, rows past the cache's offset among them, go in as zeros of V (a trimmed
+    // append may have left anything there).
+    auto store = [&](const Stage& st, int b, int t) {
         half8* const sK8 = (half8*)(lds + BUF * b);
         half8* const sV8 = (half8*)(lds + BUF * b + KBUF);
+        u32x4 keep[MASK ? PER : 1];
+        if constexpr (MASK) {
+#pragma unroll
+            for (int j = 0; j < PER; j++) keep[j] = u32x4{~0u, ~0u, ~0u, ~0u};
+            if ((t + 1) * KT - 1 > wg_lim) {
+#pragma unroll
+                for (int j = 0; j < PER; j++) keep[j] = keep_keys(wg_lim + 1 - (t * KT + 8 * vb[j]));
+            }
+        }
+        auto kept = [&](half8 y, int j) {
+            if constexpr (MASK) y = as_h8(__builtin_bit_cast(u32x4, y) & keep[j]);
+            return y;
+        };
 #pragma unroll
         for (int j = 0; j < PER; j++) {
             // chunks 4 q32 + w of key kk: KT chunks apart
@@ -619,7 +635,7 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int sl = v_phys_dim(4 * vj[j] + e, D, 16);
-                    vblk[sl + (sl >> 4)] = yv[e];
+                    vblk[sl + (sl >> 4)] = kept(yv[e], j);
                 }
                 continue;
             }
@@ -656,7 +672,7 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
                     y = deq8<FAST>(st.vc[j][e / 2][2 * (e % 2)], st.vc[j][e / 2][2 * (e % 2) + 1], vc);
                 else
                     y = as_h8(st.vc[j][e]);
-                vblk[4 * vj[j] + e + (vj[j] >> 2)] = y;  // slot s at s + (s >> 4)
+                vblk[4 * vj[j] + e + (vj[j] >> 2)] = kept(y, j);  // slot s at s + (s >> 4)
             }
         }
     };
@@ -983,7 +999,7 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
         // it, copied out to its image
         Stage st;
         load(st, blockIdx.x);
-        store(st, 0);
+        store(st, 0, blockIdx.x);
         __syncthreads();
         char* dst = a.img_w + ((int64_t)h * a.img_tiles + blockIdx.x) * BUF;
         for (int i = 16 * tid; i < BUF; i += 16 * 64 * NW) *(u32x4*)(dst + i) = *(const u32x4*)(lds + i);
@@ -1046,14 +1062,14 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
         Stage s0, s1;
         if (t0 < t1) {
             load(s0, t0);
-            store(s0, 0);
+            store(s0, 0, t0);
             if (t0 + 1 < t1) load(s0, t0 + 1);
             if (t0 + 2 < t1) load(s1, t0 + 2);
         }
         __syncthreads();
         auto round = [&](Stage& sa, int t, int b) {
             if (t + 1 < t1) {
-                store(sa, b ^ 1);
+                store(sa, b ^ 1, t + 1);
                 if (t + 3 < t1) load(sa, t + 3);
             }
             if (wave_live && t * KT <= wave_lim && (!WIN || (t + 1) * KT > wave_lo_min))
@@ -1068,14 +1084,14 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
         Stage st;
         if (t0 < t1) {
             load(st, t0);
-            store(st, 0);
+            store(st, 0, t0);
             if (t0 + 1 < t1) load(st, t0 + 1);
         }
         __syncthreads();
         for (int t = t0; t < t1; t++) {
             const int b = (t - t0) & 1;
             if (t + 1 < t1) {
-                store(st, b ^ 1);
+                store(st, b ^ 1, t + 1);
                 if (t + 2 < t1) load(st, t + 2);
             }
             if (wave_live && t * KT <= wave_lim && (!WIN || (t + 1) * KT > wave_lo_min))

@@ -64,6 +64,15 @@ __device__ __forceinline__ float wave_sum_g(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Bits that keep the first n keys of an 8-key piece of V (key e in half e) and zero the
+// others: a hidden key has weight 0 in P . V, but 0 x inf is NaN.
+__device__ __forceinline__ u32x4 keep_keys(int n) {
+    u32x4 m;
+#pragma unroll
+    for (int j = 0; j < 4; j++) m[j] = (2 * j < n ? 0xFFFFu : 0u) | (2 * j + 1 < n ? 0xFFFF0000u : 0u);
+    return m;
+}
+
 // An explicit mask in a key tile: a lane's 8 consecutive keys of one row, from
 // element offset off of a mask with key stride 1 (any alignment), n of them inside
 // the mask (n <= 0: none); raw, so that the loads can be issued ahead of the MFMAs.

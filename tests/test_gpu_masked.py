@@ -124,3 +124,33 @@ def test_masked_largest_weight_is_not_rounded(D, L):
     cache.update(_gpu(k), _gpu(np.ones_like(k)))
     out = _np(cache.attention_general(_gpu(q), 1 / 16, mask=mask))[0]
     assert np.all(out == 1), np.unique(out)
+
+
+@pytest.mark.parametrize("mode", ["affine4", "affine8", "int8", "turbo4", "fp16"])
+@pytest.mark.parametrize("D,L,causal", [(256, 13, False), (128, 40, False), (256, 3, True)])
+def test_masked_cache_after_a_trim(mode, D, L, causal):
+    """Rows that a trim left behind the offset take no part, whatever they hold: the call returns
+    what a cache that never held them does, bit for bit."""
+    import qw_amd
+
+    r = rng(D + L)
+    hq, hkv, T = 24, 4, 700
+    k, v = (r.standard_normal((hkv, T, D)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((hq, L, D)).astype(np.float16)
+    bad = np.zeros((hkv, L + 50, D), np.float16)
+    bad[:, ::2] = np.inf
+    bad[:, 1::2] = np.nan
+    _, view = _mask(r, "bool", 1, L, T)
+    outs = []
+    for poisoned in (False, True):
+        cache = qw_amd.KVCache(mode, hkv, D, capacity=1024)
+        cache.update(_gpu(k[:, :T - L]), _gpu(v[:, :T - L]))
+        if poisoned:
+            cache.update(_gpu(bad), _gpu(bad))
+            cache.trim(L + 50)
+        cache.update(_gpu(k[:, T - L:]), _gpu(v[:, T - L:]))
+        outs.append(_np(cache.attention_general(_gpu(q), D ** -0.5, causal=causal, mask=view))[0])
+    assert np.isfinite(outs[1]).all()
+    # (an affine cache that ever held a scale outside the two-step dequant's exact range rounds in
+    # two steps from then on; both are the same values)
+    np.testing.assert_array_equal(outs[0], outs[1])
