@@ -132,3 +132,40 @@ def test_rows_largest_weight_is_not_rounded(hkv, D):
     assert (G * L - 100) * T >= 1300000, "a shape of the row kernel"
     out = _np(qw_amd.attention(_gpu(q), _gpu(k), _gpu(np.ones_like(k)), 1 / 16))[0]
     assert np.all(out == 1), np.unique(out)
+
+
+@pytest.mark.parametrize("hq,hkv,D,L,T,window,softcap,masked", [
+    (24, 4, 256, 230, 1400, 0, 0.0, False),
+    (24, 4, 256, 230, 1400, 37, 30.0, False),
+    (8, 8, 128, 700, 2305, 0, 0.0, False),
+    (8, 8, 128, 701, 2305, 300, 0.0, False),
+    (8, 8, 128, 700, 2305, 61, 25.0, False),
+    (16, 2, 64, 256, 1281, 0, 0.0, False),
+    (16, 2, 64, 255, 1281, 5, 0.0, False),      # a window inside one 8-key block
+    (24, 4, 256, 100, 1290, 0, 0.0, True),
+])
+def test_rows_keep_keys_outside_their_limits_out(hq, hkv, D, L, T, window, softcap, masked):
+    """Infinite and NaN keys that none of a wave's 16 rows sees (later than the last one's position,
+    earlier than the first one's window) change none of its outputs."""
+    import qw_amd
+
+    G = hq // hkv
+    assert masked or (G * L - 100) * T >= 1300000, "a shape of the row kernel"
+    r = rng(hq + D + L + window)
+    q = _gpu(r.standard_normal((hq, L, D)).astype(np.float16))
+    k, v, kv, vv = _views(r, hkv, T, D, 0)
+    mask = torch.ones((1, 1, L, T), dtype=torch.bool, device="cuda:0") if masked else None
+    call = lambda: _np(qw_amd.attention(q, kv, vv, D ** -0.5, mask, softcap, window, True))[0]  # noqa: E731
+    clean = call()
+    ref = oracle.sdpa_general(_np(q), k, v, D ** -0.5, True, window, softcap)
+    assert_close(clean, ref, f"D={D} L={L} T={T} w={window}")
+    wave = (np.arange(G * L) // 16).reshape(L, G).T                     # of (head in group, row)
+    first, last = T - L + wave * 16 // G, T - L + np.minimum(wave * 16 + 15, G * L - 1) // G
+    for t in (T - L + 20, T - L // 2, T - L // 2 + 5, T - 7):
+        keep = kv[:, t].clone(), vv[:, t].clone()
+        kv[:, t], vv[:, t] = float("nan"), float("inf")
+        blind = (t > last) | ((t < first - window + 1) if window else False)
+        out, blind = call(), np.tile(blind, (hkv, 1))
+        assert blind.any() and np.isfinite(out[blind]).all(), f"key {t}"
+        np.testing.assert_array_equal(out[blind], clean[blind], f"key {t}")
+        kv[:, t], vv[:, t] = keep
