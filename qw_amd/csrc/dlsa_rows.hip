@@ -51,9 +51,21 @@ typedef uint16_t ushort8v __attribute__((ext_vector_type(8)));
 constexpr int kPlanSeg = 40448;  // keys a bitmap pass covers (158 KB of LDS)
 constexpr int kPlanThreads = 1024;
 
+// flags[group][hkv], nonzero for the row-by-row kernel: kLeft before the merge (by the
+// plan, or by the row kernel for all groups together), kBad where an output came out
+// infinite or NaN. No launch decides by a value that it writes: the row kernel reads
+// the plan's counts alone, the merge only whether a flag is kLeft.
+constexpr int kLeft = 1, kBad = 2;
+__device__ __forceinline__ void set_flag(int* f, int value) {
+    __hip_atomic_store(f, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool was_left(const int* f) {
+    return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kLeft;
+}
+
 // Group blockIdx.x: rows NR * blockIdx.x .. +NR-1. Writes its keys (ascending,
 // padded with (0, no rows) to whole tiles of KT), their row words and the count;
-// flags[group][hkv] = 1 and count 0 if the group is not served.
+// count -1 and flags[group][hkv] = kLeft if the group is not served.
 __global__ __launch_bounds__(kPlanThreads) void dlsa_plan_kernel(
     const int32_t* __restrict__ lists, const int32_t* __restrict__ lengths, int L, int W, int T,
     int NR, int KT, int max_union, int cap, int hkv, int32_t* __restrict__ keys,
@@ -170,8 +182,8 @@ __global__ __launch_bounds__(kPlanThreads) void dlsa_plan_kernel(
             gw[i] = 0;
         }
     }
-    if (tid == 0) counts[grp] = bad ? 0 : total;
-    for (int h = tid; h < hkv; h += kPlanThreads) flags[grp * hkv + h] = bad ? 1 : 0;
+    if (tid == 0) counts[grp] = bad ? -1 : total;
+    for (int h = tid; h < hkv; h += kPlanThreads) flags[grp * hkv + h] = bad ? kLeft : 0;
 }
 
 struct DlsaRowsArgs {
@@ -184,8 +196,8 @@ struct DlsaRowsArgs {
     float2* part_ml; // [hkv][n_split][PR] (m in log2 units)
     const int32_t* keys;    // [groups][cap]
     const uint32_t* words;
-    const int* counts;      // [groups]
-    int* flags;             // [groups][hkv]
+    const int* counts;      // [groups] (the plan's, -1: not served)
+    int* flags;             // [groups][hkv], see kLeft
     int L, G, hkv, NR, cap, groups;
     int n_main, qt0, n_split, prow0, PR;  // as RowsArgs (attend_rows.hip)
     float scale2;           // scale * log2(e)
@@ -241,7 +253,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
             qt = a.qt0 + t / (n_split * a.hkv);
         }
     }
-    if (a.flags[qt * a.hkv + h]) return;  // (uniform, before any barrier)
+    if (a.counts[qt] < 0) return;  // (this launch writes no count: all waves leave)
     const int tid = threadIdx.x, lane = tid & 63;
     {
         // Where more than a quarter of the groups is left, the fp16 row kernel serves
@@ -249,9 +261,9 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
         // (512 rows of which half share too little: 649 us, 364 us by rows alone).
         int left = 0;
         for (int i = 0; i < a.groups; i += 512)
-            left += __syncthreads_count(i + tid < a.groups && a.flags[(i + tid) * a.hkv + h] != 0);
+            left += __syncthreads_count(i + tid < a.groups && a.counts[i + tid] < 0);
         if (!BF && 4 * left > a.groups) {
-            if (tid == 0) a.flags[qt * a.hkv + h] = 1;
+            if (tid == 0) set_flag(a.flags + qt * a.hkv + h, kLeft);
             return;
         }
     }
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
             }
             bad |= !(fabsf(l) < INFINITY);
         }
-        if (bad) a.flags[qt * a.hkv + h] = 1;
+        if (bad) set_flag(a.flags + qt * a.hkv + h, kBad);
     } else {
         const int64_t pbase = ((int64_t)h * n_split + sp) * a.PR - a.prow0;
         if (g == 0 && row_ok) a.part_ml[pbase + rho] = float2{m_run, lsum};
@@ -508,7 +520,7 @@ __global__ __launch_bounds__(256) void dlsa_rows_merge_kernel(DlsaRowsArgs a) {
     const int pr = blockIdx.x * 4 + wave, h = blockIdx.y;
     if (pr >= a.PR) return;
     const int row = a.prow0 + pr, grp = row / (a.NR * a.G), fl = grp * a.hkv + h;
-    if (a.flags[fl]) return;  // left to the row kernel
+    if (was_left(a.flags + fl)) return;
     const int64_t base = (int64_t)h * a.n_split * a.PR + pr;
     float M = -INFINITY, l = 0.0f;
     vec o = {};
@@ -547,7 +559,7 @@ __global__ __launch_bounds__(256) void dlsa_rows_merge_kernel(DlsaRowsArgs a) {
         bad |= !(fabsf(y) < INFINITY);
         orow[v_logical_dim(SPL * lane + j, D, 16)] = (ET)y;
     }
-    if (bad) a.flags[fl] = 1;
+    if (bad) set_flag(a.flags + fl, kBad);
 }
 
 // The same in fp32 throughout, for every other pair of types (and D = 32): K and V
@@ -582,7 +594,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows32_kernel(DlsaRowsArgs a) {
             qt = a.qt0 + t / (n_split * a.hkv);
         }
     }
-    if (a.flags[qt * a.hkv + h]) return;  // (uniform, before any barrier)
+    if (a.counts[qt] < 0) return;  // (as above)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -767,7 +779,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows32_kernel(DlsaRowsArgs a) {
         if (g == 0 && row_ok)
             a.part_ml[((int64_t)h * n_split + sp) * a.PR - a.prow0 + rho] = float2{m_run, lsum};
     } else if (bad) {
-        a.flags[qt * a.hkv + h] = 1;
+        set_flag(a.flags + qt * a.hkv + h, kBad);
     }
 }
 
@@ -775,7 +787,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows32_kernel(DlsaRowsArgs a) {
 __global__ void dlsa_rows32_merge_kernel(DlsaRowsArgs a) {
     const int D = blockDim.x, d = threadIdx.x, pr = blockIdx.x, h = blockIdx.y;
     const int row = a.prow0 + pr, fl = row / (a.NR * a.G) * a.hkv + h;
-    if (a.flags[fl]) return;
+    if (was_left(a.flags + fl)) return;
     const int64_t base = (int64_t)h * a.n_split * a.PR + pr;
     float M = -INFINITY, o = 0.0f, l = 0.0f;
     for (int c0 = 0; c0 < a.n_split; c0 += 4) {
@@ -804,7 +816,7 @@ __global__ void dlsa_rows32_merge_kernel(DlsaRowsArgs a) {
         M = m;
     }
     const float y = l > 0.0f ? o / l : 0.0f;
-    if (!(fabsf(y) < INFINITY) || !(fabsf(l) < INFINITY)) a.flags[fl] = 1;
+    if (!(fabsf(y) < INFINITY) || !(fabsf(l) < INFINITY)) set_flag(a.flags + fl, kBad);
     store_as(a.out, a.q_dtype, ((int64_t)(h * a.G + row % a.G) * a.L + row / a.G) * D + d, y);
 }
 

@@ -53,33 +53,41 @@ def _run(q, k, v, lists, lengths, scale, bf16):
     return qw_amd.sparse_attention_typed(*t, _gpu(lists), _gpu(lengths), scale)[0].float().cpu().numpy()
 
 
+def _fp16_takes_it(hq, hkv, D, L, T, W):
+    """The fp16 rule (dlsa_rows_pays), restated."""
+    NR, entries = min(32, 128 // (hq // hkv)) & ~1, L * W * hkv
+    return (L >= 32 and L * hkv > 256 and entries >= 850000 and
+            (T <= int(0.35 * NR * W) - 1500 or entries * D >= 256 * 12000000))
+
+
 CASES = [
-    # hq, hkv, D, L, T, W, kind (fp16 calls take the kernel from 850k entries over all heads)
-    (24, 4, 256, 101, 8000, 2200, "sliding"),   # the last group one row
-    (24, 4, 256, 700, 2000, 320, "shared"),     # the union exactly five tiles
-    (24, 4, 256, 700, 2000, 321, "shared"),     # one key past them
-    (24, 4, 256, 112, 40000, 2000, "own"),      # every group left to the row kernel (fp16)
-    (24, 4, 256, 160, 40000, 1400, "mixed"),
-    (8, 8, 128, 130, 4000, 900, "sliding"),     # G = 1: 32 rows a group
-    (24, 3, 128, 96, 6000, 3000, "sliding"),    # KV heads that do not divide 256
-    (16, 2, 64, 300, 9000, 1500, "sliding"),    # 256-key tiles in two halves
-    (16, 1, 128, 600, 4000, 1500, "shared"),    # G = 16: 8 rows a group
-    (24, 4, 256, 96, 90000, 2300, "sliding"),   # three bitmap passes
-    (24, 4, 256, 1300, 2600, 400, "sliding"),   # whole rounds and a split rest
-    (24, 4, 256, 440, 2000, 512, "shared"),     # eight tiles of lists long enough for fp16
-    (24, 4, 256, 440, 2000, 513, "shared"),
-    (24, 4, 256, 700, 700, 321, "shared"),      # (fp16 takes few rows only where any union pays:
-    (16, 2, 64, 300, 6000, 1500, "sliding"),    # these are fp16's of the kinds above)
-    (16, 1, 128, 600, 2500, 1500, "shared"),
-    (24, 4, 256, 1300, 2600, 800, "sliding"),
+    # hq, hkv, D, L, T, W, kind, whether an fp16 call takes the kernel too
+    (24, 4, 256, 101, 8000, 2200, "sliding", True),   # the last group one row
+    (24, 4, 256, 700, 2000, 320, "shared", False),    # the union exactly five tiles
+    (24, 4, 256, 700, 2000, 321, "shared", False),    # one key past them
+    (24, 4, 256, 112, 40000, 2000, "own", False),
+    (24, 4, 256, 160, 40000, 1400, "mixed", False),
+    (8, 8, 128, 130, 4000, 900, "sliding", True),     # G = 1: 32 rows a group
+    (24, 3, 128, 96, 6000, 3000, "sliding", True),    # KV heads that do not divide 256
+    (16, 2, 64, 300, 9000, 1500, "sliding", False),   # 256-key tiles in two halves
+    (16, 1, 128, 600, 4000, 1500, "shared", False),   # G = 16: 8 rows a group
+    (24, 4, 256, 96, 90000, 2300, "sliding", False),  # three bitmap passes
+    (24, 4, 256, 1300, 2600, 400, "sliding", False),  # whole rounds and a split rest
+    (24, 4, 256, 440, 2000, 512, "shared", True),     # the union exactly eight tiles
+    (24, 4, 256, 440, 2000, 513, "shared", True),
+    (24, 4, 256, 700, 700, 321, "shared", True),
+    (16, 2, 64, 300, 6000, 1500, "sliding", True),
+    (16, 1, 128, 600, 2500, 1500, "shared", True),
+    (24, 4, 256, 1300, 2600, 800, "sliding", True),
 ]
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("hq,hkv,D,L,T,W,kind", CASES)
-def test_rows_match_oracle(hq, hkv, D, L, T, W, kind, bf16):
+@pytest.mark.parametrize("hq,hkv,D,L,T,W,kind,fp16", CASES)
+def test_rows_match_oracle(hq, hkv, D, L, T, W, kind, fp16, bf16):
     print(f"case hq={hq} hkv={hkv} D={D} L={L} T={T} W={W} {kind} bf16={bf16}", flush=True)
-    assert L >= 32 and L * hkv > 256 and L * W * hkv >= 850000, "a shape of the kernel"
+    assert fp16 == _fp16_takes_it(hq, hkv, D, L, T, W), "the route of the fp16 call"
+    assert L * hkv >= 192 and L * W * hkv * D >= 20000 * 256, "a shape of the bf16 call's kernel"
     if bf16 and hq // hkv > 8:
         pytest.skip("the typed read takes at most 8 heads a KV head")
     r = rng(hq + D + L + T + W)
@@ -110,6 +118,68 @@ def test_a_key_listed_twice_counts_twice(bf16):
     lengths = np.full(L, W, np.int32)
     out = _run(q, k, v, lists, lengths, 0.1, bf16)
     _check(out, q, k, v, lists, lengths, 0.1, bf16, "a key twice")
+
+
+def _fp16_inputs(r, hq, hkv, D, L, T):
+    return (r.standard_normal(s).astype(np.float16) for s in ((hq, L, D), (hkv, T, D), (hkv, T, D)))
+
+
+def _check_some(out, q, k, v, lists, lengths, scale, what):
+    """Every 23rd row and the last (the float64 restatement of a whole call would take minutes)."""
+    rows = np.unique(np.append(np.arange(0, len(lists), 23), len(lists) - 1))
+    assert np.isfinite(out).all(), what
+    _check(out[:, rows], q[:, rows], k, v, lists[rows], lengths[rows], scale, False, what)
+
+
+@pytest.mark.parametrize("hq,hkv,D,L,T,W,left", [
+    (24, 4, 256, 1400, 40000, 2200, "all"),     # every union too large: all groups handed over
+    (24, 4, 256, 1400, 40000, 2200, "half"),    # more than a quarter: the others with them
+    (24, 4, 256, 1400, 40000, 2200, "eighth"),  # served in part; a split tail of six groups
+    (24, 4, 256, 1400, 90000, 2200, "none"),    # three bitmap passes
+    (24, 4, 128, 2000, 30000, 3100, "eighth"),
+])
+def test_fp16_rows_over_many_keys(hq, hkv, D, L, T, W, left):
+    assert _fp16_takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
+    r = rng(L + T + D)
+    q, k, v = _fp16_inputs(r, hq, hkv, D, L, T)
+    n = {"all": L, "half": L // 2, "eighth": L // 8, "none": 0}[left]
+    lists = np.concatenate([_lists(r, "own", n, W, T).reshape(n, W) if n else np.zeros((0, W), np.int32),
+                            _lists(r, "sliding", L - n, W, T)] if n < L else [_lists(r, "own", L, W, T)])
+    lists = np.ascontiguousarray(np.roll(lists, L // 3, axis=0))  # away from the groups' start
+    lengths = np.full(L, W, np.int32)
+    out = _run(q, k, v, lists, lengths, D ** -0.5, False)
+    _check_some(out, q, k, v, lists, lengths, D ** -0.5, f"{left} left, T={T}")
+
+
+def test_duplicates_in_a_third_of_the_groups():
+    """More than a quarter of the groups list a key twice, in an fp16 call whose tail is split."""
+    hq, hkv, D, L, T, W = 24, 4, 256, 700, 4000, 800
+    assert _fp16_takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
+    r = rng(12)
+    q, k, v = _fp16_inputs(r, hq, hkv, D, L, T)
+    lists = _lists(r, "sliding", L, W, T)
+    lists[::60, 5] = lists[::60, 4]  # one row of every third group of 20
+    lengths = np.full(L, W, np.int32)
+    _check_some(_run(q, k, v, lists, lengths, 1 / 16, False), q, k, v, lists, lengths, 1 / 16, "duplicates")
+
+
+def test_non_finite_groups_do_not_move_the_others():
+    """Infinite values in the first 30 of 70 groups (their outputs are left to the row kernel): the
+    other groups, later workgroups and a split tail among them, give the clean call's bits."""
+    hq, hkv, D, L, T, W = 24, 4, 256, 1400, 13000, 2200
+    assert _fp16_takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
+    r = rng(13)
+    q, k, v = _fp16_inputs(r, hq, hkv, D, L, T)
+    lists = _lists(r, "sliding", L, W, T - 1)
+    lists[:600, 0] = T - 1
+    lengths = np.full(L, W, np.int32)
+    clean = _run(q, k, v, lists, lengths, 1 / 16, False)
+    _check_some(clean, q, k, v, lists, lengths, 1 / 16, "clean")
+    v[:, T - 1] = np.inf
+    for _ in range(3):
+        out = _run(q, k, v, lists, lengths, 1 / 16, False)
+        assert not np.isfinite(out[:, :600]).any()
+        np.testing.assert_array_equal(out[:, 600:], clean[:, 600:])
 
 
 @pytest.mark.parametrize("bf16", [False, True])
