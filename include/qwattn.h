@@ -24,7 +24,9 @@
  *     (mlx_cxx_dlsa_attention.cpp:429-470); the status codes carry the
  *     same checks.
  *   - Threading: a cache handle is used by one thread at a time, as the
- *     reference's KVCache is !Send/!Sync (cache.rs:483-497).
+ *     reference's KVCache is !Send/!Sync (cache.rs:483-497). Otherwise calls
+ *     may come from any thread; those of several threads on one stream are
+ *     enqueued one after another, each as a whole.
  */
 #ifndef QWATTN_H
 #define QWATTN_H

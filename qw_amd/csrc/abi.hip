@@ -18,8 +18,10 @@ struct qw_kv_cache {
         }                                                                     \
     } while (0)
 
+// (an entry that enqueues on `stream`)
 #define QW_GUARDED(expr)                                                      \
     try {                                                                     \
+        qw::StreamLock on_stream(stream);                                     \
         return (expr);                                                        \
     } catch (const std::bad_alloc&) {                                         \
         qw::set_error("host allocation failed");                              \

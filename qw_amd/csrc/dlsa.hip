@@ -838,7 +838,7 @@ static int dlsa_sparse_attention_impl(const void* q, const DlsaSource& src,
     a.flags = nullptr;
     a.group_rows = 1;
     if (auto_one_pass && !src.cache &&
-        dlsa_rows_pays(n_rows, width, n_kv_heads, n_q_heads / n_kv_heads, head_dim, n_keys)) {
+        dlsa_rows_pays(n_rows, width, n_kv_heads, n_q_heads / n_kv_heads, head_dim, n_keys, stream)) {
         // prefill row counts: neighbouring rows share their keys' gathers; the
         // kernel below then serves the groups that this one leaves
         const int rc = dlsa_rows_attention(q, QW_DTYPE_F16, src.k, src.v, QW_DTYPE_F16, src.khs,

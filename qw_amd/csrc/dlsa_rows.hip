@@ -885,7 +885,8 @@ int dlsa_rows_per_group(int G) { return std::min(32, 128 / G) & ~1; }
 // 1200 -> 1239 us; D = 256, 140 rows 416 -> 452, 400 853 -> 889, 1500 2646 -> 2506 us), and
 // nothing on the host tells them from rows that share (450 -> 196 us at 400): such a call
 // is taken from 12M entries of 256 dims over the heads, where that loss is at most 3 %.
-bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys) {
+bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys, hipStream_t stream) {
+    if (stream == hipStreamPerThread) return false;  // (one handle, a stream a thread)
     const int64_t entries = (int64_t)n_rows * width * n_kv_heads;
     if (n_rows < 32 || n_rows * (int64_t)n_kv_heads <= 256 || entries < 850000) return false;
     return n_keys <= union_limit(width, dlsa_rows_per_group(G), false) || entries * D >= (int64_t)256 * 12000000;

@@ -333,7 +333,8 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     const int64_t per16 = 16 / (int64_t)es;
     const bool aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 &&
                          khs % per16 == 0 && krs % per16 == 0 && vhs % per16 == 0 && vrs % per16 == 0;
-    if (auto_one_pass && aligned && (int64_t)n_rows * width * n_kv_heads * head_dim >= 20000 * 256) {
+    if (auto_one_pass && aligned && stream != hipStreamPerThread &&
+        (int64_t)n_rows * width * n_kv_heads * head_dim >= 20000 * 256) {
         const int rc = dlsa_rows_attention(q, q_dtype, k, v, kv_dtype, khs, krs, vhs, vrs, lists,
                                            lengths, n_rows, width, n_q_heads, n_kv_heads, head_dim,
                                            n_keys, scale, out, &a.flags, stream);

@@ -74,6 +74,12 @@ void GrowBuffer::release() {
     captured = false;
 }
 
+static std::mutex& stream_mutex(const void* stream) {
+    static std::mutex mu[64];
+    return mu[((uint64_t)(uintptr_t)stream * 0x9E3779B97F4A7C15ull) >> 58];
+}
+StreamLock::StreamLock(const void* stream) : lock(stream_mutex(stream)) {}
+
 // Dynamic-LDS limits already raised, per (kernel, device). The attribute is
 // a property of the kernel on the current device, so it is recorded per
 // device, and the mutex keeps two host threads from interleaving a check and

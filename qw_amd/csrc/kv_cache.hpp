@@ -249,7 +249,7 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
 // QW_ERR_STATE / QW_ERR_OUT_OF_MEMORY, with nothing enqueued, without a workspace.
 int dlsa_rows_per_group(int G);
 // Whether a one-pass fp16 call takes it (the rule and both sides in dlsa_rows.hip).
-bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys);
+bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys, hipStream_t stream);
 int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v, int kv_dtype,
                         int64_t k_head_stride, int64_t k_row_stride, int64_t v_head_stride, int64_t v_row_stride,
                         const int32_t* lists, const int32_t* lengths, int n_rows, int width,

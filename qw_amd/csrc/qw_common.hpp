@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -218,6 +219,19 @@ struct GrowBuffer {
     std::vector<void*> retired;
     int get(size_t need, hipStream_t stream, void** out);
     void release();
+};
+
+// Held while a call enqueues on `stream`: the per-(device, stream) workspaces are
+// written by one launch of a call and read by the next, and may be replaced when they
+// grow, so calls of several host threads on one stream go one after another as wholes.
+// (A fixed set of locks, by the stream's handle: two streams may share one and then
+// only wait for each other's enqueueing.)
+class StreamLock {
+  public:
+    explicit StreamLock(const void* stream);
+
+  private:
+    std::lock_guard<std::mutex> lock;
 };
 
 // Raises `kernel`'s dynamic-LDS limit on the current device to at least

@@ -334,8 +334,9 @@ int gen_kv_workspace(int device, hipStream_t stream, size_t need, void** out) {
 // us over 300 keys and 52.7 -> 38.4 us over 1k. A mask is read a byte or two a
 // lane here and in 8-key pieces there, so a masked call's line lies lower: 78 rows
 // over 8k keys 49 -> 33 us with the layout and the merge.
-bool rows_route(int R, int n_keys, int hkv, int D, bool mask, const void* out) {
+bool rows_route(int R, int n_keys, int hkv, int D, bool mask, const void* out, hipStream_t stream) {
     if ((uintptr_t)out % 8 != 0) return false;  // (it writes 8-byte pieces)
+    if (stream == hipStreamPerThread) return false;  // (one handle, a stream a thread)
     // images of more than 4 GiB are not kept (1.03 KB a key and head at D = 256)
     if ((int64_t)n_keys * hkv * D * 2 * sizeof(f16) > (int64_t)4 << 30) return false;
     return mask ? R > 16 && (int64_t)R * n_keys >= 500000 : (int64_t)(R - 100) * n_keys >= 1300000;
@@ -379,7 +380,7 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
     QW_REQUIRE(!o.mask || (o.mask_head_stride >= 0 && o.mask_row_stride >= 0),
                QW_ERR_INVALID_ARGUMENT, "sdpa: negative mask stride");
     const int G = n_q_heads / n_kv_heads, R = G * n_rows, D = head_dim;
-    if (rows_route(R, n_keys, n_kv_heads, D, o.mask != nullptr, out)) {
+    if (rows_route(R, n_keys, n_kv_heads, D, o.mask != nullptr, out, stream)) {
         const int rc = rows_attention(q, G, n_rows, k, v, n_kv_heads, n_keys, D, khs, krs, vhs, vrs,
                                       scale, o, out, stream);
         // without room for the images (under capture, or no memory left) the
