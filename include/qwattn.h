@@ -12,7 +12,15 @@
  *     library sets that device for the duration of a call.
  *   - `stream` is a hipStream_t passed as void* (NULL = the default stream).
  *     All device work of a call is enqueued on it; no call synchronizes the
- *     stream except where stated.
+ *     stream except where stated, and where a workspace has to grow (the
+ *     first call of a larger shape on that stream).
+ *   - Workspaces (split-K partials, tile images, key unions) belong to a
+ *     (device, stream), are kept for its next call and never shared between
+ *     streams; qw_release_workspaces frees them. The largest are tile images:
+ *     1.03 times the fp16 K and V of the keys that a long prefill call sees,
+ *     at most 4 GiB for qw_sdpa. A graph reads the workspaces of the stream
+ *     that it was captured on: replay it where no other call of that stream,
+ *     nor another graph from it, runs at the same time.
  *   - Tensors use the reference's layouts with the batch dimension of 1
  *     dropped: q [n_q_heads][n_rows][head_dim], new K/V
  *     [n_kv_heads][n_tokens][head_dim], attention output like q. Element
@@ -79,6 +87,11 @@ int qw_abi_version(void);
 
 /* Message of the last failing call on this thread ("" if none). */
 const char* qw_last_error(void);
+
+/* Waits for `stream` and frees the workspaces kept for it on the current
+ * device, but for those that a captured graph may still read; the next call
+ * that needs one makes it again. QW_ERR_STATE while the stream is captured. */
+int qw_release_workspaces(void* stream);
 
 /* ---------------------------------------------------------------- cache */
 

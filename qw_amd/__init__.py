@@ -31,7 +31,7 @@ __all__ = ["KVCacheMode", "KVCache", "QwError", "attention", "causal_attention",
            "sparse_attention", "sparse_attention_with",
            "fused_rope_qk_append", "dlsa_select", "dlsa_select_with", "turbo4_codebook",
            "turbo4_signs",
-           "lib", "LIB_PATH"]
+           "release_workspaces", "lib", "LIB_PATH"]
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libqwattn.so")
 _lib = None
@@ -63,6 +63,7 @@ _SIGNATURES = {
     "qw_kv_import_turbo4": (_i, [_p, _i, _p, _p, _p, _p, _p, _p]),
     "qw_turbo4_codebook": (_i, [_i, _i, _p]),
     "qw_turbo4_signs": (_i, [_i, ctypes.c_uint32, _p]),
+    "qw_release_workspaces": (_i, [_p]),
     "qw_kv_destroy": (_i, [_p]),
     "qw_kv_reserve": (_i, [_p, _i, _p]),
     "qw_kv_offset": (_i, [_p, ctypes.POINTER(_i)]),
@@ -183,6 +184,15 @@ def _rows2(qkv, what: str):
 def _out_like(t, H: int, L: int, D: int):
     """An output [1, H, L, D] of t's type on t's device."""
     return t.new_empty((1, H, L, D))
+
+
+def release_workspaces(device=None) -> None:
+    """Waits for the current stream and frees the workspaces that calls on it left there
+    (partials, tile images, key unions), but for those a captured graph may read."""
+    torch = _torch()
+    dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
+    with torch.cuda.device(dev):
+        _check(lib().qw_release_workspaces(_stream(dev)))
 
 
 class KVCacheMode:

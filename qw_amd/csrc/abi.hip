@@ -182,6 +182,10 @@ static int update_and_general(qw::KVCache& c, const void* q, int n_q_heads, int 
     return qw::cache_attention_general(c, q, n_q_heads, n_rows, scale, o, out, stream);
 }
 
+int qw_release_workspaces(void* stream) {
+    QW_GUARDED(qw::release_workspaces((hipStream_t)stream));
+}
+
 int qw_sdpa(const void* q, int n_q_heads, int n_rows, const void* k, const void* v,
             int n_kv_heads, int n_keys, int head_dim, int64_t k_head_stride, int64_t k_row_stride,
             int64_t v_head_stride, int64_t v_row_stride, float scale, int causal, int window,

@@ -33,8 +33,6 @@
 //   partials (fp32 m and l, the row O / l in fp16; the fused Turbo4 pass
 //   keeps O in fp32) and a split-K merge kernel.
 #include <algorithm>
-#include <map>
-#include <mutex>
 #include <type_traits>
 
 #include "append.hpp"
@@ -1377,17 +1375,6 @@ constexpr int kImageMinRows = 3072;
 // at about the images' cost.
 constexpr int kT4ImageMinRows = 1025;
 
-static std::mutex g_img_mu;
-static std::map<std::pair<int, hipStream_t>, GrowBuffer> g_img_ws;
-// The tile images' buffer, one per (device, stream) like the other
-// transient workspaces (stream-ordered reuse; capture-safe growth).
-int image_workspace(int device, hipStream_t stream, size_t need, void** out) {
-    std::lock_guard<std::mutex> lock(g_img_mu);
-    GrowBuffer& b = g_img_ws[{device, stream}];
-    b.stream_owned = true;  // only calls on `stream` use it
-    return b.get(need, stream, out);
-}
-
 // Splits `n_tiles` key tiles into about `want` parts of at least min_tiles
 // tiles (4: a workgroup's fixed costs amortized over its rounds; a window's
 // few tiles spread wider).
@@ -1464,7 +1451,7 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     if constexpr (T4M != 2) {
         if (images) {
             void* img = nullptr;
-            rc = image_workspace(cc.device, stream, (size_t)cc.hkv * n_tiles * S::BUF, &img);
+            rc = workspace(kWsImages, cc.device, stream, (size_t)cc.hkv * n_tiles * S::BUF, &img);
             if (rc) return rc;
             a.img_w = (char*)img;
             a.img = (const char*)img;

@@ -490,7 +490,7 @@ int rows_attention_d(const void* q, int G, int n_rows, const void* k, const void
     int dev = 0;
     QW_HIP_CHECK(hipGetDevice(&dev));
     void* ws = nullptr;
-    if (int rc = image_workspace(dev, stream, img_bytes + n_part * (D * sizeof(float) + sizeof(float2)), &ws))
+    if (int rc = workspace(kWsImages, dev, stream, img_bytes + n_part * (D * sizeof(float) + sizeof(float2)), &ws))
         return rc;
     a.q = (const f16*)q;
     a.out = (f16*)out;

@@ -683,19 +683,6 @@ __global__ __launch_bounds__(64 * kDMW) void dlsa_merge_kernel(const float* __re
     }
 }
 
-// Split-K workspace of the D-LSA calls, one per (device, stream): calls on
-// different streams never share partials. Each is a GrowBuffer, so growth
-// never frees memory a captured graph may still read.
-static std::mutex g_ws_mu;
-static std::map<std::pair<int, hipStream_t>, GrowBuffer> g_ws;
-
-static int dlsa_workspace(int device, hipStream_t stream, size_t need, void** out) {
-    std::lock_guard<std::mutex> lock(g_ws_mu);
-    GrowBuffer& b = g_ws[{device, stream}];
-    b.stream_owned = true;  // only calls on `stream` use it
-    return b.get(need, stream, out);
-}
-
 // Launch policy (the reference's auto_parts, mlx_cxx_dlsa_attention.cpp:379-400,
 // re-derived for 256 CUs): one pass when rows x kv_heads alone reach 192
 // workgroups, else split each list so that about 192 workgroups run (3/4 of
@@ -855,8 +842,7 @@ static int dlsa_sparse_attention_impl(const void* q, const DlsaSource& src,
         const size_t no = (size_t)n_rows * n_q_heads * parts;
         void* ws = scratch;
         if (!ws) {
-            int rc = dlsa_workspace(dev, stream, no * head_dim * sizeof(float) + no * sizeof(float2),
-                                    &ws);
+            int rc = workspace(kWsDlsa, dev, stream, no * head_dim * sizeof(float) + no * sizeof(float2), &ws);
             if (rc) return rc;
         }
         a.part_o = (float*)ws;

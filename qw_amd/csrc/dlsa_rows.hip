@@ -33,8 +33,6 @@
 // infinite or NaN: a key's V reaches every row of its group here with weight 0,
 // and 0 x inf is NaN.
 #include <algorithm>
-#include <map>
-#include <mutex>
 
 #include "block_tile.hpp"
 #include "kv_cache.hpp"
@@ -820,9 +818,6 @@ __global__ void dlsa_rows32_merge_kernel(DlsaRowsArgs a) {
     store_as(a.out, a.q_dtype, ((int64_t)(h * a.G + row % a.G) * a.L + row / a.G) * D + d, y);
 }
 
-std::mutex g_plan_mu;
-std::map<std::pair<int, hipStream_t>, GrowBuffer> g_plan_ws;
-
 template <int D, bool BF>
 int launch_rows(const DlsaRowsArgs& a, int grid, hipStream_t stream) {
     const size_t shmem = 2 * BlockShape<D>::BUF + 2 * BlockShape<D>::KT * sizeof(uint32_t);
@@ -925,13 +920,9 @@ int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v
     int dev = 0;
     QW_HIP_CHECK(hipGetDevice(&dev));
     void* ws = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(g_plan_mu);
-        GrowBuffer& b = g_plan_ws[{dev, stream}];
-        b.stream_owned = true;
-        if (int rc = b.get(part_bytes + 2 * list_bytes + count_bytes + (size_t)units * sizeof(int), stream, &ws))
-            return rc;
-    }
+    if (int rc = workspace(kWsUnions, dev, stream,
+                           part_bytes + 2 * list_bytes + count_bytes + (size_t)units * sizeof(int), &ws))
+        return rc;
     char* p = (char*)ws;
     a.part_o = (float*)p;
     a.part_ml = (float2*)(p + n_part * D * sizeof(float));

@@ -24,8 +24,6 @@
 // workgroup takes a contiguous share of the list and writes an fp32 partial
 // (m, l, unnormalized O); a merge kernel combines the parts.
 #include <algorithm>
-#include <map>
-#include <mutex>
 #include <string>
 
 #include "kv_cache.hpp"
@@ -248,10 +246,6 @@ static void launch_typed_dq(const TypedArgs& a, int kv_dtype, int D, dim3 grid, 
         launch_typed_dq_dkv<DQ, QW_DTYPE_F32>(a, D, grid, nw, stream);
 }
 
-// Split-K workspace of the typed calls, one per (device, stream).
-static std::mutex g_typed_mu;
-static std::map<std::pair<int, hipStream_t>, GrowBuffer> g_typed_ws;
-
 size_t dtype_size(int dt) { return dt == QW_DTYPE_F32 ? 4 : 2; }
 
 }  // namespace
@@ -348,13 +342,8 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     if (parts > 1) {
         const size_t no = (size_t)parts * n_rows * n_q_heads;
         void* ws = nullptr;
-        {
-            std::lock_guard<std::mutex> lock(g_typed_mu);
-            GrowBuffer& b = g_typed_ws[{dev, stream}];
-            b.stream_owned = true;
-            int rc = b.get(no * head_dim * sizeof(float) + no * sizeof(float2), stream, &ws);
-            if (rc) return rc;
-        }
+        if (int rc = workspace(kWsTyped, dev, stream, no * head_dim * sizeof(float) + no * sizeof(float2), &ws))
+            return rc;
         a.part_o = (float*)ws;
         a.part_ml = (float2*)((char*)ws + no * head_dim * sizeof(float));
     }

@@ -15,6 +15,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <tuple>
 
 #include "kv_cache.hpp"
 #include "append.hpp"
@@ -72,6 +73,43 @@ void GrowBuffer::release() {
     ptr = nullptr;
     bytes = 0;
     captured = false;
+}
+
+// (nodes stay where they are: the map's lock covers the lookup alone, a buffer is its
+// stream's, which the caller holds, and growth waits for that stream only)
+static std::mutex g_ws_mu;
+static std::map<std::tuple<int, hipStream_t, int>, GrowBuffer> g_ws;
+
+int workspace(Workspace kind, int device, hipStream_t stream, size_t need, void** out) {
+    GrowBuffer* b;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        b = &g_ws[{device, stream, kind}];
+    }
+    b->stream_owned = true;
+    return b->get(need, stream, out);
+}
+
+int release_workspaces(hipStream_t stream) {
+    int dev = 0;
+    QW_HIP_CHECK(hipGetDevice(&dev));
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    QW_HIP_CHECK(hipStreamIsCapturing(stream, &cs));
+    QW_REQUIRE(cs == hipStreamCaptureStatusNone, QW_ERR_STATE,
+               "release_workspaces: the stream is being captured");
+    QW_HIP_CHECK(hipStreamSynchronize(stream));
+    std::vector<GrowBuffer> freed;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        for (int kind = 0; kind < kWorkspaces; kind++) {
+            auto it = g_ws.find({dev, stream, kind});
+            if (it == g_ws.end() || it->second.captured || !it->second.retired.empty()) continue;
+            freed.push_back(it->second);
+            g_ws.erase(it);
+        }
+    }
+    for (GrowBuffer& b : freed) b.release();
+    return QW_OK;
 }
 
 static std::mutex& stream_mutex(const void* stream) {

@@ -315,9 +315,6 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
 int rows_attention(const void* q, int G, int n_rows, const void* k, const void* v, int hkv,
                    int n_keys, int head_dim, int64_t khs, int64_t krs, int64_t vhs, int64_t vrs,
                    float scale, const SdpaOptions& o, void* out, hipStream_t stream);
-// The tile images' workspace of a (device, stream), shared by the launches
-// that attend from images (attend_block.hip).
-int image_workspace(int device, hipStream_t stream, size_t need, void** out);
 // The first key any of n_rows causal windowed rows over T keys sees (0 without
 // a window), rounded down to a multiple of align; and the options of a call on
 // keys lo .. n_keys - 1 only (the mask's columns shifted by lo).

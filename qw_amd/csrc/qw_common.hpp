@@ -221,6 +221,24 @@ struct GrowBuffer {
     void release();
 };
 
+// The workspaces of a (device, stream): calls on one stream follow each other there,
+// calls on different streams share nothing. They are kept for the stream's next call,
+// until release_workspaces.
+enum Workspace {
+    kWsImages,   // tile images (attend_block.hip, attend_rows.hip)
+    kWsUnions,   // key unions of row groups and their partials (dlsa_rows.hip)
+    kWsSdpa,     // split-K partials of sdpa_general.hip
+    kWsSdpaKv,   // a cache's dequantized rows for it
+    kWsTurbo4,   // a Turbo4 attention's rotated rows and partials
+    kWsDlsa,     // split-K partials of the D-LSA read
+    kWsTyped,    // and of the typed one
+    kWorkspaces
+};
+int workspace(Workspace kind, int device, hipStream_t stream, size_t need, void** out);
+// Waits for the stream and frees its workspaces on the current device, but for those
+// that a captured graph may read.
+int release_workspaces(hipStream_t stream);
+
 // Held while a call enqueues on `stream`: the per-(device, stream) workspaces are
 // written by one launch of a call and read by the next, and may be replaced when they
 // grow, so calls of several host threads on one stream go one after another as wholes.

@@ -39,8 +39,6 @@
 // splits write fp32 partials (m, l, O) for the shared merge kernel.
 #include <algorithm>
 #include <cmath>
-#include <map>
-#include <mutex>
 #include <string>
 
 #include "kv_cache.hpp"
@@ -303,28 +301,6 @@ void launch_general(const GenArgs& a, int nwv, dim3 grid, hipStream_t stream) {
         launch_general<D, 4>(a, grid, stream);
 }
 
-// Split-K partials, one workspace per (device, stream).
-std::mutex g_gen_mu;
-std::map<std::pair<int, hipStream_t>, GrowBuffer> g_gen_ws;
-
-int gen_workspace(int device, hipStream_t stream, size_t need, void** out) {
-    std::lock_guard<std::mutex> lock(g_gen_mu);
-    GrowBuffer& b = g_gen_ws[{device, stream}];
-    b.stream_owned = true;
-    return b.get(need, stream, out);
-}
-
-// The dequantized rows of a cache for the general route, one per (device,
-// stream).
-std::map<std::pair<int, hipStream_t>, GrowBuffer> g_gen_kv;
-
-int gen_kv_workspace(int device, hipStream_t stream, size_t need, void** out) {
-    std::lock_guard<std::mutex> lock(g_gen_mu);
-    GrowBuffer& b = g_gen_kv[{device, stream}];
-    b.stream_owned = true;
-    return b.get(need, stream, out);
-}
-
 // Whether a call takes the row kernel (attend_rows.hip), which lays every key
 // tile out once and then runs at several times this kernel's rate: 1536 rows
 // over 9728 keys (24 heads over 4, D = 256) 1943 -> 372 us. The layout and two
@@ -427,7 +403,7 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
     if (ns > 1) {
         const size_t no = (size_t)n_kv_heads * ns * R;
         void* ws = nullptr;
-        if (int rc = gen_workspace(dev, stream, no * D * sizeof(float) + no * sizeof(float2), &ws))
+        if (int rc = workspace(kWsSdpa, dev, stream, no * D * sizeof(float) + no * sizeof(float2), &ws))
             return rc;
         a.part_o = (float*)ws;
         a.part_ml = (float2*)((char*)ws + no * D * sizeof(float));
@@ -513,7 +489,7 @@ int cache_attention_general(KVCache& c, const void* q, int n_q_heads, int n_rows
     const int n = T - lo;
     const size_t bytes = (size_t)c.hkv * n * D * sizeof(f16);
     void* ws = nullptr;
-    if (int rc = gen_kv_workspace(c.device, stream, 2 * bytes, &ws)) return rc;
+    if (int rc = workspace(kWsSdpaKv, c.device, stream, 2 * bytes, &ws)) return rc;
     char* kw = (char*)ws;
     char* vw = kw + bytes;
     if (int rc = c.dequantize(lo, n, kw, vw, stream)) return rc;  // [hkv][n][D] rows

@@ -25,8 +25,6 @@
 #include <math.h>
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 #include <string>
 
 #include <utility>
@@ -605,20 +603,11 @@ static unsigned grid_for(int64_t work) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>((work + 255) / 256, 4096));
 }
 
-// Workspace of the attention routes (the rotated fp16 K/V, q, the fp32
-// merged rows and split partials), one per (device, stream), shared by the
-// Turbo4 caches that attend on that stream as MLX's allocator shares its
-// transient buffers: calls on one stream are ordered by the stream, calls on
-// different streams never share it. A GrowBuffer, so a call captured in a HIP
-// graph keeps its buffer when a later call grows the workspace.
-std::mutex g_t4_mu;
-std::map<std::pair<int, hipStream_t>, GrowBuffer> g_t4_ws;
-
+// The attention routes' workspace (the rotated fp16 K/V, q, the fp32 merged rows and
+// split partials), shared by the Turbo4 caches that attend on a stream as MLX's
+// allocator shares its transient buffers.
 int t4_workspace(int device, hipStream_t stream, size_t need, void** out) {
-    std::lock_guard<std::mutex> lock(g_t4_mu);
-    GrowBuffer& b = g_t4_ws[{device, stream}];
-    b.stream_owned = true;  // only calls on `stream` use it
-    return b.get(need, stream, out);
+    return workspace(kWsTurbo4, device, stream, need, out);
 }
 
 }  // namespace

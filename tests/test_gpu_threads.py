@@ -1,6 +1,6 @@
 """Calls of several host threads, and on several streams, that share or own the per-stream
 workspaces (tile images, key unions and their partials): every result equals the same call made
-alone, bit for bit, also where a workspace grows in between."""
+alone, bit for bit, also where a workspace grows or is given back in between."""
 import threading
 
 import numpy as np
@@ -109,3 +109,48 @@ def test_two_streams_from_one_thread():
                     outs.append((i, c()))
     torch.cuda.synchronize()
     assert all(torch.equal(g, alone[i]) for i, g in outs)
+
+
+def test_workspaces_are_given_back():
+    import qw_amd
+
+    calls = [_dense(1, 128, 2500), _sparse(4, 128, 3000, 1700, torch.float16), _dense(8, 64, 60000)]
+    alone = [c() for c in calls]
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(2):
+            before = torch.cuda.mem_get_info()[0]
+            outs = [c() for c in calls]
+            stream.synchronize()
+            used = before - torch.cuda.mem_get_info()[0]
+            qw_amd.release_workspaces()
+            assert used >= 60000 * 4 * 1024, used  # the last call's images, at least
+            assert torch.cuda.mem_get_info()[0] >= before - (32 << 20)  # (torch's own blocks for the outputs)
+            assert all(torch.equal(a, b) for a, b in zip(outs, alone))
+
+
+def test_release_keeps_what_a_graph_reads():
+    import qw_amd
+
+    call = _dense(1, 128, 2500)
+    want = call()
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        call()
+        stream.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            out = call()
+        qw_amd.release_workspaces()
+        big = _dense(9, 64, 60000)()  # grows the stream's buffer: the graph keeps its own
+        qw_amd.release_workspaces()
+        for _ in range(3):
+            out.zero_()
+            g.replay()
+            stream.synchronize()
+            assert torch.equal(out, want)
+            del big
+            big = torch.full((64 << 20,), 7, dtype=torch.uint8, device="cuda")  # whatever was freed is written
+    torch.cuda.synchronize()
