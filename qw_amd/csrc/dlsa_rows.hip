@@ -19,13 +19,15 @@
 //     layout of block_tile.hpp, and for each score the key's bit of its row;
 //   dlsa_rows_merge_kernel sums the fp32 partials of the groups whose keys were
 //     split (the last, partial round of workgroups).
-// P enters P.V as a high part plus a remainder in the element type, as in
-// dlsa.hip (fp16; 16 bits of P in bf16, far below the output's 8).
-// What bounds it: MFMAs and LDS operand reads, as in attend_rows.hip, with three
-// MFMAs a (key, column, dim) where that kernel has two. Measured (24 heads over 4,
+// P enters P.V as a high part plus a remainder in fp16, as in dlsa.hip, and in three
+// parts in bf16, which hold the 24 bits of the fp32 P of dlsa_typed.hip (two hold 16:
+// 512 rows at 16k 156 for 175 us, and an error against 64 bits of 1.655198e-3 for
+// 1.655196e-3 here and there).
+// What bounds it: MFMAs and LDS operand reads, as in attend_rows.hip, with three (bf16
+// four) MFMAs a (key, column, dim) where that kernel has two. Measured (24 heads over 4,
 // D = 256, lists of 4 sinks, a 512-key window and 8 shared 512-key blocks): 1536 rows
 // at 32k in fp16 1312 us by row pairs -> 347 us here (502 TFLOP/s; the plan 26 us, the
-// merge 6 us of it), 512 rows at 16k in bf16 7572 -> 157 us; in f32 7530 -> 744 us.
+// merge 6 us of it), 512 rows at 16k in bf16 7572 -> 175 us; in f32 7530 -> 744 us.
 //
 // A group is left to the row-by-row kernels, launched behind with the flags of
 // this one, where (a) a row lists a key twice (it counts twice), (b) the union is
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
             m_run = m_new;
         }
         const float mref = m_run == -INFINITY ? 0.0f : m_run;
-        V8 ph[NU], pl[NU];
+        V8 ph[NU], pl[NU], pm[BF ? NU : 1];
 #pragma unroll
         for (int u = 0; u < NU; u++)
 #pragma unroll
@@ -423,7 +425,9 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
                 const float p = __builtin_amdgcn_exp2f(sf[u][e] - mref);
                 l_run += p;
                 ph[u][e] = (ET)p;
-                pl[u][e] = (ET)(p - (float)ph[u][e]);
+                const float rest = p - (float)ph[u][e];
+                pl[u][e] = (ET)rest;
+                if constexpr (BF) pm[u][e] = (ET)(rest - (float)pl[u][e]);
             }
 #pragma unroll
         for (int u = 0; u < NU; u++) {
@@ -433,17 +437,18 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
                 const V8 vv = vb8[17 * mm];
                 acc_o[mm] = E::mfma(ph[u], vv, acc_o[mm]);
                 acc_o[mm] = E::mfma(pl[u], vv, acc_o[mm]);
+                if constexpr (BF) acc_o[mm] = E::mfma(pm[u], vv, acc_o[mm]);
             }
         }
         {
-            constexpr int NQ = NU * NT, AH = 4;
+            constexpr int NQ = NU * NT, AH = 4, MF = BF ? 3 : 2;
             __builtin_amdgcn_sched_group_barrier(0x100, AH, 1);
 #pragma unroll
             for (int i = 0; i < NQ - AH; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
+                __builtin_amdgcn_sched_group_barrier(0x008, MF, 1);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 2 * AH, 1);
+            __builtin_amdgcn_sched_group_barrier(0x008, MF * AH, 1);
         }
     };
 

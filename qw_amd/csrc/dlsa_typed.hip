@@ -322,7 +322,7 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     // (dlsa_rows.hip), and the kernel here serves the groups which that leaves (or
     // every row, without room for its lists). From 20k entries over all heads at
     // D = 256 (as many bytes at others): 512 rows of 4612 entries (24 heads over 4, D =
-    // 256) in bf16 7572 -> 157 us, in f32 7530 -> 744 us; 48 rows of 128 in bf16 79 ->
+    // 256) in bf16 7572 -> 175 us, in f32 7530 -> 744 us; 48 rows of 128 in bf16 79 ->
     // 38 us, in f32 78 -> 61 us.
     const int64_t per16 = 16 / (int64_t)es;
     const bool aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 &&

@@ -237,3 +237,30 @@ def test_typed_rows_match_float64(qt, kt, hq, hkv, D, L, T, W, kind):
     ref = oracle.dlsa_attention_f64(q, k, v, lists, lengths, D ** -0.5)
     bound = np.abs(ref) * ROUND[qt] + 1e-5 * np.linalg.norm(ref, axis=-1, keepdims=True) + 1e-7
     assert np.isfinite(out).all() and np.all(np.abs(out.astype(np.float64) - ref) <= bound)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_bf16_weights_keep_32_bits(D):
+    """Two keys whose scores differ by 2^-13, of opposite values, and a third of value 0 above them:
+    what is left is the difference of two weights of about 0.7, some 3e-5, and weights held in 16
+    bits (2^-18 of them each) are up to 2e-6 off. Bound: the output's rounding, half a unit of 2^-8
+    relative, and 3e-7 for 32-bit scores, exponentials and sums (five roundings of 2^-24)."""
+    import qw_amd
+
+    hq, hkv, L, T, W = 24, 4, 64, 2000, 400
+    assert L * hkv >= 192 and L * W * hkv * D >= 20000 * 256, "a shape of the kernel"
+    f = lambda x: torch.from_numpy(x).to(torch.bfloat16)  # noqa: E731
+    q = np.zeros((hq, L, D), np.float32)
+    q[:, :, 0], q[:, :, 1] = np.linspace(0.25, 1.0, L), 2.0 ** -6
+    k, v = np.zeros((2, hkv, T, D), np.float32)
+    k[:, :, 0] = -16384
+    k[:, 2, 0], k[:, 5, 0], k[:, 9, 0], k[:, 9, 1] = 3, 1, 1, -2.0 ** -5
+    v[:, 5], v[:, 9] = 1, -1
+    q, k, v = f(q), f(k), f(v)
+    lists = np.tile(np.arange(W, dtype=np.int32), (L, 1))
+    lengths = np.full(L, W, np.int32)
+    out = qw_amd.sparse_attention_typed(q.cuda(), k.cuda(), v.cuda(), _gpu(lists), _gpu(lengths), 0.25)[0]
+    s = 0.25 * (q[:, :, 0].double().numpy()[..., None] * np.array([3, 1, 1]) - np.array([0, 0, 2.0 ** -11]))
+    w = np.exp(s - s[..., :1])
+    ref = ((w[..., 1] - w[..., 2]) / w.sum(axis=-1))[..., None]
+    assert np.all(np.abs(out.double().cpu().numpy() - ref) <= np.abs(ref) * 2.0 ** -8 + 3e-7)
