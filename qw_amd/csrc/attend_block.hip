@@ -813,12 +813,11 @@ __device__ __forceinline__ void block_body(const BlockArgs& a, char* lds) {
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
                 float sf[NU][8];
-                a.softcap.apply([&](auto f) {
 #pragma unroll
-                    for (int u = 0; u < NU; u++)
+                for (int u = 0; u < NU; u++)
 #pragma unroll
-                        for (int e = 0; e < 8; e++) sf[u][e] = f((float)(f16)acc[u][e >> 2][rt][e & 3]);
-                });
+                    for (int e = 0; e < 8; e++) sf[u][e] = (float)(f16)acc[u][e >> 2][rt][e & 3];
+                a.softcap.apply(sf);
                 if (mask) {
 #pragma unroll
                     for (int u = 0; u < NU; u++)

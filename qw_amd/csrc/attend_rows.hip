@@ -221,12 +221,11 @@ __global__ __launch_bounds__(64 * NW, 1) void rows_attend_kernel(RowsArgs a) {
         half2v sh[CAP ? 1 : NU][4];
         float sf[CAP ? NU : 1][8];
         if constexpr (CAP) {
-            a.softcap.apply([&](auto f) {
 #pragma unroll
-                for (int u = 0; u < NU; u++)
+            for (int u = 0; u < NU; u++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++) sf[u][e] = f((float)(f16)acc[u][e >> 2][e & 3]);
-            });
+                for (int e = 0; e < 8; e++) sf[u][e] = (float)(f16)acc[u][e >> 2][e & 3];
+            a.softcap.apply(sf);
         } else {
 #pragma unroll
             for (int u = 0; u < NU; u++)

@@ -192,13 +192,13 @@ __global__ __launch_bounds__(64 * NWV) void sdpa_general_kernel(GenArgs a) {
         float sv[NU][4];
         float tmax = -INFINITY;
         float capped[SOFTCAP ? NU : 1][4];
-        if constexpr (SOFTCAP)
-            a.softcap.apply([&](auto f) {
+        if constexpr (SOFTCAP) {
 #pragma unroll
-                for (int u = 0; u < NU; u++)
+            for (int u = 0; u < NU; u++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) capped[u][i] = f((float)(f16)s4[u][i]);
-            });
+                for (int i = 0; i < 4; i++) capped[u][i] = (float)(f16)s4[u][i];
+            a.softcap.apply(capped);
+        }
 #pragma unroll
         for (int u = 0; u < NU; u++)
 #pragma unroll

@@ -425,3 +425,40 @@ def test_sdpa_against_torch_fp32(causal, window, softcap, mkind):
     print(f"torch fp32 {mkind} sc={softcap} w={window}: max_abs={err.max():.3e} rel_l2={rel:.3e}",
           flush=True)
     assert err.max() < 5e-3 and rel < 3e-3
+
+
+@pytest.mark.parametrize("cap", [5.0, 50.0, 100.0, 300.0])
+@pytest.mark.parametrize("route", ["few rows", "many rows", "cache"])
+def test_softcap_keeps_small_scores(route, cap):
+    """Scores far below the cap keep their 24 bits: two keys of opposite value, one of score s and
+    one of score 0, give tanh(s / 2), s = tanh(S scale / cap) cap. Bound: the output's rounding
+    (2^-11 relative, 2^-25 below fp16's normal range), 2 2^-23 relative for s, and 3e-7 for weights
+    near 1 in two fp16 parts (2^-22), the exponentials and sums (2^-23). An error of 1.5e-7 of the
+    cap in s, as of a difference of two numbers near it, is 8e-6 at a cap of 100."""
+    import qw_amd
+
+    hq, hkv, D, scale = 24, 4, 256, 0.1
+    L, T = (300, 1000) if route == "many rows" else (4, 300)
+    assert (6 * L - 100) * T >= 1300000 or route != "many rows", "a shape of the row kernel"
+    S = np.tile(np.geomspace(2.0 ** -9, 40.0, L).astype(np.float16), (hq, 1))
+    q = np.zeros((hq, L, D), np.float16)
+    q[:, :, 0], q[:, :, 1] = S, 60000
+    k, v = (np.zeros((hkv, T, D), np.float16) for _ in range(2))
+    k[:, :, 1] = -1                                   # weight e^-cap at most, less than e^-cap over all
+    k[:, 1, 0], k[:, 1, 1], k[:, 2, 1] = 1, 0, 0
+    v[:, 1], v[:, 2] = 1, -1
+    if cap < 50:                                      # the others weigh: out of the call
+        k, v = k[:, 1:3], v[:, 1:3]
+        k, v = (np.tile(x, (1, T // 2, 1)) for x in (k, v))
+    if route == "cache":
+        cache = qw_amd.KVCache("fp16", hkv, D)
+        cache.update(_gpu(k), _gpu(v))
+        out = cache.attention_general(_gpu(q), scale, softcap=cap)
+    else:
+        out = qw_amd.attention(_gpu(q), _gpu(k), _gpu(v), scale, softcap=cap)
+    s = np.tanh(S.astype(np.float64) * scale / cap) * cap
+    ref = np.tanh(s / 2)[:, :, None]
+    out = _np(out)[0].astype(np.float64)
+    roundings = 2 if route == "cache" else 1         # the parts of a key split, and the output
+    bound = roundings * (np.abs(ref) * 2.0 ** -11 + 2.0 ** -25) + s[:, :, None] * 2.0 ** -22 + 3e-7
+    assert np.all(np.abs(out - ref) <= bound), np.max(np.abs(out - ref) / bound)
