@@ -321,3 +321,59 @@ def test_graph_general_options_replay():
         _ = (q.float() * 3).sum().item()  # eager work between replays
     del g
     c.close()
+
+
+def _row_kernel_calls():
+    """One call each of the routes that lay keys or key unions out in a per-stream workspace; each
+    also has a kernel that needs none (unsplit: R rows a KV head in 64-row tiles fill the CUs)."""
+    import qw_amd
+
+    r = rng(21)
+    H, G, D, L, T, W = 4, 6, 256, 700, 900, 820
+    q, k, v = (_gpu(r.standard_normal(s).astype(np.float16)) for s in ((H * G, L, D), (H, T, D), (H, T, D)))
+    assert (G * L - 100) * T >= 1300000 and G * L // 64 * H >= 256
+    m = torch.from_numpy(r.random((L, T)) < 0.8).cuda()
+    m[:, 0] = True
+    lists = _gpu(np.sort(np.stack([r.permutation(T)[:W]] * L), axis=1).astype(np.int32))
+    lengths = _gpu(np.full(L, W, np.int32))
+    assert L * W * H >= 850000 and T <= int(0.35 * 20 * W) - 1500
+    typed = lambda dt: (q.to(dt), k.to(dt), v.to(dt), lists, lengths, 1 / 16)  # noqa: E731
+    b16, f32 = typed(torch.bfloat16), typed(torch.float32)
+    return {"dense": lambda: qw_amd.causal_attention(q, k, v, 1 / 16),
+            "masked": lambda: qw_amd.attention(q, k, v, 1 / 16, m),
+            "sparse": lambda: qw_amd.sparse_attention(q, k, v, lists, lengths, 1 / 16),
+            "sparse bf16": lambda: qw_amd.sparse_attention_typed(*b16),
+            "sparse f32": lambda: qw_amd.sparse_attention_typed(*f32)}
+
+
+@pytest.mark.parametrize("warm", [True, False])
+def test_graph_row_kernels(warm):
+    """Captured behind a call on the capture stream (warm) they replay to the eager bits; on a stream
+    that never made one (no workspace can be made inside a capture) the kernels without a workspace
+    are recorded, whose results are those of the eager call but for rounding."""
+    calls = _row_kernel_calls()
+    s = torch.cuda.Stream()
+    want = {n: c() for n, c in calls.items()}
+    torch.cuda.synchronize()
+    if warm:
+        with torch.cuda.stream(s):
+            for c in calls.values():
+                c()
+        torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        outs = {n: c() for n, c in calls.items()}
+    for rep in range(3):
+        for o in outs.values():
+            o.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        for n, o in outs.items():
+            if warm:
+                assert torch.equal(o, want[n]), f"{n}, replay {rep}"
+            else:  # a unit of the output's type, and the softmax weights' fp16 rounding (dense, masked)
+                d = (o.double() - want[n].double()).norm() / want[n].double().norm()
+                bound = {"sparse bf16": 2.0 ** -8, "sparse f32": 1e-5}.get(n, 2.0 ** -10)
+                print(f"{n}: {float(d):.2e}", flush=True)
+                assert d <= bound, f"{n}, replay {rep}: {float(d)}"
+        _ = calls["dense"]()  # eager work between replays, on the current stream

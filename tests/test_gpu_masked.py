@@ -154,3 +154,30 @@ def test_masked_cache_after_a_trim(mode, D, L, causal):
     # (an affine cache that ever held a scale outside the two-step dequant's exact range rounds in
     # two steps from then on; both are the same values)
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("mode", ["affine4", "affine8", "int8", "turbo4", "fp16"])
+@pytest.mark.parametrize("hq,hkv,D,L,T", [
+    (32, 8, 128, 1020, 1155),   # 4080 rows a head: whole rounds of unsplit query tiles
+    (32, 16, 128, 1050, 1155),  # 2100: a round of them and a split tail in one launch
+    (24, 12, 256, 1500, 1601),  # 3000, a head count that does not divide the CUs
+    (32, 8, 128, 1030, 1155),   # 4120: dequantized once, the row kernel
+])
+def test_masked_cache_of_many_rows(mode, hq, hkv, D, L, T):
+    """Both sides of the line at 4096 rows a KV head, and the plans below it: every 97th row and the
+    last against the oracle, the causal cut put into its mask."""
+    import qw_amd
+
+    print(f"case {mode} hq={hq} hkv={hkv} D={D} L={L} T={T}", flush=True)
+    r = rng(hkv + D + L)
+    k, v = (r.standard_normal((hkv, T, D)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((hq, L, D)).astype(np.float16)
+    m, view = _mask(r, "bool", 1, L, T)
+    cache = qw_amd.KVCache(mode, hkv, D)
+    cache.update(_gpu(k), _gpu(v))
+    out = _np(cache.attention_general(_gpu(q), D ** -0.5, causal=True, mask=view))[0]
+    assert np.isfinite(out).all() and np.all(out[:, 1] == 0)
+    rows = np.unique(np.append(np.arange(0, L, 97), L - 1))
+    seen = m[:, rows] & (np.arange(T) <= (T - L + rows)[:, None])
+    ref = _reference(cache, mode, q[:, rows], D, D ** -0.5, False, seen)
+    assert_close(out[:, rows], ref, f"{mode} L={L} T={T}")
