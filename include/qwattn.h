@@ -198,6 +198,11 @@ int qw_sdpa(const void* q, int n_q_heads, int n_rows, const void* k, const void*
             float softcap, const void* mask, int mask_dtype, int64_t mask_head_stride,
             int64_t mask_row_stride, void* out, void* stream);
 
+/* 1 if a qw_sdpa call of this shape takes the row kernel (mask_dtype < 0: no
+ * mask), 0 if the generic one; no GPU is touched. */
+int qw_sdpa_takes_rows(int n_q_heads, int n_rows, int n_kv_heads, int n_keys, int head_dim,
+                       int causal, int window, float softcap, int mask_dtype);
+
 /* The same over a cache (n_keys = its offset): without mask, softcap or
  * window it is qw_kv_attention; with one of them what the runtime's masked
  * branch computes (update_and_fetch + layers::attention, qwen3_next.rs:

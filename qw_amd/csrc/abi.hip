@@ -198,6 +198,15 @@ int qw_sdpa(const void* q, int n_q_heads, int n_rows, const void* k, const void*
                                 out, (hipStream_t)stream));
 }
 
+int qw_sdpa_takes_rows(int n_q_heads, int n_rows, int n_kv_heads, int n_keys, int head_dim,
+                       int causal, int window, float softcap, int mask_dtype) {
+    if (n_kv_heads <= 0 || n_q_heads < n_kv_heads || n_q_heads % n_kv_heads || n_rows <= 0 || n_keys <= 0 ||
+        (head_dim != 64 && head_dim != 128 && head_dim != 256))
+        return 0;
+    qw::SdpaOptions o{causal != 0, window, softcap, mask_dtype < 0 ? nullptr : &o, mask_dtype, 0, 0};
+    return qw::sdpa_takes_rows(n_q_heads / n_kv_heads, n_rows, n_kv_heads, n_keys, head_dim, o);
+}
+
 int qw_kv_attention_general(qw_kv_cache* cache, const void* q, int n_q_heads, int n_rows,
                             float scale, int causal, int window, float softcap, const void* mask,
                             int mask_dtype, int64_t mask_head_stride, int64_t mask_row_stride,

@@ -462,23 +462,28 @@ RowsPlan plan_rows(int R, int hkv, int nw, int key_tiles) {
     return p;
 }
 
+// The key tiles (KT keys) that a query tile of 16 nw rows runs over: all, or its windows' span.
+int spanned_tiles(const SdpaOptions& o, int n_tiles, int KT, int nw, int G) {
+    return o.window > 0 ? (int)std::min<int64_t>(n_tiles, ((int64_t)o.window + 16 * nw / G + KT) / KT + 1)
+                        : n_tiles;
+}
+
+RowsPlan choose_plan(int R, int G, int hkv, int n_tiles, int KT, const SdpaOptions& o) {
+    RowsPlan p = plan_rows(R, hkv, 8, spanned_tiles(o, n_tiles, KT, 8, G));
+    if (!o.mask) {
+        const RowsPlan p12 = plan_rows(R, hkv, 12, spanned_tiles(o, n_tiles, KT, 12, G));
+        if (p12.cost < p.cost) p = p12;
+    }
+    return p;
+}
+
 template <int D>
 int rows_attention_d(const void* q, int G, int n_rows, const void* k, const void* v, int hkv,
                      int n_keys, int64_t khs, int64_t krs, int64_t vhs, int64_t vrs, float scale,
                      const SdpaOptions& o, void* out, hipStream_t stream) {
     using S = BlockShape<D>;
     const int R = G * n_rows, n_tiles = (n_keys + S::KT - 1) / S::KT;
-    // a split covers the keys a query tile's windows span
-    auto spanned = [&](int nw) {
-        return o.window > 0
-                   ? (int)std::min<int64_t>(n_tiles, ((int64_t)o.window + 16 * nw / G + S::KT) / S::KT + 1)
-                   : n_tiles;
-    };
-    RowsPlan p = plan_rows(R, hkv, 8, spanned(8));
-    if (!o.mask) {
-        const RowsPlan p12 = plan_rows(R, hkv, 12, spanned(12));
-        if (p12.cost < p.cost) p = p12;
-    }
+    const RowsPlan p = choose_plan(R, G, hkv, n_tiles, S::KT, o);
     RowsArgs a;
     a.prow0 = p.q_main * 16 * p.nw;
     a.PR = R - a.prow0;
@@ -537,6 +542,24 @@ int rows_attention_d(const void* q, int G, int n_rows, const void* k, const void
 }
 
 }  // namespace
+
+double rows_attention_us(int G, int n_rows, int hkv, int n_keys, int D, const SdpaOptions& o) {
+    const int KT = 16384 / D, R = G * n_rows, n_tiles = (n_keys + KT - 1) / KT;
+    const RowsPlan p = choose_plan(R, G, hkv, n_tiles, KT, o);
+    const int PR = R - p.q_main * 16 * p.nw, tail = (p.n_qt - p.q_main) * hkv;
+    const int tile0 = window_first_key(o, n_keys, n_rows, KT) / KT;
+    // the longest run of key tiles on a CU
+    const double cut = o.causal && o.window <= 0 ? 1.0 - 0.5 * n_rows / n_keys : 1.0;
+    double chain = p.q_main * hkv / 256 * spanned_tiles(o, n_tiles, KT, p.nw, G) * cut;
+    if (tail > 0) chain += (tail * p.n_split + 255) / 256 * p.tps;
+    const double laid_out = 1e-6 * (n_tiles - tile0) * hkv * 16384;
+    const double partials = p.n_split > 1 ? 8e-6 * p.n_split * hkv * PR * D : 0.0;  // MB
+    double step = 1.9 + 80.0 / D;
+    if (o.softcap > 0.0f) step += 0.2 + 150.0 / D;
+    if (o.mask) step += (o.mask_dtype == QW_MASK_BOOL ? 130.0 : 280.0) / D;
+    if (p.nw == 12) step *= 1.3;
+    return 11.5 + 1.3 * laid_out + step * chain + (0.15 + 24.0 / D) * partials;
+}
 
 int rows_attention(const void* q, int G, int n_rows, const void* k, const void* v, int hkv,
                    int n_keys, int head_dim, int64_t khs, int64_t krs, int64_t vhs, int64_t vrs,

@@ -315,6 +315,9 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
 int rows_attention(const void* q, int G, int n_rows, const void* k, const void* v, int hkv,
                    int n_keys, int head_dim, int64_t khs, int64_t krs, int64_t vhs, int64_t vrs,
                    float scale, const SdpaOptions& o, void* out, hipStream_t stream);
+// What that takes, estimated in us, and whether sdpa_general's calls take it by that.
+double rows_attention_us(int G, int n_rows, int hkv, int n_keys, int head_dim, const SdpaOptions& o);
+bool sdpa_takes_rows(int G, int n_rows, int hkv, int n_keys, int head_dim, const SdpaOptions& o);
 // The first key any of n_rows causal windowed rows over T keys sees (0 without
 // a window), rounded down to a multiple of align; and the options of a call on
 // keys lo .. n_keys - 1 only (the mask's columns shifted by lo).

@@ -301,21 +301,48 @@ void launch_general(const GenArgs& a, int nwv, dim3 grid, hipStream_t stream) {
         launch_general<D, 4>(a, grid, stream);
 }
 
-// Whether a call takes the row kernel (attend_rows.hip), which lays every key
-// tile out once and then runs at several times this kernel's rate: 1536 rows
-// over 9728 keys (24 heads over 4, D = 256) 1943 -> 372 us. The layout and two
-// more launches cost what some 100 rows a KV head do, so the line lies at
-// (R - 100) T of 1.3M: at 384 rows a head 43.8 against 46.3 us over 4k keys
-// (here) and 130.8 -> 76.0 us over 16k (there), at 1536 rows 27.8 against 31.0
-// us over 300 keys and 52.7 -> 38.4 us over 1k. A mask is read a byte or two a
-// lane here and in 8-key pieces there, so a masked call's line lies lower: 78 rows
-// over 8k keys 49 -> 33 us with the layout and the merge.
-bool rows_route(int R, int n_keys, int hkv, int D, bool mask, const void* out, hipStream_t stream) {
-    if ((uintptr_t)out % 8 != 0) return false;  // (it writes 8-byte pieces)
-    if (stream == hipStreamPerThread) return false;  // (one handle, a stream a thread)
-    // images of more than 4 GiB are not kept (1.03 KB a key and head at D = 256)
-    if ((int64_t)n_keys * hkv * D * 2 * sizeof(f16) > (int64_t)4 << 30) return false;
-    return mask ? R > 16 && (int64_t)R * n_keys >= 500000 : (int64_t)(R - 100) * n_keys >= 1300000;
+// How the kernel here divides a call. Up to 16 rows a KV head: one-wave workgroups
+// (about 1024 of them); else four-wave ones (about 256). Key splits of whole tiles, at
+// least four tiles each, at most 256 (the merge's limit).
+struct GenPlan {
+    int nwv, tiles, n_split, split_tiles, kt;  // row tiles, key tiles a split, keys a tile
+};
+GenPlan plan_general(int R, int hkv, int n_keys) {
+    GenPlan p;
+    p.nwv = R <= 16 ? 1 : 4;
+    p.kt = p.nwv == 1 ? 16 : 32;
+    p.tiles = (R + 16 * p.nwv - 1) / (16 * p.nwv);
+    const int units = p.tiles * hkv, key_tiles = (n_keys + p.kt - 1) / p.kt;
+    const int target = p.nwv == 1 ? 1024 : 256;
+    const int ns = std::max(1, std::min({target / std::max(1, units), (key_tiles + 3) / 4, 256}));
+    p.split_tiles = (key_tiles + ns - 1) / ns;
+    p.n_split = (key_tiles + p.split_tiles - 1) / p.split_tiles;
+    return p;
+}
+
+// What that takes for more than 16 rows a KV head, estimated in us.
+double general_us(int G, int n_rows, int hkv, int n_keys, int D, const SdpaOptions& o) {
+    const int R = G * n_rows;
+    const GenPlan p = plan_general(R, hkv, n_keys);
+    double tiles = p.split_tiles;  // of a workgroup
+    if (o.window > 0)
+        tiles = std::min(tiles, (double)(o.window + 64 / G) / 32 + 1);
+    else if (o.causal && p.n_split == 1)
+        tiles *= 1.0 - 0.5 * n_rows / n_keys;
+    const double rounds = std::max(1.0, (double)p.tiles * hkv * p.n_split / 256);
+    const double partials = p.n_split > 1 ? 8e-6 * p.n_split * hkv * R * D : 0.0;  // MB
+    double step = 0.7 + 0.006 * D;
+    if (o.mask) step += 1.15 + 0.0013 * D;
+    if (o.softcap > 0.0f) step += 0.2 + 0.0015 * D;
+    return 6.5 + step * tiles * rounds + (0.22 + 12.0 / D) * partials;
+}
+
+// (an output off 8 bytes: it writes 8-byte pieces; hipStreamPerThread: one handle for a
+// stream a thread, so no workspace of a stream's own)
+bool rows_route(int G, int n_rows, int hkv, int n_keys, int D, const SdpaOptions& o, const void* out,
+                hipStream_t stream) {
+    return (uintptr_t)out % 8 == 0 && stream != hipStreamPerThread &&
+           sdpa_takes_rows(G, n_rows, hkv, n_keys, D, o);
 }
 
 int mask_kind_of(int dtype) {
@@ -329,6 +356,26 @@ int mask_kind_of(int dtype) {
 }
 
 }  // namespace
+
+// Whether a call takes the row kernel (attend_rows.hip), which lays every key tile out
+// once and then runs at several times this kernel's rate: 1536 rows over 9728 keys (24
+// heads over 4, D = 256) 1943 -> 387 us. Against it stand the layout (a read and a write
+// of K and V) and a launch more, so the line depends on the rows, the keys, the heads and
+// the head dim together; it lies where the two estimates meet. Their coefficients are
+// fitted to 2,500 calls timed by both kernels (11 head geometries at D = 64 / 128 / 256,
+// 300 to 64k keys, 17 to 3072 rows a KV head; plain, windows, softcap, bool and fp16
+// masks): half of the estimates are within 3 %, nine in ten within 20 %. Rows a KV head
+// over keys, here / there in us: 24 heads over 4, D = 256, 252 over 16k 85 / 64, 510 over
+// 4k 51 / 37, but 252 over 4k 33 / 37, 1536 over 300 28 / 32; 16 over 1, D = 64, 512 over
+// 16k 27 / 23, but 1536 over 1k 12 / 20. A twentieth of the difference is left to this
+// kernel (a seventh with a window, where the estimates are wider off).
+bool sdpa_takes_rows(int G, int n_rows, int hkv, int n_keys, int D, const SdpaOptions& o) {
+    if (G * n_rows <= 16) return false;
+    // images of more than 4 GiB are not kept (1.03 KB a key and head at D = 256)
+    if ((int64_t)n_keys * hkv * D * 2 * sizeof(f16) > (int64_t)4 << 30) return false;
+    return rows_attention_us(G, n_rows, hkv, n_keys, D, o) * (o.window > 0 ? 1.15 : 1.05) <
+           general_us(G, n_rows, hkv, n_keys, D, o);
+}
 
 int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const void* v,
                  int n_kv_heads, int n_keys, int head_dim, int64_t khs, int64_t krs, int64_t vhs,
@@ -356,7 +403,7 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
     QW_REQUIRE(!o.mask || (o.mask_head_stride >= 0 && o.mask_row_stride >= 0),
                QW_ERR_INVALID_ARGUMENT, "sdpa: negative mask stride");
     const int G = n_q_heads / n_kv_heads, R = G * n_rows, D = head_dim;
-    if (rows_route(R, n_keys, n_kv_heads, D, o.mask != nullptr, out, stream)) {
+    if (rows_route(G, n_rows, n_kv_heads, n_keys, D, o, out, stream)) {
         const int rc = rows_attention(q, G, n_rows, k, v, n_kv_heads, n_keys, D, khs, krs, vhs, vrs,
                                       scale, o, out, stream);
         // without room for the images (under capture, or no memory left) the
@@ -386,18 +433,10 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
     a.window = o.window > 0 ? o.window : 0;
     a.scale_h = (float)(f16)scale;
     a.softcap = Softcap::of(scale, o.softcap);
-    // Up to 16 rows a KV head: one-wave workgroups (about 1024 of them);
-    // else four-wave ones (about 256). Key splits of whole tiles, at least
-    // four tiles each, at most 256 (the merge's limit).
-    const int nwv = R <= 16 ? 1 : 4, kt = nwv == 1 ? 16 : 32;
-    const int tiles = (R + 16 * nwv - 1) / (16 * nwv), units = tiles * n_kv_heads;
-    const int key_tiles = (n_keys + kt - 1) / kt;
-    const int target = nwv == 1 ? 1024 : 256;
-    int ns = std::max(1, std::min({target / std::max(1, units), (key_tiles + 3) / 4, 256}));
-    const int kps = ((key_tiles + ns - 1) / ns) * kt;
-    ns = (n_keys + kps - 1) / kps;
+    const GenPlan p = plan_general(R, n_kv_heads, n_keys);
+    const int ns = p.n_split;
     a.n_split = ns;
-    a.keys_per_split = kps;
+    a.keys_per_split = p.split_tiles * p.kt;
     int dev = 0;
     QW_HIP_CHECK(hipGetDevice(&dev));
     if (ns > 1) {
@@ -408,13 +447,13 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
         a.part_o = (float*)ws;
         a.part_ml = (float2*)((char*)ws + no * D * sizeof(float));
     }
-    const dim3 grid(ns, tiles, n_kv_heads);
+    const dim3 grid(ns, p.tiles, n_kv_heads);
     if (D == 256)
-        launch_general<256>(a, nwv, grid, stream);
+        launch_general<256>(a, p.nwv, grid, stream);
     else if (D == 128)
-        launch_general<128>(a, nwv, grid, stream);
+        launch_general<128>(a, p.nwv, grid, stream);
     else
-        launch_general<64>(a, nwv, grid, stream);
+        launch_general<64>(a, p.nwv, grid, stream);
     QW_HIP_CHECK(hipGetLastError());
     if (ns > 1)
         return launch_partial_merge(a.part_o, a.part_ml, ns, R, 0, R, n_kv_heads, D, G, n_rows,

@@ -132,3 +132,42 @@ def test_general_attention_contract_fails_before_device_work(qwlib):
     assert call(mask=one, md=0, mrs=-1) == 1
     assert f(None, 8, 4, one, one, 2, 100, 128, 0, 128, 0, 128, 0.1, 1, 0, 0.0, None, 0, 0, 0,
              one, None) == 1
+
+
+@pytest.mark.parametrize("hq,hkv,D,L,T,kind,generic_us,rows_us", [
+    # calls that both kernels were timed on, near the line
+    (24, 4, 256, 85, 4000, "causal", 51, 37),
+    (24, 4, 256, 42, 4000, "causal", 33, 37),
+    (24, 4, 256, 42, 16000, "causal", 85, 64),
+    (24, 4, 256, 256, 300, "causal", 28, 32),
+    (8, 8, 128, 384, 4000, "causal", 46, 33),
+    (8, 8, 128, 192, 1000, "causal", 16, 21),
+    (32, 8, 128, 64, 16000, "causal", 102, 58),
+    (16, 1, 64, 96, 4000, "causal", 24, 21),
+    (16, 1, 64, 96, 1000, "causal", 12, 20),
+    (16, 2, 64, 24, 16000, "causal", 23, 25),
+    (16, 1, 128, 12, 4000, "causal", 16, 20),
+    (24, 4, 256, 42, 4000, "bool", 43, 36),
+    (16, 2, 64, 32, 1000, "bool", 15, 25),
+    (8, 8, 128, 192, 4000, "bool", 47, 29),
+    (8, 8, 64, 96, 4000, "f16", 28, 34),
+    (8, 8, 64, 425, 4000, "window 64", 11, 23),
+    (24, 4, 256, 170, 16000, "softcap", 350, 147),
+    (8, 8, 64, 96, 4000, "softcap", 20, 27),
+])
+def test_sdpa_row_kernel_line(qwlib, hq, hkv, D, L, T, kind, generic_us, rows_us):
+    """The kernel of a qw_sdpa call: the one that measured faster."""
+    window = 64 if kind == "window 64" else 0
+    mask = {"bool": 3, "f16": 0}.get(kind, -1)
+    takes = qwlib.qw_sdpa_takes_rows(hq, L, hkv, T, D, int(mask < 0), window,
+                                     30.0 if kind == "softcap" else 0.0, mask)
+    assert takes == (rows_us < generic_us)
+
+
+def test_sdpa_row_kernel_line_limits(qwlib):
+    f = qwlib.qw_sdpa_takes_rows
+    assert f(24, 3072, 4, 524288, 256, 1, 0, 0.0, -1) == 1
+    assert f(24, 3072, 4, 2097153, 256, 1, 0, 0.0, -1) == 0  # images past 4 GiB
+    assert f(16, 1, 1, 1 << 20, 256, 1, 0, 0.0, 3) == 0      # 16 rows a KV head
+    assert f(24, 4, 5, 100, 256, 1, 0, 0.0, -1) == 0 and f(24, 0, 4, 100, 256, 1, 0, 0.0, -1) == 0
+    assert f(24, 1 << 20, 4, 1 << 20, 256, 1, 0, 0.0, -1) == 1  # (no overflow on the way)

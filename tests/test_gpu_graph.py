@@ -10,6 +10,7 @@ import pytest
 
 from conftest import rng
 from test_gpu_kv import _gpu, _np
+from test_gpu_rows import takes_rows
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -329,9 +330,10 @@ def _row_kernel_calls():
     import qw_amd
 
     r = rng(21)
-    H, G, D, L, T, W = 4, 6, 256, 700, 900, 820
+    H, G, D, L, T, W = 4, 6, 256, 700, 1200, 820
     q, k, v = (_gpu(r.standard_normal(s).astype(np.float16)) for s in ((H * G, L, D), (H, T, D), (H, T, D)))
-    assert (G * L - 100) * T >= 1300000 and G * L // 64 * H >= 256
+    assert takes_rows(H * G, H, D, L, T) and takes_rows(H * G, H, D, L, T, False, 0, 0.0, 3)
+    assert G * L // 64 * H >= 256
     m = torch.from_numpy(r.random((L, T)) < 0.8).cuda()
     m[:, 0] = True
     lists = _gpu(np.sort(np.stack([r.permutation(T)[:W]] * L), axis=1).astype(np.int32))

@@ -28,30 +28,48 @@ def _views(r, hkv, T, D, pad):
     return k, v, kb[:, :T, :D], vb[:, :T, :D]
 
 
+def takes_rows(hq, hkv, D, L, T, causal=True, window=0, softcap=0.0, mask=-1):
+    """Whether the call runs the row kernel (mask: its ABI dtype)."""
+    import qw_amd
+
+    return bool(qw_amd.lib().qw_sdpa_takes_rows(hq, L, hkv, T, D, int(causal), window, softcap, mask))
+
+
 CASES = [
     # hq, hkv, D, L, T, causal, window, softcap
     (24, 4, 256, 129, 2048, True, 0, 0.0),     # whole tiles; 774 rows a head, a ragged last tile
     (24, 4, 256, 257, 1985, True, 0, 0.0),     # one key into the last tile
     (24, 4, 256, 257, 1983, True, 0, 0.0),     # one key short of it
     (8, 8, 128, 700, 2305, True, 0, 0.0),      # G = 1
-    (32, 8, 128, 200, 2047, True, 130, 0.0),   # a window about a tile
-    (16, 2, 64, 256, 1281, True, 0, 0.0),      # 256-key tiles in two halves
-    (16, 2, 64, 300, 1500, True, 33, 20.0),    # a window below a tile, capped
+    (32, 8, 128, 200, 2047, True, 300, 0.0),   # a window of a few tiles
+    (8, 8, 128, 151, 2047, True, 130, 0.0),    # and about one
+    (24, 4, 256, 90, 1000, True, 64, 0.0),
+    (16, 2, 64, 300, 1281, True, 0, 0.0),      # 256-key tiles in two halves
+    (16, 2, 64, 300, 2500, True, 900, 20.0),   # capped, in a window
+    (24, 4, 256, 130, 1400, True, 100, 30.0),
     (24, 4, 128, 220, 1400, False, 0, 30.0),   # capped, not causal
-    (24, 4, 128, 220, 1400, True, 0, 128.0),   # the largest cap of the direct form
-    (24, 4, 128, 220, 1400, True, 0, 300.0),   # one past it
-    (12, 1, 256, 190, 1000, True, 0, 0.0),     # one KV head, G = 12
+    (24, 4, 128, 220, 1400, True, 0, 128.0),   # caps far above the scores
+    (24, 4, 128, 220, 1400, True, 0, 300.0),
+    (12, 1, 256, 300, 1000, True, 0, 0.0),     # one KV head, G = 12
     (24, 4, 256, 1100, 1100, True, 0, 0.0),    # prefill into nothing: rows from one key on
+]
+# shapes that the generic kernel serves faster (it must agree there too)
+GENERIC = [
+    (32, 8, 128, 200, 2047, True, 130, 0.0),
+    (16, 2, 64, 256, 1281, True, 0, 0.0),
+    (16, 2, 64, 300, 1500, True, 33, 20.0),
+    (12, 1, 256, 190, 1000, True, 0, 0.0),
 ]
 
 
-@pytest.mark.parametrize("hq,hkv,D,L,T,causal,window,softcap", CASES)
+@pytest.mark.parametrize("hq,hkv,D,L,T,causal,window,softcap", CASES + GENERIC)
 def test_rows_match_oracle(hq, hkv, D, L, T, causal, window, softcap):
     import qw_amd
 
     print(f"case hq={hq} hkv={hkv} D={D} L={L} T={T} causal={causal} w={window} sc={softcap}",
           flush=True)
-    assert (hq // hkv * L - 100) * T >= 1300000 or L == 190, "a shape of the row kernel"
+    shape = (hq, hkv, D, L, T, causal, window, softcap)
+    assert takes_rows(*shape) == (shape in CASES), "the kernel of the call"
     r = rng(hq + D + L + T)
     q = r.standard_normal((hq, L, D)).astype(np.float16)
     k, v, kv, vv = _views(r, hkv, T, D, 9)
@@ -64,14 +82,18 @@ def test_rows_match_oracle(hq, hkv, D, L, T, causal, window, softcap):
 @pytest.mark.parametrize("kind", ["bool", "f16", "bf16", "f32"])
 @pytest.mark.parametrize("hq,hkv,D,L,T,causal,per_head", [
     (24, 4, 256, 13, 6500, False, False),
-    (24, 4, 128, 41, 2051, True, True),
-    (16, 2, 64, 20, 3333, False, True),
+    (24, 4, 128, 60, 2051, True, True),
+    (16, 2, 64, 100, 3333, False, True),
+    (24, 4, 128, 41, 2051, True, True),       # (a bool mask alone; the others in the generic kernel)
+    (16, 2, 64, 20, 3333, False, True),       # (the generic kernel)
 ])
 def test_rows_masks_match_oracle(kind, hq, hkv, D, L, T, causal, per_head):
     import qw_amd
 
     print(f"case {kind} hq={hq} D={D} L={L} T={T} causal={causal}", flush=True)
-    assert hq // hkv * L * T >= 500000, "a shape of the row kernel"
+    code = {"bool": 3, "f16": 0, "bf16": 1, "f32": 2}[kind]
+    assert takes_rows(hq, hkv, D, L, T, causal, 0, 0.0, code) == \
+        (L in (13, 60, 100) or (L == 41 and kind == "bool")), "the kernel of the call"
     r = rng(hq + D + L + T + len(kind))
     q = r.standard_normal((hq, L, D)).astype(np.float16)
     k, v, kv, vv = _views(r, hkv, T, D, 3)
@@ -104,6 +126,7 @@ def test_rows_route_agrees_with_the_general_kernel():
 
     r = rng(5)
     hq, hkv, D, L, T = 24, 4, 256, 160, 1700
+    assert takes_rows(hq, hkv, D, L, T) and not takes_rows(hq, hkv, D, 16, T)
     q = _gpu(r.standard_normal((hq, L, D)).astype(np.float16))
     _, _, kv, vv = _views(r, hkv, T, D, 0)
     whole = _np(qw_amd.causal_attention(q, kv, vv, 1 / 16))[0]
@@ -121,7 +144,7 @@ def test_rows_largest_weight_is_not_rounded(hkv, D):
     (below e^-1 2^-12) and fp32 sums: the result is within 2^-12 of 1, which rounds to 1."""
     import qw_amd
 
-    G, L, T = 6, 200, 1300
+    G, L, T = 6, 400, 1300
     s = np.linspace(1, 5.4, L).astype(np.float16)
     q = np.zeros((G * hkv, L, D), np.float16)
     q[:, :, 0] = s * np.float16(16)
@@ -129,19 +152,20 @@ def test_rows_largest_weight_is_not_rounded(hkv, D):
     k[:, :, 0] = -60
     k[:, 3, 0] = 0
     k[:, 66 if D == 256 else 130, 0] = 1  # the next 64- or 128-key step of the same key split
-    assert (G * L - 100) * T >= 1300000, "a shape of the row kernel"
+    assert takes_rows(G * hkv, hkv, D, L, T, False), "a shape of the row kernel"
     out = _np(qw_amd.attention(_gpu(q), _gpu(k), _gpu(np.ones_like(k)), 1 / 16))[0]
     assert np.all(out == 1), np.unique(out)
 
 
 @pytest.mark.parametrize("hq,hkv,D,L,T,window,softcap,masked", [
     (24, 4, 256, 230, 1400, 0, 0.0, False),
-    (24, 4, 256, 230, 1400, 37, 30.0, False),
+    (24, 4, 256, 130, 1400, 100, 30.0, False),
     (8, 8, 128, 700, 2305, 0, 0.0, False),
     (8, 8, 128, 701, 2305, 300, 0.0, False),
-    (8, 8, 128, 700, 2305, 61, 25.0, False),
-    (16, 2, 64, 256, 1281, 0, 0.0, False),
-    (16, 2, 64, 255, 1281, 5, 0.0, False),      # a window inside one 8-key block
+    (8, 8, 128, 151, 2047, 130, 0.0, False),
+    (24, 4, 256, 90, 1000, 64, 0.0, False),
+    (16, 2, 64, 300, 1281, 0, 0.0, False),
+    (16, 2, 64, 301, 2500, 900, 25.0, False),
     (24, 4, 256, 100, 1290, 0, 0.0, True),
 ])
 def test_rows_keep_keys_outside_their_limits_out(hq, hkv, D, L, T, window, softcap, masked):
@@ -150,7 +174,7 @@ def test_rows_keep_keys_outside_their_limits_out(hq, hkv, D, L, T, window, softc
     import qw_amd
 
     G = hq // hkv
-    assert masked or (G * L - 100) * T >= 1300000, "a shape of the row kernel"
+    assert takes_rows(hq, hkv, D, L, T, True, window, softcap, 3 if masked else -1), "a shape of the row kernel"
     r = rng(hq + D + L + window)
     q = _gpu(r.standard_normal((hq, L, D)).astype(np.float16))
     k, v, kv, vv = _views(r, hkv, T, D, 0)

@@ -8,18 +8,19 @@ import pytest
 
 from conftest import rng
 from test_gpu_kv import _gpu
+from test_gpu_rows import takes_rows
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
 def _dense(seed, L, T):
-    """A row-kernel call (G L - 100) T >= 1.3M over its own keys."""
+    """A row-kernel call over its own keys."""
     import qw_amd
 
     r = rng(seed)
     q, k, v = (_gpu(r.standard_normal(s).astype(np.float16)) for s in ((24, L, 256), (4, T, 256), (4, T, 256)))
-    assert (6 * L - 100) * T >= 1300000
+    assert takes_rows(24, 4, 256, L, T)
     return lambda: qw_amd.causal_attention(q, k, v, 1 / 16)
 
 
@@ -29,7 +30,7 @@ def _masked(seed, L, T):
     r = rng(seed)
     q, k, v = (_gpu(r.standard_normal(s).astype(np.float16)) for s in ((24, L, 256), (4, T, 256), (4, T, 256)))
     m = torch.from_numpy(r.random((L, T)) < 0.8).cuda()
-    assert 6 * L * T >= 500000
+    assert takes_rows(24, 4, 256, L, T, False, 0, 0.0, 3)
     return lambda: qw_amd.attention(q, k, v, 1 / 16, m)
 
 
@@ -46,7 +47,7 @@ def _sparse(seed, L, T, W, dt):
 
 
 def _calls():
-    return [_dense(1, 128, 2500), _dense(2, 300, 4000), _masked(3, 20, 6000),
+    return [_dense(1, 128, 2500), _dense(2, 300, 4000), _masked(3, 25, 6000),
             _sparse(4, 128, 3000, 1700, torch.float16), _sparse(5, 300, 4000, 1800, torch.float16),
             _sparse(6, 128, 2000, 700, torch.bfloat16), _sparse(7, 70, 1500, 300, torch.float32)]
 
