@@ -15,7 +15,7 @@ def _shapes(r, n):
     base = r.standard_normal(n).astype(np.float32)
     top = np.sort(base)[::-1]
     yield "normal", base
-    for same in (63, 64, 65, 500):               # equal scores in a wanted bin
+    for same in (63, 64, 65, 255, 256, 257, 500):               # equal scores in a wanted bin
         s = base.copy()
         s[r.choice(n, min(n, same), replace=False)] = top[3]
         yield f"{same} equal", s
@@ -38,6 +38,19 @@ def _shapes(r, n):
     s[7] = np.nan
     yield "nan", s
     yield "descending", top.copy()
+    s = base.copy()
+    s[::3] = np.finfo(np.float32).min
+    yield "a third masked", s
+    s = base.copy()
+    s[:n // 2] = -1e4
+    yield "the first half masked", s
+    s[n // 2:] = np.where(r.random(n - n // 2) < 0.9, -np.inf, s[n // 2:])
+    yield "few finite", s
+    for k in (3, 4, 70, 300):                        # fewer than the groups of lanes, as many, more than a bin
+        s = base.copy()
+        s[r.choice(n, min(n, k), replace=False)] = np.inf if k == 3 else 1e3
+        yield f"{k} outliers", s
+    yield "heavy tail", np.exp(3 * base)
 
 
 @pytest.mark.parametrize("t,threads", [(1024, 64), (8704, 64), (8704, 256), (8704, 1024),
