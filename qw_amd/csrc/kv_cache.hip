@@ -549,9 +549,7 @@ __global__ __launch_bounds__(256) void append_fp16_kernel(RowSrc rs, int n_token
 }
 
 // The same with an element a thread: K rotated on the load (the library's sine and
-// cosine are most of the work), and appends below a block, which would leave most of
-// the pieces above empty (one token into 131071: 58.0 against 59.2 us for the whole
-// sparse decode step).
+// cosine are most of the work), and shorter appends, below kBlockCopy.
 template <int D>
 __global__ __launch_bounds__(256) void append_fp16_elem_kernel(RowSrc rs, int n_tokens, int t_old,
                                                           int cap, f16* __restrict__ k_data,
@@ -588,6 +586,13 @@ int KVCache::update(const void* k_new, const void* v_new, int n_tokens, hipStrea
 // against it, 700 tokens 8.0 / 8.4 us, 1024 8.2 / 8.5, 1500 9.5 / 8.7, 4096 18.0 / 15.0;
 // 2 heads, 2048 tokens 8.5 / 8.6, 4096 12.2 / 10.0; 16 heads, 512 tokens 12.0 / 9.8.
 constexpr int64_t kBlockAppend = 5 << 18;
+// And an fp16 append, which starts whole blocks (offset % 8 == 0) / which does not (single
+// halves of V): fewer threads of longer chains cost 1 us / 2.5 us more until the element
+// form's 2-byte stores cost that. An element a thread against it, 4 heads, D = 256: 8
+// tokens 3.2 / 3.9 us (off a block 3.2 / 5.8), 256 4.3 / 4.3 (4.3 / 5.7), 512 5.5 / 4.4 (5.5 /
+// 5.8), 1024 7.5 / 4.7 (7.6 / 6.0); 8 heads, D = 128, 512 tokens 4.6 / 4.4 (4.9 / 5.8); 16
+// heads, D = 256, 128 tokens 5.5 / 4.4 (5.5 / 5.9); the same at 1 and 2 heads by bytes.
+constexpr int64_t kBlockCopy = 3 << 17, kBlockCopyOff = 3 << 18;
 
 int KVCache::update_rows(const RowSrc& rs, int n_tokens, hipStream_t stream) {
     if (n_tokens == 0) return QW_OK;
@@ -634,7 +639,8 @@ int KVCache::update_rows(const RowSrc& rs, int n_tokens, hipStream_t stream) {
                                (uint32_t*)v_data, (f16*)v_params, fast_flag);
     } else {
         const int nblk = (offset + n_tokens - 1) / 8 - offset / 8 + 1;
-        const bool elem = rs.rope_dims > 0 || n_tokens < 8;
+        const bool elem = rs.rope_dims > 0 ||
+                          (int64_t)n_tokens * hkv * D < (offset % 8 ? kBlockCopyOff : kBlockCopy);
         const int64_t threads = elem ? (int64_t)n_tokens * D : (int64_t)nblk * (D / 8);
         const dim3 grid((unsigned)std::min<int64_t>((threads + 255) / 256, elem ? 1024 : INT_MAX), hkv);
         auto launch = [&](auto kernel) {

@@ -57,6 +57,29 @@ def test_fp16_appends_around_blocks(D):
     np.testing.assert_array_equal(V, v)
 
 
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("at,extra,skew", [(0, -1, 0), (0, 0, 0), (8, 5, 0), (3, -1, 0), (3, 0, 0),
+                                           (5, 6, 0), (7, 1, 3), (0, 2, 3)])
+def test_long_fp16_appends(D, at, extra, skew):
+    """About the line to the block-wise form (2 n D halves: 3 << 17 from a block's start, 3 << 18
+    from inside one), from and to the middle of blocks; skew: the rows off 16 bytes."""
+    import qw_amd
+
+    r, H = rng(D + at + extra), 2
+    n = (3 << (18 if at % 8 else 17)) // (H * D) + extra
+    k, v = (r.standard_normal((H, at + n, D)).astype(np.float16) for _ in range(2))
+    c, L = qw_amd.KVCache("fp16", H, D), qw_amd.lib()
+    if at:
+        c.update(_gpu(k[:, :at]), _gpu(v[:, :at]))
+    src = torch.zeros(2 * H * n * D + skew, dtype=torch.float16, device="cuda:0")
+    src[skew:] = _gpu(np.concatenate([k[:, at:].reshape(-1), v[:, at:].reshape(-1)]))
+    p = src.data_ptr() + 2 * skew
+    assert L.qw_kv_update(c._h, p, p + 2 * H * n * D, n, torch.cuda.current_stream().cuda_stream) == 0
+    K, V = (_np(x)[0] for x in c.dequantize())
+    np.testing.assert_array_equal(K, k)
+    np.testing.assert_array_equal(V, v)
+
+
 def test_fp16_pointers_off_16_bytes():
     import qw_amd
 
