@@ -16,6 +16,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <type_traits>
 
 #include "kv_cache.hpp"
 #include "append.hpp"
@@ -676,8 +677,10 @@ __device__ inline f16 mlx_dequant(uint32_t c, int off, f16 s, f16 b) {
 // bytes) a key, every load issued before the first is used; then a 16-byte store a
 // key and plane, 64 lanes covering whole rows. HBM-bound: 8192 rows of 4 heads, D =
 // 256, 4-bit (9.4 MB in, 33.6 out) in 8.8 us; one key a thread, each element's code
-// gathered for itself, took 26.4 us.
-template <int BITS, int D>
+// gathered for itself, took 26.4 us. Short windows leave the chip to few such threads
+// (64 rows 4.6 us): there a thread of KPT = 1 forms one key of the eight (3.3 us; 512 rows
+// 4.9 / 4.9, 2048 rows 5.7 in blocks).
+template <int BITS, int D, int KPT>
 __global__ __launch_bounds__(256) void fetch_kernel(const void* __restrict__ k_data,
                                                     const uint32_t* __restrict__ k_params,
                                                     const void* __restrict__ v_data,
@@ -690,8 +693,9 @@ __global__ __launch_bounds__(256) void fetch_kernel(const void* __restrict__ k_d
     constexpr int E = 16 / BITS;       // dims a piece
     constexpr int KW = BITS / 4;       // words of 8 dims of a K row
     const int h = blockIdx.y, unit = blockIdx.x * 256 + threadIdx.x;
-    const int blk = start / 8 + unit / OCT, d0 = unit % OCT * 8, g = d0 / kGroup;
-    if (8 * blk >= start + n) return;
+    const int d0 = unit % OCT * 8, g = d0 / kGroup, first = start / 8 * 8 + unit / OCT * KPT;
+    const int blk = first / 8, k0 = KPT == 8 ? 0 : first % 8;  // (keys k0 .. k0 + KPT - 1 of the block)
+    if (first >= start + n) return;
     const int64_t gblk = (int64_t)h * (cap / 8) + blk;
     u32x4 vc[NV];
 #pragma unroll
@@ -703,34 +707,34 @@ __global__ __launch_bounds__(256) void fetch_kernel(const void* __restrict__ k_d
         vs = vp[0];
         vb = vp[1];
     }
-    uint32_t kc[8][KW], ksb[8] = {};
+    uint32_t kc[KPT][KW], ksb[KPT] = {};
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const int64_t row = gblk * 8 + k;  // (rows of a block exist up to cap)
+    for (int k = 0; k < KPT; k++) {
+        const int64_t row = gblk * 8 + k0 + k;  // (rows of a block exist up to cap)
         const uint32_t* p = (const uint32_t*)k_data + (row * D + d0) * BITS / 32;
 #pragma unroll
         for (int w = 0; w < KW; w++) kc[k][w] = p[w];
         if constexpr (BITS != 16) ksb[k] = k_params[row * NG + k_param_slot(g, NG)];
     }
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const int r = 8 * blk + k - start;
+    for (int i = 0; i < KPT; i++) {
+        const int k = k0 + i, r = 8 * blk + k - start;
         if (r < 0 || r >= n) continue;
         half8 ko, vo;
-        const half2v sb = h2(ksb[k]);
+        const half2v sb = h2(ksb[i]);
         const f16 s = h2(vs[k / 2])[k & 1], b = h2(vb[k / 2])[k & 1];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             // piece e / E holds dims in turn, each 32 / 64 / 128 bits of 8 keys
             const u32x4 w = vc[e / E];
             if constexpr (BITS == 16) {
-                ko[e] = h2(kc[k][e / 2])[e & 1];
+                ko[e] = h2(kc[i][e / 2])[e & 1];
                 vo[e] = h2(w[k / 2])[k & 1];
             } else if constexpr (BITS == 8) {
-                ko[e] = mlx_dequant((kc[k][e / 4] >> (8 * (e & 3))) & 0xFFu, code_off, sb.x, sb.y);
+                ko[e] = mlx_dequant((kc[i][e / 4] >> (8 * (e & 3))) & 0xFFu, code_off, sb.x, sb.y);
                 vo[e] = mlx_dequant((w[2 * (e & 1) + k / 4] >> (8 * (k & 3))) & 0xFFu, code_off, s, b);
             } else {
-                ko[e] = mlx_dequant((kc[k][0] >> (4 * e)) & 0xFu, code_off, sb.x, sb.y);
+                ko[e] = mlx_dequant((kc[i][0] >> (4 * e)) & 0xFu, code_off, sb.x, sb.y);
                 vo[e] = mlx_dequant((w[e & 3] >> (4 * v4_nibble_pos(k))) & 0xFu, code_off, s, b);
             }
         }
@@ -739,6 +743,8 @@ __global__ __launch_bounds__(256) void fetch_kernel(const void* __restrict__ k_d
         *(half8*)(v_out + o) = vo;
     }
 }
+
+constexpr int64_t kShortFetch = 1 << 19;  // halves of K
 
 // fp16 mode into outputs off 16-byte alignment: element by element.
 __global__ __launch_bounds__(256) void fetch_fp16_kernel(const f16* __restrict__ k_data,
@@ -775,18 +781,25 @@ int KVCache::dequantize(int start, int n, void* k_out, void* v_out, hipStream_t 
         return QW_OK;
     }
     const int nblk = (start + n - 1) / 8 - start / 8 + 1;
-    const dim3 grid((unsigned)(((int64_t)nblk * (D / 8) + 255) / 256), hkv);
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, k_data, k_params, v_data,
-                           (const f16*)v_params, int8() ? 128 : 0, cap, start, n, (f16*)k_out,
-                           (f16*)v_out);
+    auto run = [&](auto kpt) {
+        constexpr int KPT = decltype(kpt)::value;
+        const dim3 grid((unsigned)(((int64_t)nblk * (8 / KPT) * (D / 8) + 255) / 256), hkv);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, k_data, k_params, v_data,
+                               (const f16*)v_params, int8() ? 128 : 0, cap, start, n, (f16*)k_out,
+                               (f16*)v_out);
+        };
+        if (D == 256)
+            bits == 4 ? launch(fetch_kernel<4, 256, KPT>)
+                      : bits == 8 ? launch(fetch_kernel<8, 256, KPT>) : launch(fetch_kernel<16, 256, KPT>);
+        else
+            bits == 4 ? launch(fetch_kernel<4, 128, KPT>)
+                      : bits == 8 ? launch(fetch_kernel<8, 128, KPT>) : launch(fetch_kernel<16, 128, KPT>);
     };
-    if (D == 256)
-        bits == 4 ? launch(fetch_kernel<4, 256>)
-                  : bits == 8 ? launch(fetch_kernel<8, 256>) : launch(fetch_kernel<16, 256>);
+    if ((int64_t)n * hkv * D < kShortFetch)
+        run(std::integral_constant<int, 1>{});
     else
-        bits == 4 ? launch(fetch_kernel<4, 128>)
-                  : bits == 8 ? launch(fetch_kernel<8, 128>) : launch(fetch_kernel<16, 128>);
+        run(std::integral_constant<int, 8>{});
     QW_HIP_CHECK(hipGetLastError());
     return QW_OK;
 }

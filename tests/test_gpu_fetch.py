@@ -42,6 +42,24 @@ def test_windows_of_a_fetch(mode, D):
 
 
 @pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("mode", ["affine4", "affine8", "int8", "fp16"])
+def test_long_windows_of_a_fetch(mode, D):
+    """Windows of 3 n D halves about 1 << 19, the line between a key and a block a thread."""
+    import qw_amd
+
+    r, n = rng(D + len(mode)), (1 << 19) // (3 * D)
+    k, v = (r.standard_normal((3, n + 30, D)).astype(np.float16) for _ in range(2))
+    c = qw_amd.KVCache(mode, 3, D)
+    c.update(_gpu(k), _gpu(v))
+    K, V = (np.concatenate([_np(c.dequantize(s, min(400, n + 30 - s))[i])[0] for s in range(0, n + 30, 400)], axis=1)
+            for i in (0, 1))
+    for start, m in ((0, n), (0, n + 1), (3, n + 1), (5, n + 9), (7, n), (29, n + 1), (0, n + 30)):
+        a, b = (_np(x)[0] for x in c.dequantize(start, m))
+        np.testing.assert_array_equal(a, K[:, start:start + m])
+        np.testing.assert_array_equal(b, V[:, start:start + m])
+
+
+@pytest.mark.parametrize("D", [128, 256])
 def test_fp16_appends_around_blocks(D):
     import qw_amd
 
