@@ -330,6 +330,13 @@ int qw_kv_update_and_dlsa_attention(qw_kv_cache* cache, const void* q, int n_q_h
 /* Mask dtype of the general attention calls: uint8, nonzero = attend. */
 #define QW_MASK_BOOL 3
 
+/* The keys that the lists of neighbouring rows may hold together for an automatic
+ * qw_dlsa_sparse_attention(_typed) call of this shape (QW_DTYPE_* of q and of
+ * K / V) to read each once for all of them; 0 where the call goes row by row
+ * (as groups of rows with a larger union do). No GPU is touched. */
+int qw_dlsa_union_keys(int q_dtype, int kv_dtype, int n_rows, int width, int n_q_heads,
+                       int n_kv_heads, int head_dim, int n_keys);
+
 /* dlsa_attention::sparse_attention_with (dlsa_attention.rs:44) with the
  * reference's full dtype and head-dim contract (mlx_cxx_dlsa_attention.cpp:
  * 429-470): q in q_dtype, K and V alike in kv_dtype, each of QW_DTYPE_F16 /

@@ -74,6 +74,7 @@ _SIGNATURES = {
     "qw_kv_dequantize": (_i, [_p, _i, _i, _p, _p, _p]),
     "qw_kv_update_and_attention": (_i, [_p, _p, _i, _i, _p, _p, _f, _i, _p, _p]),
     "qw_kv_attention": (_i, [_p, _p, _i, _i, _f, _i, _p, _p]),
+    "qw_dlsa_union_keys": (_i, [_i] * 8),
     "qw_sdpa_takes_rows": (_i, [_i, _i, _i, _i, _i, _i, _i, _f, _i]),
     "qw_sdpa": (_i, [_p, _i, _i, _p, _p, _i, _i, _i, _i64, _i64, _i64, _i64, _f, _i, _i, _f,
                      _p, _i, _i64, _i64, _p, _p]),

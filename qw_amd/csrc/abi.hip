@@ -296,6 +296,16 @@ int qw_dlsa_sparse_attention(const void* q, const void* k, const void* v, int64_
                                          (hipStream_t)stream));
 }
 
+int qw_dlsa_union_keys(int q_dtype, int kv_dtype, int n_rows, int width, int n_q_heads,
+                       int n_kv_heads, int head_dim, int n_keys) {
+    if (n_kv_heads <= 0 || n_q_heads < n_kv_heads || n_q_heads % n_kv_heads || n_rows <= 0 || width <= 0 ||
+        n_keys <= 0 || (head_dim != 32 && head_dim != 64 && head_dim != 128 && head_dim != 256) ||
+        n_q_heads / n_kv_heads > 16 || (int64_t)n_rows * n_kv_heads < 192)
+        return 0;
+    return (int)qw::dlsa_rows_union(q_dtype, kv_dtype, n_rows, width, n_kv_heads, n_q_heads / n_kv_heads,
+                                    head_dim, n_keys, nullptr);
+}
+
 int qw_dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const void* v,
                                    int kv_dtype, int64_t k_head_stride, int64_t k_row_stride,
                                    int64_t v_head_stride, int64_t v_row_stride,

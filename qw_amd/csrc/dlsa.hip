@@ -824,13 +824,16 @@ static int dlsa_sparse_attention_impl(const void* q, const DlsaSource& src,
     a.scale2 = scale * kLog2e;
     a.flags = nullptr;
     a.group_rows = 1;
-    if (auto_one_pass && !src.cache &&
-        dlsa_rows_pays(n_rows, width, n_kv_heads, n_q_heads / n_kv_heads, head_dim, n_keys, stream)) {
+    const int64_t most = auto_one_pass && !src.cache
+                             ? dlsa_rows_union(QW_DTYPE_F16, QW_DTYPE_F16, n_rows, width, n_kv_heads, G,
+                                               head_dim, n_keys, stream)
+                             : 0;
+    if (most > 0) {
         // prefill row counts: neighbouring rows share their keys' gathers; the
         // kernel below then serves the groups that this one leaves
         const int rc = dlsa_rows_attention(q, QW_DTYPE_F16, src.k, src.v, QW_DTYPE_F16, src.khs,
                                            src.krs, src.vhs, src.vrs, lists, lengths, n_rows, width, n_q_heads, n_kv_heads,
-                                           head_dim, n_keys, scale, out, &a.flags, stream);
+                                           head_dim, n_keys, most, scale, out, &a.flags, stream);
         if (rc == QW_OK)
             a.group_rows = dlsa_rows_per_group(G);
         else if (rc != QW_ERR_STATE && rc != QW_ERR_OUT_OF_MEMORY)

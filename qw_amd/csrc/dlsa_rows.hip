@@ -229,6 +229,21 @@ __device__ __forceinline__ void store_as(void* out, int dtype, int64_t at, float
     else ((__bf16*)out)[at] = (__bf16)y;
 }
 
+// Whether group qt goes to the row-by-row kernel, for all 512 threads (the launch writes no
+// count): by the plan, or because more than a quarter of the groups do. Both launches are
+// then long however few groups each has, and a mixture costs their sum: fp16, 512 rows of
+// which half share too little, 649 us, 364 by rows alone; f32, 24 heads over 3, D = 128, 1100
+// rows of which the last 12 would be served, 1038 us, 608 by rows alone.
+__device__ __forceinline__ bool group_left(const DlsaRowsArgs& a, int qt, int h) {
+    if (a.counts[qt] < 0) return true;
+    int left = 0;
+    for (int i = 0; i < a.groups; i += 512)
+        left += __syncthreads_count(i + (int)threadIdx.x < a.groups && a.counts[i + threadIdx.x] < 0);
+    if (4 * left <= a.groups) return false;
+    if (threadIdx.x == 0) set_flag(a.flags + qt * a.hkv + h, kLeft);
+    return true;
+}
+
 template <int D, bool BF>
 __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
     using S = BlockShape<D>;
@@ -253,20 +268,8 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows_kernel(DlsaRowsArgs a) {
             qt = a.qt0 + t / (n_split * a.hkv);
         }
     }
-    if (a.counts[qt] < 0) return;  // (this launch writes no count: all waves leave)
+    if (group_left(a, qt, h)) return;
     const int tid = threadIdx.x, lane = tid & 63;
-    {
-        // Where more than a quarter of the groups is left, the fp16 row kernel serves
-        // all of them: both launches are then long, and a mixture costs their sum
-        // (512 rows of which half share too little: 649 us, 364 us by rows alone).
-        int left = 0;
-        for (int i = 0; i < a.groups; i += 512)
-            left += __syncthreads_count(i + tid < a.groups && a.counts[i + tid] < 0);
-        if (!BF && 4 * left > a.groups) {
-            if (tid == 0) set_flag(a.flags + qt * a.hkv + h, kLeft);
-            return;
-        }
-    }
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int n_tiles = (a.counts[qt] + KT - 1) / KT, tps = (n_tiles + n_split - 1) / n_split;
@@ -597,7 +600,7 @@ __global__ __launch_bounds__(512, 1) void dlsa_rows32_kernel(DlsaRowsArgs a) {
             qt = a.qt0 + t / (n_split * a.hkv);
         }
     }
-    if (a.counts[qt] < 0) return;  // (as above)
+    if (group_left(a, qt, h)) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -862,58 +865,90 @@ int launch_rows32(const DlsaRowsArgs& a, int D, int grid, hipStream_t stream) {
 
 }  // namespace
 
-// A group's union may hold 0.35 of its rows' entries less 1500 keys (the launches'
-// fixed cost): there the tiles cost what gathering the rows by pairs does (512 rows
-// in groups of 20, D = 256: of 2048 entries 334 against 364 us at 0.3, 407 at 0.4; of
-// 512 entries 98 against 106 us at 0.2, 126 at 0.3). The typed kernel behind the
-// other types' calls takes fifteen times as long a row (512 rows of 4612: 7.6 ms), so there nearly any union is
-// served (in fp32 3.8 ms at 0.45 of the entries).
-static int64_t union_limit(int width, int NR, bool typed) {
-    return (int64_t)((typed ? 0.9 : 0.35) * NR * width) - (typed ? 0 : 1500);
-}
-
 int dlsa_rows_per_group(int G) { return std::min(32, 128 / G) & ~1; }
 
-// The plan and its launches take some 40 us, so the calls that one round of row
-// workgroups serves (256) stay there. By rows against this, rows of a group sharing all
-// keys / a quarter: 66 rows of 4612 entries (24 heads over 4, D = 256) 221 -> 66 / 224 ->
-// 110 us, 48 rows (32 over 8, D = 128) 115 -> 61 / 171 -> 84 us, 512 rows of 512 63 -> 56
-// / 106 -> 98 us; but 192 rows of 512 34 -> 46 / 57 -> 58 us.
-// Where the keys are more than a served union may hold, rows that share next to nothing
-// pay the plan for nothing, or for a part of the groups (24 over 4, 4612 entries of 33k
-// keys in blocks drawn for each row: D = 128, 66 rows 107 -> 178, 400 490 -> 536, 1500
-// 1200 -> 1239 us; D = 256, 140 rows 416 -> 452, 400 853 -> 889, 1500 2646 -> 2506 us), and
-// nothing on the host tells them from rows that share (450 -> 196 us at 400): such a call
-// is taken from 12M entries of 256 dims over the heads, where that loss is at most 3 %.
-bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys, hipStream_t stream) {
-    if (stream == hipStreamPerThread) return false;  // (one handle, a stream a thread)
-    const int64_t entries = (int64_t)n_rows * width * n_kv_heads;
-    if (n_rows < 32 || n_rows * (int64_t)n_kv_heads <= 256 || entries < 850000) return false;
-    return n_keys <= union_limit(width, dlsa_rows_per_group(G), false) || entries * D >= (int64_t)256 * 12000000;
+// How the groups of a call are divided: whole rounds of unsplit workgroups, the rest split
+// over their keys, at least four tiles of the largest union each (those past a smaller
+// one's end cost a launch slot and an empty partial).
+struct GroupPlan {
+    int groups, q_main, n_split;  // groups in all, in whole rounds, and the splits of the rest
+};
+static GroupPlan plan_groups(int n_rows, int n_kv_heads, int NR, int64_t tiles) {
+    GroupPlan p{(n_rows + NR - 1) / NR, 0, 1};
+    const int64_t units = (int64_t)p.groups * n_kv_heads;
+    if (units >= 256 && 256 % n_kv_heads == 0) p.q_main = (int)(units / 256) * (256 / n_kv_heads);
+    const int64_t tail = (int64_t)(p.groups - p.q_main) * n_kv_heads;
+    if (tail > 0) p.n_split = (int)std::max<int64_t>(1, std::min({256 / tail, tiles / 4, (int64_t)32}));
+    return p;
+}
+
+// The largest union of a group that is worth serving here, 0 for a call that is not: where
+// the time here, estimated from the plan, a cost of the launches and one a key of the
+// unions, meets the estimate for the kernel that runs row by row behind (by row pairs in
+// fp16, dlsa_typed.hip for the other types). A call is taken if it gains a tenth where the
+// rows share nearly all keys, as a prefill chunk's do. The coefficients are fitted to 3,100
+// calls timed by both (eight head geometries at D = 64 / 128 / 256, 64 to 4608 entries of 1k
+// to 66k keys, 33 to 1100 rows; lists shared, sliding, drawn in blocks and singly): nine in
+// ten estimates within 25 %.
+// Here / by rows, lists shared and drawn singly, in us: fp16, 24 heads over 4, D = 256, 1536
+// rows of 4612 entries 345 / 1312; 16 over 2, D = 64, 1100 rows of 1024 entries drawn singly
+// from 4k keys 110 / 72 (left); bf16, 24 over 4, D = 256, 48 rows of 128 38 / 79; f32, 8 over 8, D =
+// 128, 96 rows of 64 28 / 17 and 47 / 21 (left).
+// Where a union may be larger than that, rows that share next to nothing pay the plan
+// (some 16 us, and 0.45 a thousand keys) for nothing, and nothing on the host tells them
+// from rows that share. A typed call is taken where that is at most a quarter of its
+// time, an fp16 call from 12M entries of 256 dims over the heads, where it measured 2 to 5 %
+// (D = 256, 8 heads, 329 rows 1613 -> 1676 us; D = 128, 32 over 8, 658 rows 1444 -> 1516).
+int64_t dlsa_rows_union(int q_dtype, int kv_dtype, int n_rows, int width, int n_kv_heads, int G, int D,
+                        int n_keys, hipStream_t stream) {
+    if (stream == hipStreamPerThread) return 0;  // (one handle, a stream a thread)
+    const bool alike = q_dtype == kv_dtype && kv_dtype != QW_DTYPE_F32 && D != 32;
+    const bool pairs = alike && q_dtype == QW_DTYPE_F16;
+    if (pairs && (n_rows < 32 || (int64_t)n_rows * n_kv_heads <= 256)) return 0;
+    const int NR = dlsa_rows_per_group(G), KT = (alike ? 16384 : 8192) / D;
+    const double W = width, entries = 1e-6 * n_rows * W * n_kv_heads, drawn = (double)NR * W;
+    const double most = std::min<double>(n_keys, drawn), close = std::min<double>(n_keys, 1.3 * W + 2 * NR);
+    // row by row: a list's own length in time, however few the rows, and the entries' share
+    const double list = pairs ? 10 + 0.0085 * W : 9 + (0.045 + 0.06 * G) * W;
+    const double rows = list + (pairs ? 3 + 0.215 * D : 62 + 0.13 * D + (31 + 0.125 * D) * G) * entries;
+    const GroupPlan p = plan_groups(n_rows, n_kv_heads, NR, (int64_t)(most + KT - 1) / KT);
+    const int64_t tail = (int64_t)(p.groups - p.q_main) * n_kv_heads;
+    const double partials = p.n_split > 1 ? 8e-6 * p.n_split * n_kv_heads * D *
+                                                ((double)n_rows * G - (double)p.q_main * NR * G)
+                                          : 0.0;  // MB
+    const double rounds = (double)p.q_main * n_kv_heads / 256 +
+                          (tail > 0 ? (double)((tail * p.n_split + 255) / 256) / p.n_split : 0.0);
+    const double tile = pairs ? 2.4 + 155.0 / D : alike ? 2.6 + 180.0 / D : 7.3;
+    const double launches = (alike ? 21 : 24) + 0.45e-3 * n_keys + (0.12 + 35.0 / D) * partials;
+    const double key = tile / KT * rounds;
+    double limit = ((pairs ? 1.0 : 0.8) * rows - launches) / key;
+    if (pairs) {
+        limit = std::min(limit, 0.35 * drawn - 1500);
+    } else if (limit < most) {
+        // (a group that is left costs `list` beside the time here, so where some may be,
+        // unions far above a list are served only if both together take less)
+        limit = std::min(limit, std::max((rows - list - launches) / key, 1.1 * close));
+    }
+    if (limit <= close || (alike ? 1.1 : 1.3) * (launches + key * close) >= rows) return 0;
+    if (limit < most && (pairs ? entries * D < 12.0 * 256 : 16 + 0.45e-3 * n_keys > 0.25 * rows)) return 0;
+    return (int64_t)std::min(limit, most);
 }
 
 int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v, int kv_dtype,
                         int64_t khs, int64_t krs, int64_t vhs, int64_t vrs, const int32_t* lists,
                         const int32_t* lengths, int n_rows, int width, int n_q_heads,
-                        int n_kv_heads, int D, int n_keys, float scale, void* out,
+                        int n_kv_heads, int D, int n_keys, int64_t most, float scale, void* out,
                         const int** flags, hipStream_t stream) {
     const int G = n_q_heads / n_kv_heads, NR = dlsa_rows_per_group(G);
     const bool fp16 = q_dtype == QW_DTYPE_F16 && kv_dtype == QW_DTYPE_F16;
     const bool bf16 = q_dtype == QW_DTYPE_BF16 && kv_dtype == QW_DTYPE_BF16;
     const bool rows32 = !(fp16 || bf16) || D == 32;
-    const int KT = (rows32 ? 8192 : 16384) / D, groups = (n_rows + NR - 1) / NR;
-    const int64_t most = std::min<int64_t>(n_keys, (int64_t)NR * width);
-    const int max_union = (int)std::min<int64_t>(most, std::max<int64_t>(KT, union_limit(width, NR, !fp16 || rows32)));
+    const int KT = (rows32 ? 8192 : 16384) / D, max_union = (int)most;
     const int cap = (max_union + KT - 1) / KT * KT;
-    // whole rounds of unsplit workgroups, the rest split over their keys
+    const GroupPlan plan = plan_groups(n_rows, n_kv_heads, NR, cap / KT);
+    const int groups = plan.groups, q_main = plan.q_main, units = groups * n_kv_heads;
     DlsaRowsArgs a;
-    const int units = groups * n_kv_heads;
-    int q_main = 0;
-    if (units >= 256 && 256 % n_kv_heads == 0) q_main = units / 256 * (256 / n_kv_heads);
-    const int tail = (groups - q_main) * n_kv_heads;
-    // (splits of at least four tiles of the largest union served; those past a
-    // smaller one's end cost a launch slot and an empty partial)
-    a.n_split = tail > 0 ? std::max(1, std::min({256 / tail, cap / KT / 4, 32})) : 1;
+    a.n_split = plan.n_split;
     a.n_main = q_main * n_kv_heads;
     a.qt0 = q_main;
     a.prow0 = q_main * NR * G;

@@ -320,18 +320,19 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
     a.group_rows = 1;
     // Rows laid out for 16-byte pieces: neighbouring rows share their keys' gathers
     // (dlsa_rows.hip), and the kernel here serves the groups which that leaves (or
-    // every row, without room for its lists). From 20k entries over all heads at
-    // D = 256 (as many bytes at others): 512 rows of 4612 entries (24 heads over 4, D =
-    // 256) in bf16 7572 -> 175 us, in f32 7530 -> 744 us; 48 rows of 128 in bf16 79 ->
-    // 38 us, in f32 78 -> 61 us.
+    // every row, without room for its lists). 512 rows of 4612 entries (24 heads over 4, D =
+    // 256) in bf16 7572 -> 175 us, in f32 7530 -> 744 us; 48 rows of 128 in bf16 79 -> 38 us,
+    // in f32 78 -> 61 us.
     const int64_t per16 = 16 / (int64_t)es;
     const bool aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 &&
                          khs % per16 == 0 && krs % per16 == 0 && vhs % per16 == 0 && vrs % per16 == 0;
-    if (auto_one_pass && aligned && stream != hipStreamPerThread &&
-        (int64_t)n_rows * width * n_kv_heads * head_dim >= 20000 * 256) {
+    const int64_t most = auto_one_pass && aligned ? dlsa_rows_union(q_dtype, kv_dtype, n_rows, width, n_kv_heads,
+                                                                    G, head_dim, n_keys, stream)
+                                                  : 0;
+    if (most > 0) {
         const int rc = dlsa_rows_attention(q, q_dtype, k, v, kv_dtype, khs, krs, vhs, vrs, lists,
                                            lengths, n_rows, width, n_q_heads, n_kv_heads, head_dim,
-                                           n_keys, scale, out, &a.flags, stream);
+                                           n_keys, most, scale, out, &a.flags, stream);
         if (rc == QW_OK)
             a.group_rows = dlsa_rows_per_group(G);
         else if (rc != QW_ERR_STATE && rc != QW_ERR_OUT_OF_MEMORY)

@@ -248,13 +248,15 @@ int dlsa_sparse_attention_typed(const void* q, int q_dtype, const void* k, const
 // 0; the caller launches a row-by-row kernel behind it for the others.
 // QW_ERR_STATE / QW_ERR_OUT_OF_MEMORY, with nothing enqueued, without a workspace.
 int dlsa_rows_per_group(int G);
-// Whether a one-pass fp16 call takes it (the rule and both sides in dlsa_rows.hip).
-bool dlsa_rows_pays(int n_rows, int width, int n_kv_heads, int G, int D, int n_keys, hipStream_t stream);
+// The largest union of a group that a one-pass call is served with, 0 where the call does
+// better row by row (the rule and both sides in dlsa_rows.hip).
+int64_t dlsa_rows_union(int q_dtype, int kv_dtype, int n_rows, int width, int n_kv_heads, int G, int head_dim,
+                        int n_keys, hipStream_t stream);
 int dlsa_rows_attention(const void* q, int q_dtype, const void* k, const void* v, int kv_dtype,
                         int64_t k_head_stride, int64_t k_row_stride, int64_t v_head_stride, int64_t v_row_stride,
                         const int32_t* lists, const int32_t* lengths, int n_rows, int width,
-                        int n_q_heads, int n_kv_heads, int head_dim, int n_keys, float scale,
-                        void* out, const int** flags, hipStream_t stream);
+                        int n_q_heads, int n_kv_heads, int head_dim, int n_keys, int64_t most,
+                        float scale, void* out, const int** flags, hipStream_t stream);
 // The same for a Turbo4 cache (one query tile, at least 256 cached rows,
 // capacity reserved): fused as launch_block_attention_t4's fused pass (out:
 // the rows rotated back), else its fp16 arithmetic (out: rotated-basis rows).

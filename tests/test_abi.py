@@ -171,3 +171,31 @@ def test_sdpa_row_kernel_line_limits(qwlib):
     assert f(16, 1, 1, 1 << 20, 256, 1, 0, 0.0, 3) == 0      # 16 rows a KV head
     assert f(24, 4, 5, 100, 256, 1, 0, 0.0, -1) == 0 and f(24, 0, 4, 100, 256, 1, 0, 0.0, -1) == 0
     assert f(24, 1 << 20, 4, 1 << 20, 256, 1, 0, 0.0, -1) == 1  # (no overflow on the way)
+
+
+@pytest.mark.parametrize("dt,hq,hkv,D,L,T,W,kind,rows_us,here_us", [
+    # calls timed row by row and by the unions of neighbouring rows, near the line
+    ("f16", 24, 4, 256, 1536, 33280, 4612, "sliding", 1312, 345),
+    ("f16", 16, 2, 64, 1100, 4000, 1024, "single draws", 72, 110),
+    ("f16", 32, 8, 128, 97, 8000, 1100, "shared", 39, 44),
+    ("f16", 16, 2, 64, 194, 8000, 2200, "shared", 39, 42),
+    ("bf16", 24, 4, 256, 512, 16000, 4612, "sliding", 7572, 175),
+    ("bf16", 24, 4, 256, 48, 1000, 128, "sliding", 79, 38),
+    ("bf16", 8, 8, 128, 96, 1000, 64, "shared", 16, 24),
+    ("f32", 8, 8, 128, 96, 1000, 64, "single draws", 21, 47),
+    ("f32", 4, 2, 256, 192, 1000, 64, "shared", 22, 36),
+    ("f32", 24, 4, 256, 512, 16000, 4612, "sliding", 7530, 744),
+])
+def test_dlsa_union_line(qwlib, dt, hq, hkv, D, L, T, W, kind, rows_us, here_us):
+    """Whether a sparse read's rows share their gathers: where that measured faster."""
+    c = {"f16": 0, "bf16": 1, "f32": 2}[dt]
+    n = qwlib.qw_dlsa_union_keys(c, c, L, W, hq, hkv, D, T)
+    assert (n > 0) == (here_us < rows_us) and n <= T
+
+
+def test_dlsa_union_line_limits(qwlib):
+    f = qwlib.qw_dlsa_union_keys
+    assert f(1, 1, 47, 4612, 24, 4, 256, 100000) == 0                 # split lists
+    assert 0 < f(1, 1, 1 << 20, 1 << 16, 24, 4, 256, 1 << 30) < 1 << 30  # (no overflow on the way)
+    assert f(0, 0, 1 << 20, 1 << 20, 16, 1, 64, (1 << 31) - 1) >= 0
+    assert f(0, 0, 0, 64, 16, 1, 64, 100) == 0 and f(0, 0, 9999, 64, 17, 1, 64, 100) == 0

@@ -53,11 +53,17 @@ def _run(q, k, v, lists, lengths, scale, bf16):
     return qw_amd.sparse_attention_typed(*t, _gpu(lists), _gpu(lengths), scale)[0].float().cpu().numpy()
 
 
-def _fp16_takes_it(hq, hkv, D, L, T, W):
-    """The fp16 rule (dlsa_rows_pays), restated."""
-    NR, entries = min(32, 128 // (hq // hkv)) & ~1, L * W * hkv
-    return (L >= 32 and L * hkv > 256 and entries >= 850000 and
-            (T <= int(0.35 * NR * W) - 1500 or entries * D >= 256 * 12000000))
+TYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+# half a unit in the last place of the output's type, relative to the value
+ROUND = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 0.0}
+
+
+def _takes_it(hq, hkv, D, L, T, W, dt="f16"):
+    """Whether the call's rows share their keys' gathers."""
+    import qw_amd
+
+    c = {"f16": 0, "bf16": 1, "f32": 2}[dt]
+    return qw_amd.lib().qw_dlsa_union_keys(c, c, L, W, hq, hkv, D, T) > 0
 
 
 CASES = [
@@ -73,11 +79,15 @@ CASES = [
     (16, 1, 128, 600, 4000, 1500, "shared", False),   # G = 16: 8 rows a group
     (24, 4, 256, 96, 90000, 2300, "sliding", False),  # three bitmap passes
     (24, 4, 256, 1300, 2600, 400, "sliding", False),  # whole rounds and a split rest
-    (24, 4, 256, 440, 2000, 512, "shared", True),     # the union exactly eight tiles
-    (24, 4, 256, 440, 2000, 513, "shared", True),
-    (24, 4, 256, 700, 700, 321, "shared", True),
-    (16, 2, 64, 300, 6000, 1500, "sliding", True),
-    (16, 1, 128, 600, 2500, 1500, "shared", True),
+    (24, 4, 256, 440, 2000, 512, "shared", False),    # the union exactly eight tiles
+    (24, 4, 256, 440, 2000, 513, "shared", False),
+    (16, 2, 64, 300, 6000, 1500, "sliding", False),
+    (16, 1, 128, 600, 2500, 1500, "shared", False),
+    (24, 4, 256, 700, 700, 321, "shared", True),      # (fp16's of the kinds above)
+    (24, 4, 256, 900, 2000, 512, "shared", True),
+    (24, 4, 256, 900, 2000, 513, "shared", True),
+    (16, 2, 64, 300, 6000, 3000, "sliding", True),
+    (16, 1, 128, 600, 3000, 2500, "shared", True),
     (24, 4, 256, 1300, 2600, 800, "sliding", True),
 ]
 
@@ -86,8 +96,8 @@ CASES = [
 @pytest.mark.parametrize("hq,hkv,D,L,T,W,kind,fp16", CASES)
 def test_rows_match_oracle(hq, hkv, D, L, T, W, kind, fp16, bf16):
     print(f"case hq={hq} hkv={hkv} D={D} L={L} T={T} W={W} {kind} bf16={bf16}", flush=True)
-    assert fp16 == _fp16_takes_it(hq, hkv, D, L, T, W), "the route of the fp16 call"
-    assert L * hkv >= 192 and L * W * hkv * D >= 20000 * 256, "a shape of the bf16 call's kernel"
+    assert fp16 == _takes_it(hq, hkv, D, L, T, W), "the route of the fp16 call"
+    assert _takes_it(hq, hkv, D, L, T, W, "bf16"), "a shape of the bf16 call's kernel"
     if bf16 and hq // hkv > 8:
         pytest.skip("the typed read takes at most 8 heads a KV head")
     r = rng(hq + D + L + T + W)
@@ -120,6 +130,37 @@ def test_a_key_listed_twice_counts_twice(bf16):
     _check(out, q, k, v, lists, lengths, 0.1, bf16, "a key twice")
 
 
+@pytest.mark.parametrize("dt,hq,hkv,D,L,T,W,served", [
+    ("f32", 24, 3, 128, 1100, 16000, 256, False),   # every union but the last, short group's too large
+    ("bf16", 8, 8, 128, 384, 30000, 256, False),
+    ("f32", 4, 2, 256, 200, 4000, 256, False),      # (no whole group served)
+    ("bf16", 8, 8, 128, 600, 30000, 512, True),     # an eighth of the groups left, the others served
+    ("f32", 24, 4, 256, 300, 30000, 700, True),
+])
+def test_typed_rows_left_in_part_or_together(dt, hq, hkv, D, L, T, W, served):
+    """Unions past the limit: more than a quarter of the groups takes the others along."""
+    import qw_amd
+
+    c = {"bf16": 1, "f32": 2}[dt]
+    NR, limit = min(32, 128 // (hq // hkv)) & ~1, qw_amd.lib().qw_dlsa_union_keys(c, c, L, W, hq, hkv, D, T)
+    r = rng(D + L + T)
+    own = L // 8 if served else L
+    lists = np.stack([np.sort(r.permutation(T)[:W]) for _ in range(own)] +
+                     [np.sort(r.permutation(T)[:W])] * (L - own)).astype(np.int32)
+    unions = [len(np.unique(lists[g:g + NR])) for g in range(0, L, NR)]
+    left = sum(n > limit for n in unions)
+    assert 0 < limit < max(unions) and (0 < 4 * left <= len(unions) if served else 4 * left > len(unions))
+    dev = [torch.from_numpy(r.standard_normal(s).astype(np.float32)).to(TYPES[dt]).cuda()
+           for s in ((hq, L, D), (hkv, T, D), (hkv, T, D))]
+    q, k, v = (x.float().cpu().numpy() for x in dev)
+    lengths = np.full(L, W, np.int32)
+    out = qw_amd.sparse_attention_typed(*dev, _gpu(lists), _gpu(lengths), D ** -0.5)[0].float().cpu().numpy()
+    rows = np.unique(np.append(np.arange(0, L, 7), L - 1))
+    ref = oracle.dlsa_attention_f64(q[:, rows], k, v, lists[rows], lengths[rows], D ** -0.5)
+    bound = np.abs(ref) * ROUND[dt] + 1e-5 * np.linalg.norm(ref, axis=-1, keepdims=True) + 1e-7
+    assert np.isfinite(out).all() and np.all(np.abs(out[:, rows].astype(np.float64) - ref) <= bound)
+
+
 def _fp16_inputs(r, hq, hkv, D, L, T):
     return (r.standard_normal(s).astype(np.float16) for s in ((hq, L, D), (hkv, T, D), (hkv, T, D)))
 
@@ -139,7 +180,7 @@ def _check_some(out, q, k, v, lists, lengths, scale, what):
     (24, 4, 128, 2000, 30000, 3100, "eighth"),
 ])
 def test_fp16_rows_over_many_keys(hq, hkv, D, L, T, W, left):
-    assert _fp16_takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
+    assert _takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
     r = rng(L + T + D)
     q, k, v = _fp16_inputs(r, hq, hkv, D, L, T)
     n = {"all": L, "half": L // 2, "eighth": L // 8, "none": 0}[left]
@@ -153,8 +194,8 @@ def test_fp16_rows_over_many_keys(hq, hkv, D, L, T, W, left):
 
 def test_duplicates_in_a_third_of_the_groups():
     """More than a quarter of the groups list a key twice, in an fp16 call whose tail is split."""
-    hq, hkv, D, L, T, W = 24, 4, 256, 700, 4000, 800
-    assert _fp16_takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
+    hq, hkv, D, L, T, W = 24, 4, 256, 700, 4000, 1600
+    assert _takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
     r = rng(12)
     q, k, v = _fp16_inputs(r, hq, hkv, D, L, T)
     lists = _lists(r, "sliding", L, W, T)
@@ -167,7 +208,7 @@ def test_non_finite_groups_do_not_move_the_others():
     """Infinite values in the first 30 of 70 groups (their outputs are left to the row kernel): the
     other groups, later workgroups and a split tail among them, give the clean call's bits."""
     hq, hkv, D, L, T, W = 24, 4, 256, 1400, 13000, 2200
-    assert _fp16_takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
+    assert _takes_it(hq, hkv, D, L, T, W), "a shape of the kernel"
     r = rng(13)
     q, k, v = _fp16_inputs(r, hq, hkv, D, L, T)
     lists = _lists(r, "sliding", L, W, T - 1)
@@ -201,17 +242,13 @@ def test_infinite_values_stay_with_the_rows_that_list_them(bf16):
     assert not np.isfinite(out[:, 41, 5]).any()
 
 
-TYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
-# half a unit in the last place of the output's type, relative to the value
-ROUND = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8, "f32": 0.0}
-
-
 @pytest.mark.parametrize("qt,kt", [("f32", "f32"), ("bf16", "f16"), ("f16", "f32"), ("f32", "bf16"),
                                    ("f16", "bf16"), ("f16", "f16")])
 @pytest.mark.parametrize("hq,hkv,D,L,T,W,kind", [
     (24, 4, 256, 101, 3000, 300, "sliding"),   # 32-key tiles; the last group one row
-    (16, 2, 128, 70, 900, 128, "shared"),      # the union exactly two tiles
-    (16, 2, 128, 70, 900, 129, "own"),
+    (16, 2, 128, 96, 900, 128, "shared"),      # the union exactly two tiles
+    (16, 2, 128, 96, 900, 129, "own"),
+    (16, 2, 128, 70, 900, 129, "own"),         # (row by row: split lists)
     (8, 8, 64, 99, 2000, 333, "mixed"),        # G = 1
     (6, 1, 32, 200, 2000, 500, "sliding"),     # 256-key tiles
 ])
@@ -221,6 +258,9 @@ def test_typed_rows_match_float64(qt, kt, hq, hkv, D, L, T, W, kind):
     import qw_amd
 
     print(f"case q={qt} kv={kt} hq={hq} hkv={hkv} D={D} L={L} W={W} {kind}", flush=True)
+    c = {"f16": 0, "bf16": 1, "f32": 2}
+    here = qw_amd.lib().qw_dlsa_union_keys(c[qt], c[kt], L, W, hq, hkv, D, T) > 0
+    assert here == (L != 70 and (qt != kt or qt != "f16" or D == 32)), "the kernel of the call"
     r = rng(hq + D + L + T + W)
     dev = [torch.from_numpy(r.standard_normal(s).astype(np.float32)).to(TYPES[t]).cuda()
            for s, t in (((hq, L, D), qt), ((hkv, T, D), kt), ((hkv, T, D), kt))]
@@ -248,7 +288,7 @@ def test_bf16_weights_keep_32_bits(D):
     import qw_amd
 
     hq, hkv, L, T, W = 24, 4, 64, 2000, 400
-    assert L * hkv >= 192 and L * W * hkv * D >= 20000 * 256, "a shape of the kernel"
+    assert _takes_it(hq, hkv, D, L, T, W, "bf16"), "a shape of the kernel"
     f = lambda x: torch.from_numpy(x).to(torch.bfloat16)  # noqa: E731
     q = np.zeros((hq, L, D), np.float32)
     q[:, :, 0], q[:, :, 1] = np.linspace(0.25, 1.0, L), 2.0 ** -6

@@ -338,7 +338,7 @@ def _row_kernel_calls():
     m[:, 0] = True
     lists = _gpu(np.sort(np.stack([r.permutation(T)[:W]] * L), axis=1).astype(np.int32))
     lengths = _gpu(np.full(L, W, np.int32))
-    assert L * W * H >= 850000 and T <= int(0.35 * 20 * W) - 1500
+    assert all(qw_amd.lib().qw_dlsa_union_keys(c, c, L, W, H * G, H, D, T) > 0 for c in (0, 1, 2))
     typed = lambda dt: (q.to(dt), k.to(dt), v.to(dt), lists, lengths, 1 / 16)  # noqa: E731
     b16, f32 = typed(torch.bfloat16), typed(torch.float32)
     return {"dense": lambda: qw_amd.causal_attention(q, k, v, 1 / 16),

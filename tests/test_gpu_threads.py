@@ -42,6 +42,8 @@ def _sparse(seed, L, T, W, dt):
     q, k, v = (_gpu(r.standard_normal(s).astype(np.float16)).to(dt) for s in ((24, L, 256), (4, T, 256), (4, T, 256)))
     lists = _gpu(np.sort(np.stack([r.permutation(T)[:W]] * L), axis=1).astype(np.int32))
     lengths = _gpu(np.full(L, W, np.int32))
+    c = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}[dt]
+    assert qw_amd.lib().qw_dlsa_union_keys(c, c, L, W, 24, 4, 256, T) > 0
     f = qw_amd.sparse_attention if dt == torch.float16 else qw_amd.sparse_attention_typed
     return lambda: f(q, k, v, lists, lengths, 1 / 16)
 
