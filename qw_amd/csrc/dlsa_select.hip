@@ -170,10 +170,10 @@ __global__ __launch_bounds__(1024) void dlsa_select_kernel(SelectArgs a) {
             // the kernel at one row of 16,384 buckets). The range starts at the worst
             // of the threads' best keys, which as many keys as threads reach (so the
             // picks, if they are no more; the others are not even counted), and ends
-            // at the worst of the best keys of four interleaved groups, some eight
-            // keys below the top: neither masked nor outlying scores widen it (over all
+            // at the worst of the best keys of four groups of waves, some eight keys
+            // below the top: neither masked nor outlying scores widen it (over all
             // finite scores, a third of them at -3.4e38 took 43.0 us and one of 1000
-            // 37.0, where the radix select alone takes 32 and this 17). Rows with a
+            // 37.0, where the radix select alone takes 32 and this 16.4). Rows with a
             // NaN, next to no range, or more than kBinMax keys in a wanted bin (many
             // equal scores, heavy tails) take the radix select below; the attempt
             // costs them 1 to 5 us (33 to 38 us for e^(3 x), x normal, at 64 rows).
@@ -185,39 +185,54 @@ __global__ __launch_bounds__(1024) void dlsa_select_kernel(SelectArgs a) {
                               sizeof(whist) >= kSelectMax * sizeof(uint64_t),
                           "the bins share the other path's arrays");
             const bool wide = n_sel > T;  // (more picks than threads: from the worst finite key)
+            const int left = v - t;       // column t + j T is there if j T < left
             float hi = -INFINITY, mn = INFINITY;
 #pragma unroll
             for (int j = 0; j < kKeysPerThread; j++)
-                if (t + j * T < v) {
-                    hi = fmaxf(hi, f[j]);
-                    if (f[j] > -INFINITY) mn = fminf(mn, f[j]);
-                }
-            if (!wide) mn = hi > -INFINITY ? hi : INFINITY;
-            mn = wave_reduce(mn, OpMin());
+                if (j * T < left) hi = fmaxf(hi, f[j]);
+            if (wide) {
 #pragma unroll
-            for (int x = 4; x < 64; x <<= 1) hi = fmaxf(hi, __shfl_xor(hi, x));
-            float* const red = reinterpret_cast<float*>(hist);  // [16] and [16][4]
-            if ((t & 63) == 0) red[wave] = mn;
-            if ((t & 63) < 4) red[16 + 4 * wave + (t & 63)] = hi;
+                for (int j = 0; j < kKeysPerThread; j++)
+                    if (j * T < left && f[j] > -INFINITY) mn = fminf(mn, f[j]);
+            } else if (hi > -INFINITY) {
+                mn = hi;
+            }
+            hi = wave_reduce(hi, OpMax());
+            mn = wave_reduce(mn, OpMin());
+            float* const red = reinterpret_cast<float*>(hist);  // [2][16]
+            if ((t & 63) == 0) {
+                red[wave] = hi;
+                red[16 + wave] = mn;
+            }
             for (int i = t; i < NB; i += T) cursor[i] = 0;
             const bool any_nan = __syncthreads_or(nan);
-            float4v top = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-            for (int w = 0; w < n_waves; w++) {
-                mn = fminf(mn, red[w]);
+            // (waves: a power of two; fewer than four of them are read again)
+            float top[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+            for (int w = 0; w < n_waves; w += 4)
 #pragma unroll
-                for (int i = 0; i < 4; i++) top[i] = fmaxf(top[i], red[16 + 4 * w + i]);
-            }
+                for (int i = 0; i < 4; i++) {
+                    const int at = (w + i) & (n_waves - 1);
+                    top[i] = fmaxf(top[i], red[at]);
+                    mn = fminf(mn, red[16 + at]);
+                }
             hi = fminf(fminf(top[0], top[1]), fminf(top[2], top[3]));
             const float range = hi - mn;
             if (!any_nan && range > 1e-30f && range < INFINITY) {
                 const float inv = (float)NB / range;
                 auto bin = [&](float x) {
-                    return (int)fminf(fmaxf((hi - x) * inv, 0.0f), (float)(NB - 1));
+                    return (int)__builtin_amdgcn_fmed3f((hi - x) * inv, 0.0f, (float)(NB - 1));
                 };
-                auto counted = [&](int j) { return t + j * T < v && (wide || f[j] >= mn); };
+                const float from = wide ? -INFINITY : mn;
+                int bins[kKeysPerThread];  // (NB: not counted)
 #pragma unroll
-                for (int j = 0; j < kKeysPerThread; j++)
-                    if (counted(j)) atomicAdd(&cursor[bin(f[j])], 1);
+                for (int j = 0; j < kKeysPerThread; j++) {
+                    const bool counted = j * T < left && f[j] >= from;
+                    bins[j] = NB;
+                    if (counted) {
+                        bins[j] = bin(f[j]);
+                        atomicAdd(&cursor[bins[j]], 1);
+                    }
+                }
                 __syncthreads();
                 const int per = NB / T;  // consecutive bins a thread
                 int sum = 0;
@@ -242,11 +257,8 @@ __global__ __launch_bounds__(1024) void dlsa_select_kernel(SelectArgs a) {
                 if (!crowded && kept <= kSelectMax) {
 #pragma unroll
                     for (int j = 0; j < kKeysPerThread; j++)
-                        if (counted(j)) {
-                            const int b = bin(f[j]);
-                            if (b <= last)
-                                sel[atomicAdd(&cursor[b], 1)] = ((uint64_t)kr[j] << 32) | (uint32_t)(t + j * T);
-                        }
+                        if (bins[j] <= last)
+                            sel[atomicAdd(&cursor[bins[j]], 1)] = ((uint64_t)kr[j] << 32) | (uint32_t)(t + j * T);
                     __syncthreads();
                     for (int i = t; i < kept; i += T) {
                         const uint64_t x = sel[i];
@@ -254,7 +266,9 @@ __global__ __launch_bounds__(1024) void dlsa_select_kernel(SelectArgs a) {
                         const int b = bin(__uint_as_float((ord & 0x80000000u) ? ord ^ 0x80000000u : ~ord));
                         const int b0 = start[b], b1 = cursor[b];
                         int place = b0;
-                        for (int q = b0; q < b1; q++) place += sel[q] < x;
+                        for (int q = b0; q < b1; q += 4)  // (four reads in flight)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) place += q + i < b1 && sel[min(q + i, b1 - 1)] < x;
                         if (place < n_sel) out[place] = x;
                     }
                     picks = out;
