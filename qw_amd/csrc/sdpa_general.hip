@@ -469,10 +469,12 @@ int sdpa_general(const void* q, int n_q_heads, int n_rows, const void* k, const 
 #endif
 
 // Query rows a KV head up to which a masked call over a cache runs the block kernel
-// on the codes (dequantizing them again for each 128-row tile): at 2160 rows, 24 heads
-// over 4, D = 256, 8-bit, 138 against 159 us over 8k keys and 475 against 561 us over 33k
-// for dequantizing once and the row kernel; 78 rows 75 -> 23 us over 8k, where the
-// general kernel took them.
+// on the codes (dequantizing them again for each 128-row tile), against dequantizing once
+// and the row kernel. 24 heads over 4, D = 256, over 8k and 32k keys, in us: 2160 rows 4-bit 137 /
+// 153 and 423 / 505, 8-bit 144 / 152 and 460 / 504, fp16 159 / 154 and 504 / 518, Turbo4 172 / 161
+// and 521 / 510; 4086 rows 4-bit 206 / 218 and 671 / 745, 8-bit 216 / 224 and 695 / 744, fp16 237 / 222
+// and 725 / 754, Turbo4 259 / 236 and 789 / 759. 32 over 8, D = 128, 4088 rows: within 2 % or less.
+// The general kernel, which took them before, 980 and 3790.
 constexpr int kMaskedBlockRows = 4096;
 
 int window_first_key(const SdpaOptions& o, int T, int n_rows, int align) {
