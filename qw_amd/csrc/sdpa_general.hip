@@ -326,7 +326,7 @@ double general_us(int G, int n_rows, int hkv, int n_keys, int D, const SdpaOptio
     const GenPlan p = plan_general(R, hkv, n_keys);
     double tiles = p.split_tiles;  // of a workgroup
     if (o.window > 0)
-        tiles = std::min(tiles, (double)(o.window + 64 / G) / 32 + 1);
+        tiles = std::min(tiles, (o.window + 64.0 / G) / 32 + 1);
     else if (o.causal && p.n_split == 1)
         tiles *= 1.0 - 0.5 * n_rows / n_keys;
     const double rounds = std::max(1.0, (double)p.tiles * hkv * p.n_split / 256);

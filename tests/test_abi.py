@@ -169,6 +169,7 @@ def test_sdpa_row_kernel_line_limits(qwlib):
     assert f(24, 3072, 4, 524288, 256, 1, 0, 0.0, -1) == 1
     assert f(24, 3072, 4, 2097153, 256, 1, 0, 0.0, -1) == 0  # images past 4 GiB
     assert f(16, 1, 1, 1 << 20, 256, 1, 0, 0.0, 3) == 0      # 16 rows a KV head
+    assert f(24, 1536, 4, 9728, 256, 1, (1 << 31) - 1, 0.0, -1) == 1  # a window past any position
     assert f(24, 4, 5, 100, 256, 1, 0, 0.0, -1) == 0 and f(24, 0, 4, 100, 256, 1, 0, 0.0, -1) == 0
     assert f(24, 1 << 20, 4, 1 << 20, 256, 1, 0, 0.0, -1) == 1  # (no overflow on the way)
 
