@@ -1504,7 +1504,7 @@ static int launch_block_bits(KVCache& cc, const f16* q, int G, int Tq, float sca
     const int want = std::max(1, 256 / (q_tail * cc.hkv));
     // (a window: the keys from a query tile's first window start to its last row)
     const int plan_tiles =
-        window > 0 ? std::min(n_tiles, (window + wg_rows / G + 1 + S::KT - 1) / S::KT + 1) : n_tiles;
+        window > 0 ? (int)std::min<int64_t>(n_tiles, ((int64_t)window + wg_rows / G + S::KT) / S::KT + 1) : n_tiles;
     split_keys(plan_tiles, T4M == 2 ? std::min(std::max(want, 2), 128) : want, &n_split, &tps,
                window > 0 ? QW_WINDOW_MIN_TILES : 4);
     QW_REQUIRE(T4M != 2 || n_split > 1, QW_ERR_INVALID_ARGUMENT,

@@ -463,3 +463,20 @@ def test_softcap_keeps_small_scores(route, cap):
     roundings = 2 if route == "cache" else 1         # the parts of a key split, and the output
     bound = roundings * (np.abs(ref) * 2.0 ** -11 + 2.0 ** -25) + s[:, :, None] * 2.0 ** -22 + 3e-7
     assert np.all(np.abs(out - ref) <= bound), np.max(np.abs(out - ref) / bound)
+
+
+@pytest.mark.parametrize("window", [1 << 30, (1 << 31) - 400, (1 << 31) - 1])
+def test_windows_past_any_position(window):
+    """The largest windows, over a cache and over views (both kernels), see every key."""
+    import qw_amd
+
+    r = rng(31)
+    hq, hkv, D, T = 24, 4, 256, 1200
+    k, v = (r.standard_normal((hkv, T, D)).astype(np.float16) for _ in range(2))
+    cache = qw_amd.KVCache("fp16", hkv, D)
+    cache.update(_gpu(k), _gpu(v))
+    for L in (1, 7, 300):
+        q = _gpu(r.standard_normal((hq, L, D)).astype(np.float16))
+        ref = oracle.sdpa_general(_np(q), k, v, 1 / 16, True)
+        assert_close(_np(cache.attention_general(q, 1 / 16, causal=True, window=window))[0], ref, f"cache L={L}")
+        assert_close(_np(qw_amd.causal_attention(q, _gpu(k), _gpu(v), 1 / 16, 0.0, window))[0], ref, f"views L={L}")
