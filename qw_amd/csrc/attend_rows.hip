@@ -24,7 +24,7 @@
 // What bounds it: the LDS operand reads (one 1 KB read an MFMA) and the MFMAs;
 // laying the tiles out costs one read and one write of K and V. Before, every
 // workgroup of 64 rows transposed V into LDS with 2-byte stores and rescaled
-// its accumulators every 32 keys. Measured: see rows_route in sdpa_general.hip.
+// its accumulators every 32 keys. Measured: see sdpa_takes_rows in sdpa_general.hip.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
